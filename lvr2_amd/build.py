@@ -11,6 +11,7 @@ import os
 import shlex
 import subprocess
 import sys
+import tempfile
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
@@ -30,7 +31,6 @@ HIP_FLAGS = [
     "-O3",
     "-std=c++17",
     "-fPIC",
-    "-shared",
     "-ffp-contract=off",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-Wno-unused-result",
@@ -42,11 +42,24 @@ def _run(cmd: list[str]) -> None:
     subprocess.run(cmd, check=True)
 
 
+# The library's translation units, compiled in parallel and linked into one shared object.
+HIP_UNITS = ["lvrhip", "knn_tile_p8", "knn_tile_p4", "knn_tile_p2"]
+
+
 def build_lib() -> str:
-    src = os.path.join(CSRC, "lvrhip.hip")
-    tmp = LIB + ".tmp"
-    _run([HIPCC, *HIP_FLAGS, f"-I{INCLUDE}", f"-I{CSRC}", src, "-o", tmp])
-    os.replace(tmp, LIB)
+    with tempfile.TemporaryDirectory(prefix="lvrhip_build_") as tmpdir:
+        objs = [os.path.join(tmpdir, u + ".o") for u in HIP_UNITS]
+        procs = []
+        for u, o in zip(HIP_UNITS, objs):
+            cmd = [HIPCC, *HIP_FLAGS, f"-I{INCLUDE}", f"-I{CSRC}", "-c", os.path.join(CSRC, u + ".hip"), "-o", o]
+            print("+", " ".join(shlex.quote(c) for c in cmd), flush=True)
+            procs.append((cmd, subprocess.Popen(cmd)))
+        failed = [(cmd, p.returncode) for cmd, p in procs if p.wait() != 0]
+        if failed:
+            raise subprocess.CalledProcessError(failed[0][1], failed[0][0])
+        tmp = LIB + ".tmp"
+        _run([HIPCC, f"--offload-arch={ARCH}", "-shared", "-fPIC", *objs, "-o", tmp])
+        os.replace(tmp, LIB)
     return LIB
 
 

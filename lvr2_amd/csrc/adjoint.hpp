@@ -120,7 +120,7 @@ struct SinkSdfAdjoint {
 // the factor 2/n, for SinkPcaAdjoint; flags[j] = 1 + adaptive round (0: no gradient).
 constexpr int ADJ_STRIDE = 10;  // cxx cxy cxz cyy cyz czz, mux muy muz, 2/n
 
-__global__ __launch_bounds__(256) void pca_adjoint_prep_kernel(
+static __global__ __launch_bounds__(256) void pca_adjoint_prep_kernel(
     int64_t n, const float* __restrict__ px, const float* __restrict__ py, const float* __restrict__ pz,
     const float* __restrict__ nx, const float* __restrict__ ny, const float* __restrict__ nz,
     const float* __restrict__ mom, const uint8_t* __restrict__ kround, int kn, int64_t kmax,
@@ -179,7 +179,7 @@ __global__ __launch_bounds__(256) void pca_adjoint_prep_kernel(
 }
 
 // flags[i] == want for the query slots i < n (round selection of the PCA reverse pass)
-__global__ void select_round_kernel(const uint32_t* __restrict__ flags, int64_t n, uint32_t want,
+static __global__ void select_round_kernel(const uint32_t* __restrict__ flags, int64_t n, uint32_t want,
                                     uint32_t* __restrict__ out)
 {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -234,7 +234,7 @@ struct SinkPcaAdjoint {
 };
 
 // grad_xyz[pidx[j]] += (gpx, gpy, gpz)[j]
-__global__ void accumulate_grad_kernel(const float* __restrict__ gpx, const float* __restrict__ gpy,
+static __global__ void accumulate_grad_kernel(const float* __restrict__ gpx, const float* __restrict__ gpy,
                                        const float* __restrict__ gpz, const uint32_t* __restrict__ pidx, int64_t n,
                                        float* __restrict__ out)
 {
@@ -247,7 +247,7 @@ __global__ void accumulate_grad_kernel(const float* __restrict__ gpx, const floa
     out[3 * (int64_t)j + 2] += gpz[i];
 }
 
-__global__ void zero_f32_kernel(float* __restrict__ p, int64_t n)
+static __global__ void zero_f32_kernel(float* __restrict__ p, int64_t n)
 {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) p[i] = 0.0f;

@@ -344,18 +344,7 @@ __global__ __launch_bounds__(BF_THREADS) void bf_knn_kernel(const BvhView bv, co
     for (;;) {
         int64_t chunk = -1;
         if (queue) {
-            while (seg_k < QUEUE_SEGS) {
-                const int seg = (xcd + seg_k) % QUEUE_SEGS;
-                uint32_t r = 0;
-                if (lane == 0) r = atomicAdd(queue + seg * QUEUE_STRIDE, 1u);
-                r = (uint32_t)__builtin_amdgcn_readlane((int)r, 0);
-                const int64_t cand = ((int64_t)(r / QUEUE_CHUNK) * QUEUE_SEGS + seg) * QUEUE_CHUNK + r % QUEUE_CHUNK;
-                if (cand < nchunks) {
-                    chunk = cand;
-                    break;
-                }
-                seg_k++;  // this XCD's chunks only grow with r: all taken
-            }
+            chunk = queue_take(queue, nchunks, xcd, seg_k);
         } else if (!once) {
             chunk = blockIdx.x;
             once = true;

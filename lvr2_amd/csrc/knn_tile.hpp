@@ -141,20 +141,21 @@ enum {
 
 __device__ __forceinline__ unsigned long long cycles() { return (unsigned long long)clock64(); }
 
-// Wave-local counters, flushed with one atomic per counter at the end of the wave.
+// Wave-local counters, flushed with one atomic per counter at the end of the wave.  They exist only
+// in the kernels launched while profiling is on: sixteen 64-bit counters and their clock reads,
+// live through the whole kernel, had cost every launch 160-190 spilled SGPRs (each a lane write and
+// read in VALU instructions) and 9 VGPRs.
+template <bool kOn>
 struct WaveStats {
     unsigned long long c[KS_COUNT];
-    bool timing;
     __device__ void clear()
     {
 #pragma unroll
         for (int i = 0; i < KS_COUNT; i++) c[i] = 0;
     }
-    __device__ __forceinline__ unsigned long long tick() const { return timing ? cycles() : 0ull; }
-    __device__ __forceinline__ void tock(int i, unsigned long long t0)
-    {
-        if (timing) c[i] += cycles() - t0;
-    }
+    __device__ __forceinline__ void add(int i, unsigned v) { c[i] += v; }
+    __device__ __forceinline__ unsigned long long tick() const { return cycles(); }
+    __device__ __forceinline__ void tock(int i, unsigned long long t0) { c[i] += cycles() - t0; }
     __device__ __forceinline__ void flush(unsigned long long* dst)
     {
         if (!dst || lane_id() != 0) return;
@@ -162,6 +163,14 @@ struct WaveStats {
         for (int i = 0; i < KS_COUNT; i++)
             if (c[i]) atomicAdd(&dst[i], c[i]);
     }
+};
+template <>
+struct WaveStats<false> {
+    __device__ __forceinline__ void clear() {}
+    __device__ __forceinline__ void add(int, unsigned) {}
+    __device__ __forceinline__ unsigned long long tick() const { return 0ull; }
+    __device__ __forceinline__ void tock(int, unsigned long long) {}
+    __device__ __forceinline__ void flush(unsigned long long*) {}
 };
 
 template <int Q, int BUF, int NT>
@@ -179,6 +188,45 @@ struct TileSmem {
     uint32_t bcnt[NT][Q];
     uint32_t scnt[NT][Q];  // per-query sink slot counters
 };
+
+// ---- work queue ---------------------------------------------------------------------------
+
+// Takes the wave's next item of n from a queue of QUEUE_SEGS counters (dealt in blocks of QUEUE_CHUNK
+// to the segments in turn), first from segment xcd, then from the others in turn; -1 when all are
+// drained.  seg_k: 0 until the wave's own segment is drained.  A counter only grows, so a segment once
+// seen drained stays drained: a wave that is done with its own looks at all eight at once (lane s reads
+// segment s's counter) and adds only to one that still holds items.  Adding to every segment's counter in
+// turn, as each wave's exit did before, put 8 serialised atomics per wave on eight addresses: an empty
+// launch of 4,096 waves took 88 us (the four empty later rounds of the 300,000-point plain scene: a
+// third of its normals pass, 1,052 -> 704 us without them).
+__device__ __forceinline__ int64_t queue_item(uint32_t r, int seg)
+{
+    return ((int64_t)(r / QUEUE_CHUNK) * QUEUE_SEGS + seg) * QUEUE_CHUNK + r % QUEUE_CHUNK;
+}
+__device__ __forceinline__ int64_t queue_take(uint32_t* queue, int64_t n, int xcd, int& seg_k)
+{
+    const int lane = lane_id();
+    for (;;) {
+        int seg = xcd;
+        if (seg_k > 0) {
+            bool open = false;
+            if (lane < QUEUE_SEGS) {
+                const int sl = (xcd + lane) % QUEUE_SEGS;
+                const uint32_t c = __hip_atomic_load(queue + sl * QUEUE_STRIDE, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                open = queue_item(c, sl) < n;
+            }
+            const uint64_t m = ballot(open);
+            if (m == 0) return -1;
+            seg = (xcd + __ffsll((long long)m) - 1) % QUEUE_SEGS;
+        }
+        uint32_t r = 0;
+        if (lane == 0) r = atomicAdd(queue + seg * QUEUE_STRIDE, 1u);
+        r = (uint32_t)__builtin_amdgcn_readlane((int)r, 0);
+        const int64_t item = queue_item(r, seg);
+        if (item < n) return item;
+        seg_k = 1;
+    }
+}
 
 // ---- traversal ---------------------------------------------------------------------------
 
@@ -202,9 +250,9 @@ struct TileBox {
 // With rej != NULL, *rej is lowered to the smallest box distance of a child the traversal
 // rejected (a lower bound of the distance of every point outside the list).  With
 // store = false the leaves are only counted (up to cap).
-template <class Sm>
+template <class Sm, class Ws>
 __device__ __forceinline__ int fill_leaves(Sm& sm, const BvhView& bv, const TileBox& tb, float r2, int& sp, int cap,
-                                           WaveStats& ws, float* rej = nullptr, bool store = true)
+                                           Ws& ws, float* rej = nullptr, bool store = true)
 {
     constexpr int NONE = 0x7fffffff;
     const int lane = lane_id();
@@ -224,7 +272,7 @@ __device__ __forceinline__ int fill_leaves(Sm& sm, const BvhView& bv, const Tile
             sp = -1;
             return nl;
         }
-        ws.c[KS_POPS] += (unsigned)w;
+        ws.add(KS_POPS, (unsigned)w);
         const int ref = lane < w ? sm.stack[sp - 1 - lane] : NONE;
         sp -= w;
         __syncthreads();
@@ -481,9 +529,9 @@ struct Cands {
 // Calls f(nl, base) once per staged chunk of nl leaves starting at sm.tleaf[base].
 // The kernel's helpers are all inlined: a call would move the structs it passes by
 // reference (views, counters) into scratch memory.
-template <class Sm, class F>
+template <class Sm, class Ws, class F>
 __device__ __forceinline__ bool for_each_chunk(Sm& sm, const BvhView& bv, const TileBox& tb, float R2, int cur,
-                                               Cands& cs, WaveStats& ws, F&& f)
+                                               Cands& cs, Ws& ws, F&& f)
 {
     if (cs.ntl >= 0) {
         if (cs.resident) {
@@ -497,10 +545,10 @@ __device__ __forceinline__ bool for_each_chunk(Sm& sm, const BvhView& bv, const 
             const int base = (cs.reverse ? nch - 1 - i : i) * CHUNK_LEAVES;
             const int nl = min(CHUNK_LEAVES, cs.ntl - base);
             if (base != cs.staged) {
-                const auto t0 = ws.tick();
+                [[maybe_unused]] const auto t0 = ws.tick();
                 load_chunk(sm, bv, base, nl);
                 ws.tock(KS_CY_LOAD, t0);
-                ws.c[KS_CHUNKS] += 1;
+                ws.add(KS_CHUNKS, 1);
                 cs.staged = base;
             }
             f(nl, base);
@@ -519,7 +567,7 @@ __device__ __forceinline__ bool for_each_chunk(Sm& sm, const BvhView& bv, const 
         t0 = ws.tick();
         load_chunk(sm, bv, 0, nl);
         ws.tock(KS_CY_LOAD, t0);
-        ws.c[KS_CHUNKS] += 1;
+        ws.add(KS_CHUNKS, 1);
         f(nl, 0);
         __syncthreads();
         if (sp == 0) return true;
@@ -663,7 +711,7 @@ constexpr bool tile_three_waves()
     return P == 8 && Sink::kTargets <= 2;
 }
 
-template <int P, class Sink>
+template <int P, class Sink, bool kStats>
 __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(tile_three_waves<P, Sink>() ? 3 : 1,
                                                                        tile_three_waves<P, Sink>() ? 3 : 2))) void knn_tile_kernel(
     BvhView bv, QueryView qv, TileParams prm, Sink sink)
@@ -676,9 +724,8 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(tile_thre
     const int lane = lane_id();
     const int g = lane / P, s = lane % P;
     float r2 = fmaxf(prm.r2_init, 1e-30f);
-    WaveStats ws;
+    WaveStats<kStats> ws;
     ws.clear();
-    ws.timing = prm.stats != nullptr;
     const auto t_wave = ws.tick();
     give_lds(sink, sm.cand, 0);
     if (lane < LEAF) sm.cand[CAP + lane] = make_float4(__builtin_nanf(""), __builtin_nanf(""), __builtin_nanf(""), 0.0f);
@@ -698,21 +745,12 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(tile_thre
     const int xcd = (int)(blockIdx.x % QUEUE_SEGS);
     int seg_k = 0;
     int64_t run = -1;
+    // a grid sized for an upper bound of the list: the first nruns waves are enough, so the others
+    // leave the queue's counters alone
+    if (prm.queue && (int64_t)blockIdx.x >= nruns) return;
     for (;;) {
         if (prm.queue) {
-            run = -1;
-            while (seg_k < QUEUE_SEGS) {
-                const int seg = (xcd + seg_k) % QUEUE_SEGS;
-                uint32_t r = 0;
-                if (lane == 0) r = atomicAdd(prm.queue + seg * QUEUE_STRIDE, 1u);
-                r = (uint32_t)__builtin_amdgcn_readlane((int)r, 0);
-                const int64_t cand = ((int64_t)(r / QUEUE_CHUNK) * QUEUE_SEGS + seg) * QUEUE_CHUNK + r % QUEUE_CHUNK;
-                if (cand < nruns) {
-                    run = cand;
-                    break;
-                }
-                seg_k++;  // this XCD's runs only grow with r: all taken
-            }
+            run = queue_take(prm.queue, nruns, xcd, seg_k);
             if (run < 0) break;
         } else {
             run = run < 0 ? (int64_t)blockIdx.x : run + gridDim.x;
@@ -742,7 +780,7 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(tile_thre
         const float qz = valid ? qv.qz[qpos] : 0.0f;
         const int scan = (valid && bv.scan_of) ? (int)bv.scan_of[qpos] : 0;
         bool active = valid && prm.t0 > 0;
-        ws.c[KS_TILES] += 1;
+        ws.add(KS_TILES, 1);
         if (prm.hint_in) {
             // the earlier target's neighbourhood of each query, grown for this one
             const float h = uniformf(wave_max(valid ? prm.hint_in[qpos] : 0.0f));
@@ -764,7 +802,7 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(tile_thre
             if (h > 0.0f && h < 1e37f) r2 = h;
         }
         if (tt == 1 && prm.tiles_per_wave > 2) {
-            const auto t0 = ws.tick();
+            [[maybe_unused]] const auto t0 = ws.tick();
             const int64_t q0 = qbase, q1 = min((run + 1) * prm.tiles_per_wave * Q, (int64_t)nq);
             const uint32_t p0 = qv.qsel ? qv.qsel[q0] : (uint32_t)q0;
             run_scan = bv.scan_of ? uniform((int)bv.scan_of[p0]) : 0;
@@ -840,13 +878,13 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(tile_thre
             tb.hy = uniformf(wave_max(act ? qy : -INFINITY));
             tb.hz = uniformf(wave_max(act ? qz : -INFINITY));
             const float R2 = r2;
-            ws.c[KS_ATTEMPTS] += 1;
+            ws.add(KS_ATTEMPTS, 1);
 
             // --- candidate leaves of the tile -------------------------------------------------
             Cands cs;
             float rej = INFINITY;  // nearest box the traversal left out
             {
-                const auto t0 = ws.tick();
+                [[maybe_unused]] const auto t0 = ws.tick();
                 int sp = 0, nl = 0;
                 if (run_ok && cur == run_scan && R2 <= run_r2 && tb.lx >= rbox.lx && tb.ly >= rbox.ly &&
                     tb.lz >= rbox.lz && tb.hx <= rbox.hx && tb.hy <= rbox.hy && tb.hz <= rbox.hz) {
@@ -924,13 +962,13 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(tile_thre
                     }
                 });
                 ws.tock(KS_CY_HIST, t0);
-                if (prm.stats) ws.c[KS_CANDIDATES] += (unsigned)(LEAF * wave_sum_int(s == 0 ? len : 0));
+                if constexpr (kStats) ws.add(KS_CANDIDATES, (unsigned)(LEAF * wave_sum_int(s == 0 ? len : 0)));
             });
             if (!fine) {
                 if (lane == 0) atomicMax(prm.err, 5);
                 return;
             }
-            if (cs.resident) ws.c[KS_RESIDENT] += 1;
+            if (cs.resident) ws.add(KS_RESIDENT, 1);
 
             // --- targets -----------------------------------------------------------------------
             const auto t_sel = ws.tick();
@@ -976,7 +1014,7 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(tile_thre
                 for (int guard = 0; guard < 16; guard++) {
                     const bool need = ok && tg[tau].refine;
                     if (ballot(need) == 0) break;
-                    ws.c[KS_REFINE] += 1;
+                    ws.add(KS_REFINE, 1);
                     const uint64_t span = tg[tau].khi - tg[tau].klo;
                     const int nbits = span ? 64 - __clzll((long long)span) : 0;
                     const int shift = nbits > nbb ? nbits - nbb : 0;
@@ -1095,7 +1133,8 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(tile_thre
                         for (int i = 0; i < nb; i++) rank += sm.bkey[tau][g][i] < kj ? 1 : 0;
                         if (rank < need) {
                             const uint32_t sp_ = bv.rank[(uint32_t)kj];
-                            sink.accept(tau, g, s, bv.px[sp_], bv.py[sp_], bv.pz[sp_], kj, sp_, sm.scnt[tau]);
+                            const float4 p = bv.pts4[sp_];  // one 16-byte load
+                            sink.accept(tau, g, s, p.x, p.y, p.z, kj, sp_, sm.scnt[tau]);
                         }
                         if (tau == 0 && rank == need - 1) kth = bitsf((uint32_t)(kj >> 32));
                     }
@@ -1115,7 +1154,7 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(tile_thre
             kth_max = fmaxf(kth_max, uniformf(wave_max(est)));
             const float disc_ok = uniformf(wave_max((ok && kth >= 0.0f) ? kth - dm : 0.0f));
             if (disc_ok > 0.0f) disc_hint = disc_ok;
-            ws.c[KS_RESOLVED] += (unsigned)__popcll(ballot(ok && s == 0));
+            ws.add(KS_RESOLVED, (unsigned)__popcll(ballot(ok && s == 0)));
             active = active && !ok;
             if (ballot(act && !ok) != 0) {  // queries of this scan still short of t: grow R
                 // Each short query estimates the radius^2 that holds t0 points from what it saw:

@@ -94,7 +94,7 @@ __device__ __forceinline__ float ord_dec(uint32_t e)
 }
 
 // per scan box (encoded): box[6 s + 0..2] = min, [6 s + 3..5] = max; cleared by box_init_kernel
-__global__ void box_init_kernel(uint32_t* __restrict__ box, int ns)
+static __global__ void box_init_kernel(uint32_t* __restrict__ box, int ns)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < 6 * ns) box[i] = (i % 6) < 3 ? 0xFFFFFFFFu : 0u;
@@ -104,7 +104,7 @@ constexpr int SB_ITEMS = 16;  // points per lane
 
 // One wave per 64 * SB_ITEMS consecutive input points: reduced in registers and merged with one
 // atomic per coordinate when they belong to one scan, per point otherwise.
-__global__ __launch_bounds__(256) void scan_bbox_kernel(const float* __restrict__ xyz, int64_t n,
+static __global__ __launch_bounds__(256) void scan_bbox_kernel(const float* __restrict__ xyz, int64_t n,
                                                         const int64_t* __restrict__ off, int ns,
                                                         uint32_t* __restrict__ box)
 {
@@ -154,7 +154,7 @@ __global__ __launch_bounds__(256) void scan_bbox_kernel(const float* __restrict_
 }
 
 // Morton frame of each scan: its box corner, a cubic cell size over the largest extent.
-__global__ void scan_frames_kernel(const uint32_t* __restrict__ box, int ns, MortonFrame* __restrict__ frames)
+static __global__ void scan_frames_kernel(const uint32_t* __restrict__ box, int ns, MortonFrame* __restrict__ frames)
 {
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
     if (s >= ns) return;
@@ -172,7 +172,7 @@ __global__ void scan_frames_kernel(const uint32_t* __restrict__ box, int ns, Mor
 
 // Sort keys of the input points: the 63-bit Morton code in the scan's own frame; with more
 // than one scan, the scan index in the top 16 bits above the code's leading 48 bits.
-__global__ __launch_bounds__(256) void morton_scan_kernel(const float* __restrict__ xyz, int64_t n,
+static __global__ __launch_bounds__(256) void morton_scan_kernel(const float* __restrict__ xyz, int64_t n,
                                                           const int64_t* __restrict__ off, int ns,
                                                           const MortonFrame* __restrict__ frames,
                                                           uint64_t* __restrict__ keys, uint32_t* __restrict__ vals)
@@ -188,7 +188,7 @@ __global__ __launch_bounds__(256) void morton_scan_kernel(const float* __restric
 // Padded sorted SoA layout, one thread per padded position p: the point (NaN for padding),
 // its input index (~0 for padding), the inverse permutation, the sort key, the list of real
 // positions in sort order, and the scan of each position.
-__global__ __launch_bounds__(256) void gather_padded_kernel(
+static __global__ __launch_bounds__(256) void gather_padded_kernel(
     const float* __restrict__ xyz, const int64_t* __restrict__ off, const int64_t* __restrict__ pstart, int ns,
     int64_t npad, const uint32_t* __restrict__ order, const uint64_t* __restrict__ skeys, float* __restrict__ px,
     float* __restrict__ py, float* __restrict__ pz, uint32_t* __restrict__ pidx, uint32_t* __restrict__ rank,
@@ -221,7 +221,7 @@ __global__ __launch_bounds__(256) void gather_padded_kernel(
 }
 
 // Leaf boxes: one lane per point, LEAF lanes per leaf; also the leaf codes.
-__global__ __launch_bounds__(256) void leaf_boxes_kernel(const float* __restrict__ px, const float* __restrict__ py,
+static __global__ __launch_bounds__(256) void leaf_boxes_kernel(const float* __restrict__ px, const float* __restrict__ py,
                                                          const float* __restrict__ pz, int64_t n,
                                                          const uint64_t* __restrict__ codes, int nleaf,
                                                          float4* __restrict__ leaf_lo, float4* __restrict__ leaf_hi,
@@ -257,7 +257,7 @@ __global__ __launch_bounds__(256) void leaf_boxes_kernel(const float* __restrict
 // agg[3 l + 2] = (yz, zz, 0, 0) of sum (p - c)(p - c)^T.  One thread per leaf.
 __device__ __forceinline__ float leaf_centre(float lo, float hi) { return (lo + hi) * 0.5f; }
 
-__global__ __launch_bounds__(256) void leaf_sums_kernel(const float* __restrict__ px, const float* __restrict__ py,
+static __global__ __launch_bounds__(256) void leaf_sums_kernel(const float* __restrict__ px, const float* __restrict__ py,
                                                         const float* __restrict__ pz, int64_t n,
                                                         const float4* __restrict__ leaf_lo,
                                                         const float4* __restrict__ leaf_hi, int nleaf,
@@ -298,7 +298,7 @@ __device__ __forceinline__ int karras_delta(const uint64_t* codes, int nl, int i
     return 64 + __clz((int)((uint32_t)i ^ (uint32_t)j));
 }
 
-__global__ __launch_bounds__(256) void karras_kernel(const uint64_t* __restrict__ codes, int nl,
+static __global__ __launch_bounds__(256) void karras_kernel(const uint64_t* __restrict__ codes, int nl,
                                                      BvhNode* __restrict__ nodes, int* __restrict__ leaf_parent)
 {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -364,7 +364,7 @@ __device__ __forceinline__ void put_child_box(BvhNode* nd, bool left, const floa
     }
 }
 
-__global__ __launch_bounds__(256) void refit_leaf_slots_kernel(int nl, const int* __restrict__ leaf_parent,
+static __global__ __launch_bounds__(256) void refit_leaf_slots_kernel(int nl, const int* __restrict__ leaf_parent,
                                                                const float4* __restrict__ leaf_lo,
                                                                const float4* __restrict__ leaf_hi, BvhNode* nodes)
 {
@@ -376,7 +376,7 @@ __global__ __launch_bounds__(256) void refit_leaf_slots_kernel(int nl, const int
 }
 
 // level j of the doubling table from level j - 1 (half = 2^(j-1)); entries i <= nl - 2 * half
-__global__ __launch_bounds__(256) void range_union_level_kernel(int nl, int half, const float4* __restrict__ lo_in,
+static __global__ __launch_bounds__(256) void range_union_level_kernel(int nl, int half, const float4* __restrict__ lo_in,
                                                                 const float4* __restrict__ hi_in,
                                                                 float4* __restrict__ lo_out, float4* __restrict__ hi_out)
 {
@@ -388,7 +388,7 @@ __global__ __launch_bounds__(256) void range_union_level_kernel(int nl, int half
 }
 
 // the internal nodes whose leaf count has floor(log2) == j: own box, and the parent's child slot
-__global__ __launch_bounds__(256) void refit_level_kernel(int nint, int j, const float4* __restrict__ tlo,
+static __global__ __launch_bounds__(256) void refit_level_kernel(int nint, int j, const float4* __restrict__ tlo,
                                                           const float4* __restrict__ thi, BvhNode* nodes,
                                                           float4* __restrict__ node_lo, float4* __restrict__ node_hi)
 {
@@ -407,14 +407,14 @@ __global__ __launch_bounds__(256) void refit_level_kernel(int nint, int j, const
     if (r.z >= 0) put_child_box(&nodes[r.z], nodes[r.z].r.x == i, lo, hi);
 }
 
-__global__ void fill_u32_kernel(uint32_t* p, int64_t n, uint32_t v)
+static __global__ void fill_u32_kernel(uint32_t* p, int64_t n, uint32_t v)
 {
     int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) p[i] = v;
 }
 
 // BvhNode4 of every internal node.  One thread per node.
-__global__ __launch_bounds__(256) void node4_kernel(const BvhNode* __restrict__ nodes, int nint,
+static __global__ __launch_bounds__(256) void node4_kernel(const BvhNode* __restrict__ nodes, int nint,
                                                     BvhNode4* __restrict__ node4)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -463,7 +463,7 @@ constexpr int FRONTIER_LEVELS = 8;
 constexpr int FRONTIER = 1 << FRONTIER_LEVELS;
 constexpr int FR_NONE = (int)0x80000000;  // an empty slot
 
-__global__ __launch_bounds__(FRONTIER) void frontier_kernel(const BvhNode* __restrict__ nodes,
+static __global__ __launch_bounds__(FRONTIER) void frontier_kernel(const BvhNode* __restrict__ nodes,
                                                             const float4* __restrict__ leaf_lo,
                                                             const float4* __restrict__ leaf_hi, int nleaf,
                                                             const int* __restrict__ roots, int* __restrict__ fr_ref,
@@ -529,7 +529,7 @@ __global__ __launch_bounds__(FRONTIER) void frontier_kernel(const BvhNode* __res
 // Root of each scan's subtree: scan s covers leaves [pstart[s] / LEAF, pstart[s+1] / LEAF), a
 // contiguous run sharing the scan's key prefix, which in a radix tree is exactly the leaf
 // range of one node (the lowest ancestor of its first leaf that reaches its last leaf).
-__global__ void scan_roots_kernel(const int64_t* __restrict__ pstart, int ns, const int* __restrict__ leaf_parent,
+static __global__ void scan_roots_kernel(const int64_t* __restrict__ pstart, int ns, const int* __restrict__ leaf_parent,
                                   const BvhNode* __restrict__ nodes, int* __restrict__ roots)
 {
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
@@ -552,7 +552,7 @@ __global__ void scan_roots_kernel(const int64_t* __restrict__ pstart, int ns, co
 // Median of n <= 8192 samples (bitonic sort in LDS, one block of 1024 threads): out = the
 // element of rank n / 2.
 constexpr int MEDIAN_MAX = 8192;
-__global__ __launch_bounds__(1024) void median_kernel(const float* __restrict__ v, int n, float* __restrict__ out)
+static __global__ __launch_bounds__(1024) void median_kernel(const float* __restrict__ v, int n, float* __restrict__ out)
 {
     __shared__ float a[MEDIAN_MAX];
     for (int i = threadIdx.x; i < MEDIAN_MAX; i += blockDim.x) a[i] = i < n ? v[i] : INFINITY;

@@ -6,6 +6,7 @@
 #include "lbvh.hpp"
 #include "knn_tile.hpp"
 #include "sinks.hpp"
+#include "tile_launch.hpp"
 #include "knn_bestfirst.hpp"
 #include "adjoint.hpp"
 #include "lattice.hpp"
@@ -513,24 +514,6 @@ void launch_bf_wave(const BvhView& bv, const float* qx, const float* qy, const f
     LVRHIP_LAUNCH_CHECK();
 }
 
-// ki list without normals (used when ki > 2*kn, so the first normal round cannot supply it);
-// unordered, like the one written by SinkNormals.
-template <int P>
-struct SinkKiOnly {
-    static constexpr int kTargets = 2;
-    uint32_t* out;
-    int kw;
-    uint32_t qpos_;
-    __device__ __forceinline__ void begin(int, int, int64_t, uint32_t qpos, float, float, float) { qpos_ = qpos; }
-    __device__ __forceinline__ void accept(int tau, int g, int, float, float, float, uint64_t, uint32_t sp, uint32_t* cnt)
-    {
-        if (tau != 0) return;
-        const uint32_t slot = atomicAdd(&cnt[g], 1u);
-        if (slot < (uint32_t)kw) out[(size_t)qpos_ * kw + slot] = sp;
-    }
-    __device__ __forceinline__ void finish(int, int, bool, uint32_t, float, float, float, const uint32_t*, const uint32_t*) {}
-};
-
 // hipEvent pairs around kernels on the handle's stream, accumulated per timer.
 struct Profiler {
     bool on = false;
@@ -589,25 +572,6 @@ struct Profiler {
         for (auto e : pool) (void)hipEventDestroy(e);
     }
 };
-
-// With a work queue the grid is capped at `resident` waves (the ones the device holds at once):
-// they drain the queue; without, one wave per run of tiles.
-template <int P, template <int> class SinkT>
-void launch_tile_p(const BvhView& bv, const QueryView& qv, const TileParams& prm, const SinkT<P>& sink,
-                   hipStream_t st, int64_t resident)
-{
-    constexpr int Q = kWave / P;
-    const int64_t ntiles = ceil_div(qv.nq, Q);
-    int64_t grid = ceil_div(ntiles, prm.tiles_per_wave);
-    if (grid == 0) return;
-    if (prm.queue) {
-        grid = std::min(grid, resident);
-        fill_u32_kernel<<<1, 256, 0, st>>>(prm.queue, QUEUE_SEGS * QUEUE_STRIDE, 0u);
-        LVRHIP_LAUNCH_CHECK();
-    }
-    knn_tile_kernel<P, SinkT<P>><<<(unsigned)grid, kWave, 0, st>>>(bv, qv, prm, sink);
-    LVRHIP_LAUNCH_CHECK();
-}
 
 // ---- the no-allocation signed distances (lvrhip_distances_device_noalloc) -----------------------
 // Its scratch lives in one file-scope device array, `scratch`, that every device holds from the

@@ -18,7 +18,7 @@ constexpr int RS_ITEMS = 16;
 constexpr int RS_TILE = RS_THREADS * RS_ITEMS;
 constexpr int RS_RADIX = 256;
 
-__global__ __launch_bounds__(RS_THREADS) void rs_hist_kernel(const uint64_t* __restrict__ keys, int64_t n, int shift,
+static __global__ __launch_bounds__(RS_THREADS) void rs_hist_kernel(const uint64_t* __restrict__ keys, int64_t n, int shift,
                                                               uint32_t* __restrict__ ghist, int ntiles)
 {
     __shared__ uint32_t h[RS_RADIX];
@@ -78,7 +78,7 @@ __device__ __forceinline__ uint32_t scan_segment(uint32_t* __restrict__ a, int64
 }
 
 // In-place exclusive scan of a[0..len) with one 1024-thread block, one segment per step.
-__global__ __launch_bounds__(1024) void scan_exclusive_kernel(uint32_t* __restrict__ a, int64_t len,
+static __global__ __launch_bounds__(1024) void scan_exclusive_kernel(uint32_t* __restrict__ a, int64_t len,
                                                               uint32_t* __restrict__ total)
 {
     __shared__ uint32_t wsum[16];
@@ -90,7 +90,7 @@ __global__ __launch_bounds__(1024) void scan_exclusive_kernel(uint32_t* __restri
 // Multi-block form for long tables (the radix sort's digit table: 256 entries per 4096 keys):
 // (1) each block sums its segment, (2) one block scans the segment sums, (3) each block scans
 // its segment from its carry.
-__global__ __launch_bounds__(1024) void scan_segsum_kernel(const uint32_t* __restrict__ a, int64_t len,
+static __global__ __launch_bounds__(1024) void scan_segsum_kernel(const uint32_t* __restrict__ a, int64_t len,
                                                            uint32_t* __restrict__ sums)
 {
     __shared__ uint32_t wsum[16];
@@ -113,7 +113,7 @@ __global__ __launch_bounds__(1024) void scan_segsum_kernel(const uint32_t* __res
     }
 }
 
-__global__ __launch_bounds__(1024) void scan_segapply_kernel(uint32_t* __restrict__ a, int64_t len,
+static __global__ __launch_bounds__(1024) void scan_segapply_kernel(uint32_t* __restrict__ a, int64_t len,
                                                              const uint32_t* __restrict__ carry)
 {
     __shared__ uint32_t wsum[16];
@@ -144,7 +144,7 @@ inline void scan_exclusive(uint32_t* a, int64_t len, uint32_t* sums, hipStream_t
     LVRHIP_LAUNCH_CHECK();
 }
 
-__global__ __launch_bounds__(RS_THREADS) void rs_scatter_kernel(const uint64_t* __restrict__ kin,
+static __global__ __launch_bounds__(RS_THREADS) void rs_scatter_kernel(const uint64_t* __restrict__ kin,
                                                                  const uint32_t* __restrict__ vin,
                                                                  uint64_t* __restrict__ kout,
                                                                  uint32_t* __restrict__ vout, int64_t n, int shift,

@@ -14,6 +14,8 @@
 
 #include "common.hpp"
 #include "eig3.hpp"
+#include "knn_tile.hpp"
+#include "lbvh.hpp"
 
 namespace lvrhip {
 
@@ -344,7 +346,7 @@ struct SinkLevels {
 
 // Adaptive-round counts of the queries of the merged later rounds: cnt[r] += #(kround >= r),
 // r = 3..5 (cnt[2], the queries themselves, comes from the compaction).
-__global__ __launch_bounds__(256) void round_count_kernel(const uint32_t* __restrict__ qsel,
+static __global__ __launch_bounds__(256) void round_count_kernel(const uint32_t* __restrict__ qsel,
                                                           const uint32_t* __restrict__ nq_dev, int64_t nq,
                                                           const uint8_t* __restrict__ kround, uint32_t* __restrict__ cnt)
 {
@@ -388,7 +390,7 @@ struct PlaneFitParams {
     int round;
 };
 
-__global__ __launch_bounds__(256) void plane_fit_kernel(PlaneFitParams a)
+static __global__ __launch_bounds__(256) void plane_fit_kernel(PlaneFitParams a)
 {
     const int64_t qi = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const int64_t nq = a.nq_dev ? (int64_t)*a.nq_dev : a.nq;
@@ -578,6 +580,24 @@ struct SinkList {
         if (tau != 0) return;
         const uint32_t slot = atomicAdd(&cnt[g], 1u);
         if (slot < (uint32_t)kw) out[(size_t)row_ * kw + slot] = key;
+    }
+    __device__ __forceinline__ void finish(int, int, bool, uint32_t, float, float, float, const uint32_t*, const uint32_t*) {}
+};
+
+// ki list without normals (used when ki > 2*kn, so the first normal round cannot supply it);
+// unordered, like the one written by SinkNormals.
+template <int P>
+struct SinkKiOnly {
+    static constexpr int kTargets = 2;
+    uint32_t* out;
+    int kw;
+    uint32_t qpos_;
+    __device__ __forceinline__ void begin(int, int, int64_t, uint32_t qpos, float, float, float) { qpos_ = qpos; }
+    __device__ __forceinline__ void accept(int tau, int g, int, float, float, float, uint64_t, uint32_t sp, uint32_t* cnt)
+    {
+        if (tau != 0) return;
+        const uint32_t slot = atomicAdd(&cnt[g], 1u);
+        if (slot < (uint32_t)kw) out[(size_t)qpos_ * kw + slot] = sp;
     }
     __device__ __forceinline__ void finish(int, int, bool, uint32_t, float, float, float, const uint32_t*, const uint32_t*) {}
 };
