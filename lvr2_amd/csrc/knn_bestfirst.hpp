@@ -9,11 +9,17 @@
 // (AdaptiveKSearchSurface.tcc:414-457, called from PointsetGrid.tcc:123-149) and
 // SearchKDTree::kSearch / radiusSearch (KDTree.tcc:331-387) for k <= BF_KMAX.
 //
-//   1. A greedy descent from the root to the leaf whose box is nearest at every level; its
-//      points seed the list, so the bound is finite before anything is pushed.
-//   2. Best-first from the root over BvhNode4 (four grandchildren per node): children within
-//      the bound are pushed farthest first, each with its box distance, onto a per-lane LDS
-//      stack; a popped entry beyond the (meanwhile tightened) bound is dropped.
+// A lane keeps a pool of subtrees not yet entered, each with a lower bound of its distance.  A step
+// takes the nearest of them and descends from it, always to the nearest child (BvhNode4: four
+// grandchildren per node), until it reaches a leaf; what is left of every node passed (its other
+// children within the bound) goes into the pool as one entry.  The search ends when the pool's nearest
+// entry is beyond the t-th key.
+// The order decides the work: a depth-first stack (nearest child first) returns to the siblings of
+// its first leaf, near the query or not, while the bound is still wide.  On the lattice vertices of the
+// 4M-point room (t = 10) that scanned 21 leaves and expanded about 50 nodes per query; taking the nearest
+// pool entry after every leaf scans 8.6 and expands 37 (a strict best-first queue: 7.7 and 25, but it
+// holds four times the entries).  Signed distances at 700,000 vertices of that lattice, sort included:
+// 5.17 -> 1.19 ms.
 // The few queries whose lane stack overflows (hundreds of leaves within their bound) are searched
 // again by a whole wave each (bf_knn_wave_kernel), and the tile kernel takes any that outgrow
 // that stack too.
@@ -30,135 +36,160 @@
 namespace lvrhip {
 
 constexpr int BF_THREADS = 64;  // one wave per workgroup
-constexpr int BF_STACK = 16;    // stack entries per lane (ref, box d^2) in LDS: 8 KB per wave
-constexpr int BF_SPILL = 48;    // further entries per lane in global memory (deep traversals only)
-
-// A lane's traversal stack: CAP entries of (node or leaf reference, box d^2 bits).
-// The first BF_STACK entries in LDS (the pointer carries the LDS address space, so that the
-// two parts are never addressed through one generic pointer), the rest in global memory.
-typedef __attribute__((address_space(3))) uint2 lds_uint2;
-struct BfLdsStack {
-    lds_uint2* s;  // this lane's LDS entries, interleaved with the wave's other lanes
-    uint2* spill;  // this lane's spill entries, interleaved likewise
-    int cap;       // BF_STACK + the spill entries per lane
-    __device__ __forceinline__ int capacity() const { return cap; }
-    __device__ __forceinline__ uint2 get(int i) const
-    {
-        uint2 v;
-        if (i < BF_STACK) {
-            const lds_uint2& e = s[i * BF_THREADS];
-            v.x = e.x;
-            v.y = e.y;
-        } else {
-            v = spill[(size_t)(i - BF_STACK) * BF_THREADS];
-        }
-        return v;
-    }
-    __device__ __forceinline__ void put(int i, uint2 v) const
-    {
-        if (i < BF_STACK) {
-            lds_uint2& e = s[i * BF_THREADS];
-            e.x = v.x;
-            e.y = v.y;
-        } else {
-            spill[(size_t)(i - BF_STACK) * BF_THREADS] = v;
-        }
-    }
+// A lane's pool: BF_POOL entries in LDS, then BF_SPILL more in global memory (a few lanes in 10,000).
+// An entry is a node with the mask of its children still to be entered (the top 4 bits), and the upper
+// 16 bits of the smallest of their box distances: rounded towards zero, so still a lower bound.  24
+// entries of 6 bytes are 9.2 KB per wave: 17 waves per CU by LDS (99 % of the room's queries never hold
+// more than 21).
+constexpr int BF_POOL = 24;
+constexpr int BF_SPILL = 40;
+constexpr uint32_t BF_NODE_MASK = 0x0FFFFFFFu;  // node index of an entry (n < 2^32 points: nodes < 2^28)
+typedef uint32_t __attribute__((may_alias)) bf_word;  // two 16-bit distances read as one word
+struct BfPool {
+    uint32_t ref[BF_POOL][BF_THREADS];
+    alignas(4) uint16_t d[BF_POOL / 2][BF_THREADS][2];  // slots 2 w and 2 w + 1 of a lane share a word; 0xFFFF: free
 };
 
 constexpr int BF_KMAX = 32;
 // key of an empty list slot: above every key of a finite d^2 (and of d^2 = inf with a real index)
 constexpr uint64_t BF_EMPTY = 0x7F800000FFFFFFFFull;
+constexpr uint64_t BF_NONE = 0x7FE0000000000000ull;  // no candidate: above every key, a finite double
 
-// The t smallest keys seen so far, ascending in key[K - t, K).  The slots below K - t hold 0,
-// which no candidate displaces (candidates enter by a strict comparison), so the t-th key is
-// always key[K - 1] and every index into the arrays is a compile-time constant.
+// Keys as doubles.  A key's upper word is a non-negative float's bits (at most 0x7F800000), so as a
+// double it is positive and finite, and doubles order like the 64-bit integers they are made of: a
+// compare-exchange is one v_min_f64 and one v_max_f64 (full rate on gfx950) where 64-bit integers take a
+// compare and four selects.  Tiny keys (d^2 = 0) are denormal doubles, which the double unit keeps.
+__device__ __forceinline__ double bf_as_f64(uint64_t k) { return __longlong_as_double((long long)k); }
+__device__ __forceinline__ uint64_t bf_as_u64(double k) { return (uint64_t)__double_as_longlong(k); }
+__device__ __forceinline__ double bf_min(double a, double b)
+{
+    double r;
+    asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+__device__ __forceinline__ double bf_max(double a, double b)
+{
+    double r;
+    asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+__device__ __forceinline__ void bf_cas(double& a, double& b)
+{
+    const double lo = bf_min(a, b), hi = bf_max(a, b);
+    a = lo;
+    b = hi;
+}
+
+// Batcher's odd-even merge sort of c[0, 16) (63 compare-exchanges).
+__device__ __forceinline__ void bf_sort16(double (&c)[16])
+{
+#pragma unroll
+    for (int p = 1; p < 16; p *= 2)
+#pragma unroll
+        for (int k = p; k >= 1; k /= 2)
+#pragma unroll
+            for (int j = k % p; j + k < 16; j += 2 * k)
+#pragma unroll
+                for (int i = 0; i < k; i++)
+                    if (i + j + k < 16 && (i + j) / (2 * p) == (i + j + k) / (2 * p)) bf_cas(c[i + j], c[i + j + k]);
+}
+
+// Sort a bitonic sequence (ascending, then descending) in x[B, B + N), N <= 16.  It is taken as the end of
+// a 16-entry one whose first 16 - N entries are below every key: a compare-exchange with one of those
+// changes nothing and is left out.
+template <int B, int N, int SZ>
+__device__ __forceinline__ void bf_bitonic(double (&x)[SZ])
+{
+    constexpr int PAD = 16 - N;
+#pragma unroll
+    for (int d = 8; d >= 1; d /= 2)
+#pragma unroll
+        for (int i = PAD; i < 16; i++)
+            if ((i & d) == 0 && i + d < 16) bf_cas(x[B + i - PAD], x[B + i + d - PAD]);
+}
+
+// The t smallest keys seen so far, ascending in key[K - t, K).  The slots below K - t hold 0, which
+// stays first, so the t-th key is always key[K - 1] and every index into the arrays is a compile-time
+// constant.  Unfilled slots hold `empty`, above every key that may enter.
 template <int K>
 struct BfList {
-    uint64_t key[K];
-    uint32_t sp[K];  // sorted position of each key's point (~0: empty)
+    static_assert(K <= 16 || K == 32, "list lengths up to 16, or 32");
+    double k[K];
+    uint64_t key[K];  // after finish(): the keys, and
+    uint32_t sp[K];   // the sorted position of each key's point (~0: empty)
+    uint64_t empty;
 
-    __device__ __forceinline__ void init(int t, uint64_t empty)
+    __device__ __forceinline__ void init(int t, uint64_t e)
+    {
+        empty = e;
+#pragma unroll
+        for (int j = 0; j < K; j++) k[j] = bf_as_f64(j < K - t ? 0ull : e);
+    }
+    __device__ __forceinline__ uint64_t worst() const { return bf_as_u64(k[K - 1]); }
+    // d^2 of the t-th key: the pruning bound
+    __device__ __forceinline__ float bound() const { return bitsf((uint32_t)(worst() >> 32)); }
+    // every one of the t slots holds a point
+    __device__ __forceinline__ bool full() const { return sp[K - 1] != ~0u; }
+
+    // the K smallest of the list and the 16 sorted candidates c
+    __device__ __forceinline__ void merge(const double (&c)[16])
+    {
+        if constexpr (K <= 16) {
+#pragma unroll
+            for (int i = 0; i < K; i++) k[i] = bf_min(k[i], c[K - 1 - i]);
+            bf_bitonic<0, K>(k);
+        } else {
+            // the candidates against the larger half, then the halves against each other
+#pragma unroll
+            for (int i = 0; i < 16; i++) k[16 + i] = bf_min(k[16 + i], c[15 - i]);
+            bf_bitonic<16, 16>(k);
+#pragma unroll
+            for (int i = 0; i < 8; i++) {  // k[i] with k[31 - i]: both halves become bitonic
+                bf_cas(k[i], k[31 - i]);
+                bf_cas(k[15 - i], k[16 + i]);
+            }
+            bf_bitonic<0, 16>(k);
+            bf_bitonic<16, 16>(k);
+        }
+    }
+
+    // keys and sorted positions for the consumer
+    __device__ __forceinline__ void finish(const uint32_t* __restrict__ rank, int t)
     {
 #pragma unroll
         for (int j = 0; j < K; j++) {
-            key[j] = j < K - t ? 0ull : empty;
-            sp[j] = ~0u;
-        }
-    }
-    __device__ __forceinline__ uint64_t worst() const { return key[K - 1]; }
-    // every one of the t slots holds a point (unfilled slots hold the largest keys)
-    __device__ __forceinline__ bool full() const { return sp[K - 1] != ~0u; }
-    // d^2 of the t-th key: the pruning bound
-    __device__ __forceinline__ float bound() const { return bitsf((uint32_t)(key[K - 1] >> 32)); }
-    __device__ __forceinline__ bool contains(uint64_t c) const
-    {
-        bool f = false;
-#pragma unroll
-        for (int j = 0; j < K; j++) f = f || key[j] == c;
-        return f;
-    }
-
-    // insert c (c < worst()), dropping the largest
-    __device__ __forceinline__ void insert(uint64_t c, uint32_t s)
-    {
-        bool ltp = c < key[0];
-        uint64_t pk = key[0];
-        uint32_t ps = sp[0];
-        key[0] = ltp ? c : pk;
-        sp[0] = ltp ? s : ps;
-#pragma unroll
-        for (int j = 1; j < K; j++) {
-            const bool lt = c < key[j];
-            const uint64_t kj = key[j];
-            const uint32_t sj = sp[j];
-            key[j] = lt ? (ltp ? pk : c) : kj;
-            sp[j] = lt ? (ltp ? ps : s) : sj;
-            pk = kj;
-            ps = sj;
-            ltp = lt;
+            key[j] = bf_as_u64(k[j]);
+            sp[j] = j >= K - t && key[j] < empty ? rank[(uint32_t)key[j]] : ~0u;
         }
     }
 };
 
-// The leaf's points whose key beats the current t-th enter the list smallest first: each round
-// finds the smallest remaining candidate (compile-time indices only) and inserts it, so a wave
-// runs as many insertion rounds as its busiest lane has improving points, not one per point.
-// kDedup: the list may already hold some of the leaf's points (a search started from a known
-// neighbour set); those are not inserted twice.
-template <int K, bool kDedup = false>
+// The leaf's points whose key beats the current t-th: sorted by a network and merged into the list, with
+// no loop and no branch per point (the search's leaf work is the same for every lane of the wave; taking
+// the points in one by one had run as many rounds as the busiest lane had improving points).
+template <int K>
 __device__ __forceinline__ void bf_scan_leaf(const BvhView& bv, int leaf, float qx, float qy, float qz, BfList<K>& L)
 {
     const float4* p = bv.pts4 + (size_t)leaf * LEAF;
     float4 v[LEAF];
 #pragma unroll
     for (int j = 0; j < LEAF; j++) v[j] = p[j];
-    uint64_t c[LEAF];
+    static_assert(LEAF == 16, "the sorting network");
+    double c[LEAF];
     const uint64_t w = L.worst();
+    bool any = false;
 #pragma unroll
     for (int j = 0; j < LEAF; j++) {
         const float d = d2_contract(qx, qy, qz, v[j].x, v[j].y, v[j].z);
         const uint64_t key = make_key(d, fbits(v[j].w));
-        // padding slots have NaN coordinates: never a neighbour
-        c[j] = (d == d && key < w) ? key : ~0ull;
+        // padding slots have NaN coordinates: their keys are above every bound
+        const bool in = key < w;
+        any = any || in;
+        c[j] = bf_as_f64(in ? key : BF_NONE);
     }
-    // Keys are unique (they end in the point's index), so each round takes the smallest key above
-    // the previous round's instead of clearing the taken slot: the same sequence of insertions.
-    uint64_t lo = 0;
-    for (int round = 0; round < LEAF; round++) {
-        uint64_t best = ~0ull;
-        int bj = 0;
-#pragma unroll
-        for (int j = 0; j < LEAF; j++) {
-            if (c[j] >= lo && c[j] < best) {
-                best = c[j];
-                bj = j;
-            }
-        }
-        if (!(best < L.worst())) break;  // the rest cannot enter (~0 marks none)
-        if (!kDedup || !L.contains(best)) L.insert(best, (uint32_t)(leaf * LEAF + bj));
-        lo = best + 1;  // best < worst <= ~0: no wrap
-    }
+    if (ballot(any) == 0) return;
+    bf_sort16(c);
+    L.merge(c);
 }
 
 __device__ __forceinline__ float bf_child_d2(const float* f, int k, float qx, float qy, float qz)
@@ -167,116 +198,153 @@ __device__ __forceinline__ float bf_child_d2(const float* f, int k, float qx, fl
                   qz);
 }
 
-// The search of one lane; returns false if its stack overflowed (the list is then incomplete).
-template <int K, bool kDedup, class Stack>
-__device__ __forceinline__ bool bf_search(const BvhView& bv, const Stack& stk, float qx, float qy, float qz,
-                                          BfList<K>& L, int& leaves, int& nodes)
+// The pool of lane `lane`: which slots are free, and how many entries were spilled.
+struct BfLane {
+    uint32_t free;  // bit i: slot i of the LDS pool is free
+    int nspill;
+    uint2* spill;  // this lane's spilled entries (ref, d), interleaved with the wave's other lanes
+    int spill_cap;
+};
+
+// Puts an entry into the pool; false if neither the LDS slots nor the spill area hold it.
+__device__ __forceinline__ bool bf_put(BfPool& pool, BfLane& ln, int lane, uint32_t ref, uint32_t d16, float bound)
 {
-    const int root = bv.nleaf > 1 ? 0 : leaf_ref(0);
-    // 1. greedy descent: the seed leaf
-    int ref = root;
-    while (ref >= 0) {
-        const BvhNode4 nd = bv.nodes4[ref];
-        const float* f = reinterpret_cast<const float*>(nd.b);
-        const int rr[4] = {nd.r.x, nd.r.y, nd.r.z, nd.r.w};
-        float best = INFINITY;
-        int next = rr[0];  // slot 0 always holds a child
+    if (ln.free == 0u) {  // drop the entries the bound has left behind
 #pragma unroll
-        for (int k = 0; k < 4; k++) {
-            const float d = bf_child_d2(f, k, qx, qy, qz);
-            if (rr[k] != EMPTY4 && d < best) {
-                best = d;
-                next = rr[k];
+        for (int i = 0; i < BF_POOL; i++) {
+            const uint32_t e = pool.d[i / 2][lane][i & 1];
+            if (bitsf(e << 16) > bound) {
+                ln.free |= 1u << i;
+                pool.d[i / 2][lane][i & 1] = 0xFFFFu;
             }
         }
-        ref = next;
     }
-    const int seed = -1 - ref;
-    bf_scan_leaf<K, kDedup>(bv, seed, qx, qy, qz, L);
-    leaves++;
-    if (root < 0) return true;
-    // 2. best-first from the root.  Each pass pops (expanding nodes) until the lane holds a leaf
-    // to scan, then the lanes scan their leaves together: leaf scans, the costly part, run with
-    // most lanes of the wave active instead of interleaving with other lanes' node expansions.
-    int sp = 0;
-    uint2 e = make_uint2((uint32_t)root, 0u);  // the entry to process next
-    bool have = true;                           // e holds an entry (else pop one)
+    if (ln.free == 0u) {
+        if (ln.nspill == ln.spill_cap) return false;
+        ln.spill[(size_t)ln.nspill * BF_THREADS] = make_uint2(ref, d16);
+        ln.nspill++;
+        return true;
+    }
+    const int slot = __ffs((int)ln.free) - 1;
+    ln.free &= ln.free - 1u;
+    pool.ref[slot][lane] = ref;
+    pool.d[slot / 2][lane][slot & 1] = (uint16_t)d16;
+    return true;
+}
+
+// Takes the nearest entry within the bound out of the pool; false if there is none.
+__device__ __forceinline__ bool bf_take(BfPool& pool, BfLane& ln, int lane, float bound, uint32_t& ref)
+{
     for (;;) {
+        // minimum of (d, slot) over all slots, two per LDS word; a free slot's d is above every bound
+        uint32_t m = ~0u;
+        const bf_word* w = reinterpret_cast<const bf_word*>(&pool.d[0][lane][0]);
+#pragma unroll
+        for (int i = 0; i < BF_POOL / 2; i++) {
+            const uint32_t x = w[i * BF_THREADS];
+            const uint32_t e0 = (x << 16) | (uint32_t)(2 * i), e1 = (x & 0xFFFF0000u) | (uint32_t)(2 * i + 1);
+            m = min(m, min(e0, e1));
+        }
+        if (bitsf(m & 0xFFFF0000u) <= bound) {  // (a free slot: NaN, never)
+            const int slot = (int)(m & 0xFFFFu);
+            ref = pool.ref[slot][lane];
+            pool.d[slot / 2][lane][slot & 1] = 0xFFFFu;
+            ln.free |= 1u << slot;
+            return true;
+        }
+        if (ln.nspill == 0) return false;
+        // every LDS entry is beyond the bound: free them all and bring spilled ones back
+#pragma unroll
+        for (int i = 0; i < BF_POOL; i++) pool.d[i / 2][lane][i & 1] = 0xFFFFu;
+        ln.free = (1u << BF_POOL) - 1u;
+        while (ln.nspill > 0 && ln.free != 0u) {
+            ln.nspill--;
+            const uint2 e = ln.spill[(size_t)ln.nspill * BF_THREADS];
+            const int slot = __ffs((int)ln.free) - 1;
+            ln.free &= ln.free - 1u;
+            pool.ref[slot][lane] = e.x;
+            pool.d[slot / 2][lane][slot & 1] = (uint16_t)e.y;
+        }
+    }
+}
+
+// The search of one lane; returns false if its pool overflowed (the list is then incomplete).
+template <int K>
+__device__ __forceinline__ bool bf_search(const BvhView& bv, BfPool& pool, BfLane& ln, int lane, float qx, float qy,
+                                          float qz, BfList<K>& L, int& leaves, int& nodes)
+{
+    constexpr int NONE = EMPTY4;
+    if (bv.nleaf <= 1) {
+        bf_scan_leaf<K>(bv, 0, qx, qy, qz, L);
+        leaves++;
+        return true;
+    }
+#pragma unroll
+    for (int i = 0; i < BF_POOL; i++) pool.d[i / 2][lane][i & 1] = 0xFFFFu;
+    ln.free = (1u << BF_POOL) - 1u;
+    ln.nspill = 0;
+    int cur = 0;          // the node to expand next (NONE: take one from the pool)
+    uint32_t want = 15u;  // its children still to be entered
+    for (;;) {
+        // descend until the lane holds a leaf; then the lanes scan their leaves together
         int leaf = -1;
+        const float bound = L.bound();
         for (;;) {
-            if (!have) {
-                if (sp == 0) break;
-                e = stk.get(--sp);
-            }
-            have = false;
-            const float bound = L.bound();
-            if (bitsf(e.y) > bound) continue;
-            const int r = (int)e.x;
-            if (r < 0) {
-                if (-1 - r != seed) {
-                    leaf = -1 - r;
-                    break;
-                }
-                continue;
+            if (cur == NONE) {
+                uint32_t e;
+                if (!bf_take(pool, ln, lane, bound, e)) break;
+                cur = (int)(e & BF_NODE_MASK);
+                want = e >> 28;
             }
             nodes++;
-            const BvhNode4 nd = bv.nodes4[r];
+            const BvhNode4 nd = bv.nodes4[cur];
             const float* f = reinterpret_cast<const float*>(nd.b);
-            int c[4] = {nd.r.x, nd.r.y, nd.r.z, nd.r.w};
-            float d[4];
-            int nv = 0;
+            const int c[4] = {nd.r.x, nd.r.y, nd.r.z, nd.r.w};
+            float d[4], best = INFINITY;
+            int next = NONE, bk = 0;
+            uint32_t rest = 0u;
 #pragma unroll
             for (int k = 0; k < 4; k++) {
                 d[k] = bf_child_d2(f, k, qx, qy, qz);
-                if (c[k] == EMPTY4 || !(d[k] <= bound)) {
-                    c[k] = EMPTY4;
-                    d[k] = -1.0f;  // sorts last
-                } else {
-                    nv++;
+                const bool in = c[k] != EMPTY4 && ((want >> k) & 1u) && d[k] <= bound;
+                if (!in) d[k] = INFINITY;
+                rest |= in ? 1u << k : 0u;
+                if (in && (next == NONE || d[k] < best)) {
+                    best = d[k];
+                    next = c[k];
+                    bk = k;
                 }
             }
-            // descending by distance: the valid children first, the nearest of them last
-            auto cswap = [&](int x, int y) {
-                if (d[x] < d[y]) {
-                    const float td = d[x];
-                    d[x] = d[y];
-                    d[y] = td;
-                    const int tc = c[x];
-                    c[x] = c[y];
-                    c[y] = tc;
-                }
-            };
-            cswap(0, 1);
-            cswap(2, 3);
-            cswap(0, 2);
-            cswap(1, 3);
-            cswap(1, 2);
-            // the nearest child is processed next without a trip through the stack; the others
-            // are pushed farthest first
+            if (next == NONE) {
+                cur = NONE;
+                continue;
+            }
+            rest &= ~(1u << bk);
+            if (rest != 0u) {
+                float dr = INFINITY;
 #pragma unroll
-            for (int k = 0; k < 4; k++) {
-                if (k + 1 < nv) {
-                    if (sp == stk.capacity()) return false;
-                    stk.put(sp, make_uint2((uint32_t)c[k], fbits(d[k])));
-                    sp++;
-                } else if (k + 1 == nv) {
-                    e = make_uint2((uint32_t)c[k], fbits(d[k]));
-                    have = true;
-                }
+                for (int k = 0; k < 4; k++) dr = k == bk ? dr : fminf(dr, d[k]);
+                if (!bf_put(pool, ln, lane, (uint32_t)cur | (rest << 28), fbits(dr) >> 16, bound)) return false;
+            }
+            cur = next;
+            want = 15u;
+            if (cur < 0) {
+                leaf = -1 - cur;
+                cur = NONE;
+                break;
             }
         }
-        if (leaf < 0) break;  // stack empty: the list is final
-        bf_scan_leaf<K, kDedup>(bv, leaf, qx, qy, qz, L);
+        if (leaf < 0) return true;  // nothing left within the bound: the list is final
+        bf_scan_leaf<K>(bv, leaf, qx, qy, qz, L);
         leaves++;
     }
-    return true;
 }
 
 // One lane per query i < m (queries in Morton order for locality): Out(i, list, t, ok, q)
 // consumes the result.  empty: the key an unfilled slot holds (BF_EMPTY, or (r^2, 0) to keep
 // only points with d^2 < r^2).
-// Outputs that start a query's search from a known neighbour set declare kPrefill = true and
-// prefill_list(i, L, t, x, y, z).
+// Outputs that know a neighbour set of the query beforehand declare kPrefill = true and
+// first_bound(i, t, x, y, z, empty): a key above the t-th, which the search starts from.
 template <class O, class = void>
 struct bf_prefills : std::false_type {
 };
@@ -334,8 +402,7 @@ __global__ __launch_bounds__(BF_THREADS) void bf_knn_kernel(const BvhView bv, co
                                                             unsigned long long* stats, uint32_t* queue, uint2* spill,
                                                             int spill_cap)
 {
-    __shared__ uint2 stk[BF_STACK][BF_THREADS];
-    uint2* const my_spill = spill + (size_t)blockIdx.x * spill_cap * BF_THREADS + threadIdx.x;
+    __shared__ BfPool pool;
     const int lane = threadIdx.x;
     const int64_t nchunks = (m + BF_THREADS - 1) / BF_THREADS;
     const int xcd = (int)(blockIdx.x % QUEUE_SEGS);
@@ -356,12 +423,13 @@ __global__ __launch_bounds__(BF_THREADS) void bf_knn_kernel(const BvhView bv, co
         bool ok = true;
         if (i < m) {  // no barrier in the search: lanes are independent
             const float x = qx[i * qs], y = qy[i * qs], z = qz[i * qs];
+            uint64_t start = empty;
+            if constexpr (bf_prefills<Out>::value) start = out.first_bound(i, t, x, y, z, empty);
             BfList<K> L;
-            L.init(t, empty);
-            if constexpr (bf_prefills<Out>::value) out.template prefill_list<K>(i, L, t, x, y, z);
-            ok = bf_search<K, bf_prefills<Out>::value>(
-                bv, BfLdsStack{(lds_uint2*)&stk[0][lane], my_spill, BF_STACK + spill_cap}, x, y, z, L, leaves,
-                nodes);
+            L.init(t, start);
+            BfLane ln{0u, 0, spill + (size_t)blockIdx.x * spill_cap * BF_THREADS + lane, spill_cap};
+            ok = bf_search<K>(bv, pool, ln, lane, x, y, z, L, leaves, nodes);
+            L.finish(bv.rank, t);
             out.template emit<K>(i, L, t, ok, x, y, z);
             ok = ok && L.full();
         }
@@ -556,6 +624,7 @@ __global__ __launch_bounds__(BF_THREADS) void bf_knn_wave_kernel(const BvhView b
         __syncthreads();
         if (lane == 0) {
             BfList<K> L;
+            L.empty = empty;
 #pragma unroll
             for (int q = 0; q < K; q++) {
                 const int o = q - (K - t);
@@ -725,7 +794,7 @@ struct BfCentroidOut {
     uint32_t* redo;
     // optional: the query's vertex (caller index -> vertex id) and, per vertex, the t neighbours
     // (sorted positions) of its last search, which a later search of the vertex starts from
-    // (prefill): their keys at the new position bound the search at once.  The result is the
+    // (first_bound): their keys at the new position bound the search at once.  The result is the
     // same exact neighbour set.
     const uint32_t* vid;
     uint32_t* nbr;
@@ -733,19 +802,24 @@ struct BfCentroidOut {
     uint32_t npts;  // sorted positions
     static constexpr bool kPrefill = true;
 
-    template <int K>
-    __device__ __forceinline__ void prefill_list(int64_t i, BfList<K>& L, int t, float qx, float qy, float qz) const
+    // the t neighbours of the vertex's last search are t points of the cloud: the t-th key is at most the
+    // largest of their keys at the new position
+    __device__ __forceinline__ uint64_t first_bound(int64_t i, int t, float qx, float qy, float qz,
+                                                    uint64_t empty) const
     {
-        if (!prefill || !vid || !nbr) return;
+        if (!prefill || !vid || !nbr) return empty;
         const size_t v = vid[qorig[i]];
+        uint64_t top = 0;
         for (int j = 0; j < t; j++) {
             const uint32_t s = nbr[v * t + j];
-            if (s >= npts) continue;
+            if (s >= npts) return empty;
             const float4 p = pts[s];
             const float d = d2_contract(qx, qy, qz, p.x, p.y, p.z);
+            if (!(d == d)) return empty;
             const uint64_t key = make_key(d, fbits(p.w));
-            if (d == d && key < L.worst() && !L.contains(key)) L.insert(key, s);
+            top = key > top ? key : top;
         }
+        return top < empty ? top + 1 : empty;
     }
 
     template <int K>
