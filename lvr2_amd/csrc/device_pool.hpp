@@ -1,0 +1,193 @@
+// Device memory of destroyed handles and finished host calls, kept for the next ones.
+//
+// hipMalloc and hipFree dominated short jobs: a surface of 500,000 points made and freed for one normals
+// pass spent 3.6 ms in its frees and 1 ms in its allocations beside 7 ms of kernels.  A freed block goes to
+// a list of its device and size class instead and serves the next allocation of that class.
+//  - Safe across streams and threads: a block enters the list only from a scope that has waited for the
+//    device's work on it (IdleScope); freed anywhere else it goes back to the runtime.  One mutex
+//    guards the lists.
+//  - Bounded: at most CACHE_BYTES per device, no block above a quarter of that.
+//  - Given back: blocks that no allocation took over the last KEEP handle destructions are freed, and all of a
+//    device's blocks when one of its allocations fails (which is then tried again).
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <cstdint>
+#include <map>
+#include <mutex>
+#include <unordered_map>
+#include <utility>
+#include <vector>
+
+namespace lvrhip {
+
+class DevicePool {
+public:
+    static constexpr size_t CACHE_BYTES = (size_t)2 << 30;
+    static constexpr uint64_t KEEP = 16;
+    static constexpr size_t PINNED_BYTES = 64;
+    static constexpr size_t PINNED_KEPT = 64;
+
+    static DevicePool& get()
+    {
+        static DevicePool* p = new DevicePool;  // never destroyed: handles may outlive static destructors
+        return *p;
+    }
+
+    // a block of at least `bytes` on the current device
+    hipError_t alloc(void** p, size_t bytes)
+    {
+        int dev = 0;
+        hipError_t e = hipGetDevice(&dev);
+        if (e != hipSuccess) return e;
+        const size_t size = size_class(bytes);
+        {
+            std::lock_guard<std::mutex> lk(mu_);
+            auto& c = cache_[dev];
+            auto it = c.blocks.find(size);
+            if (it != c.blocks.end() && !it->second.empty()) {
+                *p = it->second.back().first;
+                it->second.pop_back();
+                c.bytes -= size;
+                live_[*p] = {dev, size};
+                return hipSuccess;
+            }
+        }
+        size_t got = size;
+        e = hipMalloc(p, size);
+        if (e == hipErrorOutOfMemory) {
+            (void)hipGetLastError();
+            trim(dev, ~0ull);
+            got = bytes;
+            e = hipMalloc(p, bytes);
+        }
+        if (e != hipSuccess) return e;
+        std::lock_guard<std::mutex> lk(mu_);
+        live_[*p] = {dev, got};
+        return hipSuccess;
+    }
+
+    // idle: no work of any stream on the block is left
+    void free(void* p, bool idle)
+    {
+        bool keep = false;
+        {
+            std::lock_guard<std::mutex> lk(mu_);
+            auto it = live_.find(p);
+            if (it != live_.end()) {
+                const auto [dev, size] = it->second;
+                live_.erase(it);
+                auto& c = cache_[dev];
+                if (idle && size == size_class(size) && size <= CACHE_BYTES / 4 && c.bytes + size <= CACHE_BYTES) {
+                    c.blocks[size].emplace_back(p, now_);
+                    c.bytes += size;
+                    keep = true;
+                }
+            }
+        }
+        if (!keep) (void)hipFree(p);
+    }
+
+    // a handle was destroyed on the current device: what nobody took for KEEP of these is freed
+    void tick()
+    {
+        int dev = 0;
+        if (hipGetDevice(&dev) != hipSuccess) return;
+        uint64_t t;
+        {
+            std::lock_guard<std::mutex> lk(mu_);
+            t = ++now_;
+        }
+        if (t > KEEP) trim(dev, t - KEEP);
+    }
+
+    // pinned host words for readbacks
+    hipError_t alloc_pinned(uint32_t** p)
+    {
+        {
+            std::lock_guard<std::mutex> lk(mu_);
+            if (!pinned_.empty()) {
+                *p = pinned_.back();
+                pinned_.pop_back();
+                return hipSuccess;
+            }
+        }
+        return hipHostMalloc(reinterpret_cast<void**>(p), PINNED_BYTES, hipHostMallocPortable);
+    }
+    void free_pinned(uint32_t* p, bool idle)
+    {
+        if (idle) {
+            std::lock_guard<std::mutex> lk(mu_);
+            if (pinned_.size() < PINNED_KEPT) {
+                pinned_.push_back(p);
+                return;
+            }
+        }
+        (void)hipHostFree(p);
+    }
+
+private:
+    struct Cache {
+        std::map<size_t, std::vector<std::pair<void*, uint64_t>>> blocks;  // by size: (block, when freed)
+        size_t bytes = 0;
+    };
+    std::mutex mu_;
+    std::map<int, Cache> cache_;
+    std::unordered_map<void*, std::pair<int, size_t>> live_;
+    std::vector<uint32_t*> pinned_;
+    uint64_t now_ = 0;
+
+    // sizes in steps of an eighth of the power of two below (at most 12.5 % more than asked for)
+    static size_t size_class(size_t bytes)
+    {
+        if (bytes <= 4096) return 4096;
+        const size_t step = ((size_t)1 << (63 - __builtin_clzll(bytes))) / 8;
+        return (bytes + step - 1) / step * step;
+    }
+
+    // frees the device's kept blocks that were freed before `before`
+    void trim(int dev, uint64_t before)
+    {
+        std::vector<void*> out;
+        {
+            std::lock_guard<std::mutex> lk(mu_);
+            auto& c = cache_[dev];
+            for (auto& [size, v] : c.blocks) {
+                size_t w = 0;
+                for (auto& b : v) {
+                    if (b.second < before) {
+                        out.push_back(b.first);
+                        c.bytes -= size;
+                    } else {
+                        v[w++] = b;
+                    }
+                }
+                v.resize(w);
+            }
+        }
+        for (void* p : out) (void)hipFree(p);
+    }
+};
+
+// While one is set on a thread, the blocks that the thread frees are known to be idle: set it after waiting
+// for all work on them.
+struct IdleScope {
+    bool on = false;
+    static bool& flag()
+    {
+        static thread_local bool f = false;
+        return f;
+    }
+    void set()
+    {
+        on = true;
+        flag() = true;
+    }
+    ~IdleScope()
+    {
+        if (on) flag() = false;
+    }
+};
+
+}  // namespace lvrhip

@@ -2,6 +2,7 @@
 // include/lvrhip.h).  One handle = one point cloud resident on one device:
 // Morton-sorted SoA points, the LBVH, and the normals once computed.
 #include "common.hpp"
+#include "device_pool.hpp"
 #include "radix_sort.hpp"
 #include "lbvh.hpp"
 #include "knn_tile.hpp"
@@ -51,7 +52,7 @@ hipError_t dev_malloc(void** p, size_t bytes)
         if (made >= std::atoll(v)) return hipErrorOutOfMemory;
         made++;
     }
-    return hipMalloc(p, bytes);
+    return DevicePool::get().alloc(p, bytes);
 }
 
 template <typename T>
@@ -67,7 +68,7 @@ struct DBuf {
     }
     void release()
     {
-        if (p) (void)hipFree(p);
+        if (p) DevicePool::get().free(p, IdleScope::flag());
         p = nullptr;
         cap = 0;
     }
@@ -857,7 +858,7 @@ struct lvrhip_surface {
 
     ~lvrhip_surface()
     {
-        if (h_pin) (void)hipHostFree(h_pin);
+        if (h_pin) DevicePool::get().free_pinned(h_pin, IdleScope::flag());
         if (gexec) (void)hipGraphExecDestroy(gexec);
         if (graph) (void)hipGraphDestroy(graph);
         if (own_gst && gst) (void)hipStreamDestroy(gst);
@@ -999,7 +1000,7 @@ struct lvrhip_surface {
         d_cnt.reserve(CNT_SLOTS);
         fill_u32_kernel<<<1, 64, 0, st>>>(d_cnt.p, CNT_SLOTS, 0u);
         LVRHIP_LAUNCH_CHECK();
-        if (!h_pin) LVRHIP_CHECK(hipHostMalloc(reinterpret_cast<void**>(&h_pin), 64, hipHostMallocDefault));
+        if (!h_pin) LVRHIP_CHECK(DevicePool::get().alloc_pinned(&h_pin));
         if (n == 0) return;
         d_off.reserve(ns + 1);
         d_pstart.reserve(ns + 1);
@@ -1170,7 +1171,7 @@ struct lvrhip_surface {
         mom.reserve((size_t)npad * 9);
         if (kiw > 0) ki_list.reserve((size_t)npad * kiw);
         s_flags.reserve(n);
-        s_list0.reserve(std::max<int64_t>(n, 4 * (int64_t)SPEC_POINTS));
+        s_list0.reserve(n);
         s_list1.reserve(n);
         a_sel.reserve(n);
         a_list.reserve(n);
@@ -1179,15 +1180,17 @@ struct lvrhip_surface {
         pst.reserve(npad);
         act.reserve(npad);
         s_seg.reserve(ROUND_SEGS + 2);
-        spec_mom.reserve(4 * 9 * (size_t)SPEC_POINTS);
-        spec_ok.reserve(4 * (size_t)SPEC_POINTS);
+        spec_mom.reserve(4 * 9 * (size_t)spec_points());
+        spec_ok.reserve(4 * (size_t)spec_points());
         s_bsum.reserve(ROUND_SEGS * std::max<int64_t>(ceil_div(n, CF_TILE), 1) + 1);
     }
 
     // A rejected list up to this length is searched for rounds 2..5 at once: 4 x 16,384 searches are
     // about three times what the device holds, as long as the launches one after the other (four of
     // 130-290 us for the 4,000 rejected points of the 30,000-point plain scene).
+    // A quarter of the cloud at most, so that its buffers are no larger than the others.
     static constexpr uint32_t SPEC_POINTS = 16384;
+    uint32_t spec_points() const { return (uint32_t)std::min<int64_t>(SPEC_POINTS, n / 4); }
     DBuf<float> spec_mom;   // per entry of that launch: its moments,
     DBuf<uint8_t> spec_ok;  // and whether its box passes
 
@@ -1268,7 +1271,7 @@ struct lvrhip_surface {
             partition_stages(rejected, nq0, pass == 0);
             enqueue_round(2, s_list0.p, nq0, s_seg.p);
             if (pass == 0) {
-                spec_resolve_kernel<<<SPEC_POINTS / 256, 256, 0, st>>>(s_seg.p, s_list0.p, spec_mom.p, spec_ok.p,
+                spec_resolve_kernel<<<(unsigned)ceil_div(std::max(spec_points(), 1u), 256), 256, 0, st>>>(s_seg.p, s_list0.p, spec_mom.p, spec_ok.p,
                                                                       mom.p, kround.p, act.p);
                 LVRHIP_LAUNCH_CHECK();
             }
@@ -1283,10 +1286,10 @@ struct lvrhip_surface {
     }
 
     // s_list0 = the points of list[0, *counter(2)) by their next stage, s_seg = the segments (the first
-    // time, a list of at most SPEC_POINTS points: every round of every point)
+    // time, a list of at most spec_points(): every round of every point)
     void partition_stages(const uint32_t* list, int64_t nq0, bool first)
     {
-        const uint32_t spec = first ? SPEC_POINTS : 0u;
+        const uint32_t spec = first ? spec_points() : 0u;
         const int64_t nb = std::max<int64_t>(ceil_div(nq0, CF_TILE), 1);
         part_sums_kernel<<<(unsigned)nb, CF_THREADS, 0, st>>>(act.p, list, counter(2), spec, first ? nq0 : 0, s_bsum.p);
         LVRHIP_LAUNCH_CHECK();
@@ -2486,8 +2489,10 @@ int lvrhip_destroy(lvrhip_t h)
     return guarded([&] {
         if (!h) return;
         DeviceGuard dg(h->device);
-        (void)hipStreamSynchronize(h->st);
+        IdleScope idle;  // the handle may have worked on several streams
+        if (hipDeviceSynchronize() == hipSuccess) idle.set();
         delete h;
+        DevicePool::get().tick();
     });
 }
 
@@ -2568,6 +2573,7 @@ int lvrhip_set_normals(lvrhip_t h, const float* normals)
             h->nx.reserve(R);
             h->ny.reserve(R);
             h->nz.reserve(R);
+            IdleScope idle;
             DBuf<float> d;
             d.reserve(3 * (size_t)N);
             LVRHIP_CHECK(hipMemcpyAsync(d.p, normals, 3 * (size_t)N * sizeof(float), hipMemcpyHostToDevice, h->st));
@@ -2575,6 +2581,7 @@ int lvrhip_set_normals(lvrhip_t h, const float* normals)
                                                                                h->nz.p);
             LVRHIP_LAUNCH_CHECK();
             LVRHIP_CHECK(hipStreamSynchronize(h->st));
+            idle.set();
         }
         h->has_normals = true;
     });
@@ -2600,12 +2607,14 @@ int lvrhip_get_normals(lvrhip_t h, float* out)
         if (h->n == 0) return;
         REQUIRE(out, "output pointer is NULL");
         DeviceGuard dg(h->device);
+        IdleScope idle;
         DBuf<float> d;
         d.reserve(3 * (size_t)h->n);
         int rc = lvrhip_get_normals_device(h, d.p);
         if (rc != LVRHIP_OK) throw Error(rc, g_last_error);
         LVRHIP_CHECK(hipMemcpyAsync(out, d.p, 3 * (size_t)h->n * sizeof(float), hipMemcpyDeviceToHost, h->st));
         LVRHIP_CHECK(hipStreamSynchronize(h->st));
+        idle.set();
     });
 }
 
@@ -2618,6 +2627,7 @@ int lvrhip_knn(lvrhip_t h, const float* q, size_t m, int k, int32_t* out_idx, fl
         REQUIRE(m < (size_t)0x7FFFFFFF, "too many queries");
         if (m == 0) return;
         DeviceGuard dg(h->device);
+        IdleScope idle;
         DBuf<float> dq;
         DBuf<int32_t> di;
         DBuf<float> dd;
@@ -2630,6 +2640,7 @@ int lvrhip_knn(lvrhip_t h, const float* q, size_t m, int k, int32_t* out_idx, fl
         if (out_d2)
             LVRHIP_CHECK(hipMemcpyAsync(out_d2, dd.p, m * (size_t)k * sizeof(float), hipMemcpyDeviceToHost, h->st));
         LVRHIP_CHECK(hipStreamSynchronize(h->st));
+        idle.set();
     });
 }
 
@@ -2644,6 +2655,7 @@ int lvrhip_radius_search(lvrhip_t h, const float* q, size_t m, int k, float r, i
         REQUIRE(m < (size_t)0x7FFFFFFF, "too many queries");
         if (m == 0) return;
         DeviceGuard dg(h->device);
+        IdleScope idle;
         DBuf<float> dq, dd;
         DBuf<int32_t> di, dc;
         dq.reserve(3 * m);
@@ -2658,6 +2670,7 @@ int lvrhip_radius_search(lvrhip_t h, const float* q, size_t m, int k, float r, i
         if (out_count)
             LVRHIP_CHECK(hipMemcpyAsync(out_count, dc.p, m * sizeof(int32_t), hipMemcpyDeviceToHost, h->st));
         LVRHIP_CHECK(hipStreamSynchronize(h->st));
+        idle.set();
     });
 }
 
@@ -2672,6 +2685,7 @@ int lvrhip_interpolated_normals(lvrhip_t h, const float* q, size_t m, float* out
             h->interpolated_normals_device(nullptr, 0, nullptr);
             return;
         }
+        IdleScope idle;
         DBuf<float> dq, dn;
         dq.reserve(3 * m);
         dn.reserve(3 * m);
@@ -2679,6 +2693,7 @@ int lvrhip_interpolated_normals(lvrhip_t h, const float* q, size_t m, float* out
         h->interpolated_normals_device(dq.p, (int64_t)m, dn.p);
         LVRHIP_CHECK(hipMemcpyAsync(out_xyz, dn.p, 3 * m * sizeof(float), hipMemcpyDeviceToHost, h->st));
         LVRHIP_CHECK(hipStreamSynchronize(h->st));
+        idle.set();
     });
 }
 
@@ -2725,6 +2740,7 @@ int lvrhip_distances(lvrhip_t h, const float* q, size_t m, float voxel, float* o
         REQUIRE(m == 0 || q, "NULL query pointer");
         if (m == 0) return;
         DeviceGuard dg(h->device);
+        IdleScope idle;
         DBuf<float> dq, dp, de;
         DBuf<uint8_t> di;
         dq.reserve(3 * m);
@@ -2738,6 +2754,7 @@ int lvrhip_distances(lvrhip_t h, const float* q, size_t m, float voxel, float* o
         if (out_invalid)
             LVRHIP_CHECK(hipMemcpyAsync(out_invalid, di.p, m * sizeof(uint8_t), hipMemcpyDeviceToHost, h->st));
         LVRHIP_CHECK(hipStreamSynchronize(h->st));
+        idle.set();
     });
 }
 
@@ -2770,6 +2787,7 @@ int lvrhip_get_adaptive_k(lvrhip_t h, int32_t* out_k)
         if (h->n == 0) return;
         REQUIRE(out_k, "output pointer is NULL");
         DeviceGuard dg(h->device);
+        IdleScope idle;
         DBuf<int32_t> d;
         d.reserve((size_t)h->n);
         adaptive_k_kernel<<<(unsigned)ceil_div(h->npad, 256), 256, 0, h->st>>>(
@@ -2777,6 +2795,7 @@ int lvrhip_get_adaptive_k(lvrhip_t h, int32_t* out_k)
         LVRHIP_LAUNCH_CHECK();
         LVRHIP_CHECK(hipMemcpyAsync(out_k, d.p, (size_t)h->n * sizeof(int32_t), hipMemcpyDeviceToHost, h->st));
         LVRHIP_CHECK(hipStreamSynchronize(h->st));
+        idle.set();
     });
 }
 

@@ -1,7 +1,7 @@
 """The adaptive rounds out of order: the neighbourhood size every point stops at, and how many points
 reach each round, bit-exact against the oracle's round-by-round loop, on both sides of the lines where the
-order of the searches changes (all rounds at once up to 16,384 rejected points; round 5 first only where
-at most 45 % of the points are rejected), single- and multi-scan, and against the merged rounds."""
+order of the searches changes (all rounds at once up to 16,384 rejected points and a quarter of the cloud;
+round 5 first only where at most 45 % of the points are rejected), single- and multi-scan, and against the merged rounds."""
 import numpy as np
 import pytest
 
