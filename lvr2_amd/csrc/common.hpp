@@ -183,4 +183,10 @@ __device__ __forceinline__ uint64_t make_key(float d2, uint32_t idx)
     return ((uint64_t)fbits(d2) << 32) | (uint64_t)idx;
 }
 
+static __global__ void fill_u32_kernel(uint32_t* p, int64_t n, uint32_t v)
+{
+    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) p[i] = v;
+}
+
 }  // namespace lvrhip

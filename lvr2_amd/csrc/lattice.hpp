@@ -20,6 +20,9 @@
 // that first cell, as the reference computes it).
 #pragma once
 
+#include <algorithm>
+#include <cmath>
+
 #include "common.hpp"
 #include "lbvh.hpp"
 
@@ -38,22 +41,48 @@ __device__ __forceinline__ int lat_bct(int v, int axis)
     return axis == 0 ? x : axis == 1 ? y : z;
 }
 
-__device__ __forceinline__ uint64_t lat_pack(int x, int y, int z)
-{
-    return ((uint64_t)(uint32_t)(x + LAT_BIAS) << 42) | ((uint64_t)(uint32_t)(y + LAT_BIAS) << 21) |
-           (uint64_t)(uint32_t)(z + LAT_BIAS);
-}
-__device__ __forceinline__ void lat_unpack(uint64_t k, int& x, int& y, int& z)
-{
-    x = (int)(k >> 42) - LAT_BIAS;
-    y = (int)((k >> 21) & ((1ull << 21) - 1)) - LAT_BIAS;
-    z = (int)(k & ((1ull << 21) - 1)) - LAT_BIAS;
-}
-
 struct LatBox {
     float lo[3], hi[3];
     float voxel;
+    // cell and corner keys: the index relative to base, x over y over z in by + bz and bz bits (lat_key_bits),
+    // so that a sort's passes cover the cells the box can hold and not 21 bits per axis
+    int base[3];
+    int by, bz;
 };
+
+__device__ __forceinline__ uint64_t lat_pack(const LatBox& b, int x, int y, int z)
+{
+    return ((uint64_t)(uint32_t)(x - b.base[0]) << (b.by + b.bz)) | ((uint64_t)(uint32_t)(y - b.base[1]) << b.bz) |
+           (uint64_t)(uint32_t)(z - b.base[2]);
+}
+__device__ __forceinline__ void lat_unpack(const LatBox& b, uint64_t k, int& x, int& y, int& z)
+{
+    x = (int)(k >> (b.by + b.bz)) + b.base[0];
+    y = (int)((k >> b.bz) & ((1ull << b.by) - 1)) + b.base[1];
+    z = (int)(k & ((1ull << b.bz) - 1)) + b.base[2];
+}
+inline int lat_bits(int64_t n)  // bits that hold 0 .. n - 1
+{
+    int b = 1;
+    while (((int64_t)1 << b) < n) b++;
+    return b;
+}
+// Sets the key layout of the box (its cells' and their corners' indices, two to spare on each side for
+// the fp32 division of the points' cells) and returns the bits a sort must cover: one more than
+// the keys have (at most 63), which only the sentinel sets.
+inline int lat_key_bits(LatBox& b)
+{
+    int bits[3];
+    for (int j = 0; j < 3; j++) {
+        const int64_t lo = std::max<int64_t>((int64_t)std::floor((double)b.lo[j] / b.voxel) - 2, -LAT_BIAS);
+        const int64_t hi = std::min<int64_t>((int64_t)std::floor((double)b.hi[j] / b.voxel) + 3, LAT_BIAS - 1);
+        b.base[j] = (int)lo;
+        bits[j] = lat_bits(hi - lo + 1);
+    }
+    b.by = bits[1];
+    b.bz = bits[2];
+    return bits[0] + bits[1] + bits[2] + 1;
+}
 
 // BoundingBox::contains (BoundingBox.tcc:166-171) of the cell centre
 __device__ __forceinline__ bool lat_contains(const LatBox& b, int x, int y, int z)
@@ -73,7 +102,7 @@ __global__ __launch_bounds__(256) void lat_point_cells_kernel(const float* __res
     uint64_t k = LAT_SENTINEL;
     if (pidx[i] != ~0u) {
         const int x = (int)floorf(px[i] / b.voxel), y = (int)floorf(py[i] / b.voxel), z = (int)floorf(pz[i] / b.voxel);
-        if (lat_contains(b, x, y, z)) k = lat_pack(x, y, z);
+        if (lat_contains(b, x, y, z)) k = lat_pack(b, x, y, z);
     }
     keys[i] = k;
     vals[i] = (uint32_t)i;
@@ -104,24 +133,24 @@ __global__ __launch_bounds__(256) void lat_extrude_kernel(const uint64_t* __rest
     const int64_t c = i / 27;
     const int d = (int)(i % 27);
     int x, y, z;
-    lat_unpack(cells[c], x, y, z);
+    lat_unpack(b, cells[c], x, y, z);
     x += d / 9 - 1;
     y += (d / 3) % 3 - 1;
     z += d % 3 - 1;
-    keys[i] = lat_contains(b, x, y, z) ? lat_pack(x, y, z) : LAT_SENTINEL;
+    keys[i] = lat_contains(b, x, y, z) ? lat_pack(b, x, y, z) : LAT_SENTINEL;
     vals[i] = (uint32_t)i;
 }
 
 // corner key of (cell rank r, slot v), value = its order r * 8 + v
-__global__ __launch_bounds__(256) void lat_corners_kernel(const uint64_t* __restrict__ cells, int64_t nc,
+__global__ __launch_bounds__(256) void lat_corners_kernel(const uint64_t* __restrict__ cells, int64_t nc, LatBox b,
                                                           uint64_t* __restrict__ keys, uint32_t* __restrict__ vals)
 {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= nc * 8) return;
     const int v = (int)(i % 8);
     int x, y, z;
-    lat_unpack(cells[i / 8], x, y, z);
-    keys[i] = lat_pack(x + (lat_bct(v, 0) + 1) / 2, y + (lat_bct(v, 1) + 1) / 2, z + (lat_bct(v, 2) + 1) / 2);
+    lat_unpack(b, cells[i / 8], x, y, z);
+    keys[i] = lat_pack(b, x + (lat_bct(v, 0) + 1) / 2, y + (lat_bct(v, 1) + 1) / 2, z + (lat_bct(v, 2) + 1) / 2);
     vals[i] = (uint32_t)i;
 }
 
@@ -185,26 +214,27 @@ __global__ void lat_cells_kernel(const uint32_t* __restrict__ gid, const uint32_
 
 // vertex j at centre(first cell) + box_creation_table[slot] * voxel / 2 (HashGrid.tcc:333-345)
 __global__ void lat_vertices_kernel(const uint64_t* __restrict__ sorted_first, const uint64_t* __restrict__ cells,
-                                    int64_t nv, float voxel, float* __restrict__ vtx)
+                                    int64_t nv, LatBox b, float* __restrict__ vtx)
 {
     const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (j >= nv) return;
     const uint64_t o = sorted_first[j];
     const int v = (int)(o % 8);
     int x, y, z;
-    lat_unpack(cells[o / 8], x, y, z);
-    const float half = voxel / 2.0f;
+    lat_unpack(b, cells[o / 8], x, y, z);
+    const float voxel = b.voxel, half = voxel / 2.0f;
     vtx[3 * j] = ((float)x + 0.5f) * voxel + (float)lat_bct(v, 0) * half;
     vtx[3 * j + 1] = ((float)y + 0.5f) * voxel + (float)lat_bct(v, 1) * half;
     vtx[3 * j + 2] = ((float)z + 0.5f) * voxel + (float)lat_bct(v, 2) * half;
 }
 
-__global__ void lat_cell_index_kernel(const uint64_t* __restrict__ cells, int64_t nc, int32_t* __restrict__ out)
+__global__ void lat_cell_index_kernel(const uint64_t* __restrict__ cells, int64_t nc, LatBox b,
+                                      int32_t* __restrict__ out)
 {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= nc) return;
     int x, y, z;
-    lat_unpack(cells[i], x, y, z);
+    lat_unpack(b, cells[i], x, y, z);
     out[3 * i] = x;
     out[3 * i + 1] = y;
     out[3 * i + 2] = z;

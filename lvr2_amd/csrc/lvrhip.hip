@@ -1063,9 +1063,12 @@ struct lvrhip_surface {
         LVRHIP_LAUNCH_CHECK();
         // sort by (scan, Morton code)
         const unsigned gb = (unsigned)ceil_div(N, 256);
-        morton_scan_kernel<<<gb, 256, 0, st>>>(src, N, d_off.p, ns, frames.p, s_k0.p, s_v0.p);
+        const int key_bits = ns > 1 ? 48 + lat_bits(ns) : 64;
+        const bool odd = rs_passes(key_bits) & 1;  // the sort then starts from its other buffers
+        morton_scan_kernel<<<gb, 256, 0, st>>>(src, N, d_off.p, ns, frames.p, odd ? s_k1.p : s_k0.p,
+                                               odd ? s_v1.p : s_v0.p);
         LVRHIP_LAUNCH_CHECK();
-        radix_sort_pairs(s_k0.p, s_v0.p, s_k1.p, s_v1.p, N, s_hist.p, st);
+        radix_sort_pairs(s_k0.p, s_v0.p, s_k1.p, s_v1.p, N, s_hist.p, st, key_bits);
         const unsigned gp = (unsigned)ceil_div(npad, 256);
         gather_padded_kernel<<<gp, 256, 0, st>>>(src, d_off.p, d_pstart.p, ns, npad, s_v0.p, s_k0.p, px.p, py.p, pz.p,
                                                  pidx.p, rank.p, s_k1.p, qreal.p, ns > 1 ? scan_of.p : nullptr,
@@ -1829,7 +1832,10 @@ struct lvrhip_surface {
     DBuf<int32_t> grid_cells, grid_cidx;
     int64_t grid_nv = 0, grid_nc = 0;
 
-    void lat_sort(uint64_t* k, uint32_t* v, int64_t m, int end_bit = 64)
+    // sorts by key bits [0, end_bit) into (k, v); the input is in in_keys(k, end_bit) and in_vals(v, end_bit)
+    uint64_t* in_keys(uint64_t* k, int end_bit) { return rs_passes(end_bit) & 1 ? g_k1.p : k; }
+    uint32_t* in_vals(uint32_t* v, int end_bit) { return rs_passes(end_bit) & 1 ? g_v1.p : v; }
+    void lat_sort(uint64_t* k, uint32_t* v, int64_t m, int end_bit)
     {
         g_hist.reserve(rs_hist_size(m));
         radix_sort_pairs(k, v, g_k1.p, g_v1.p, m, g_hist.p, st, end_bit);
@@ -1886,16 +1892,17 @@ struct lvrhip_surface {
             if (!(a > -(double)(LAT_BIAS - 2) && c < (double)(LAT_BIAS - 2)))
                 throw Error(LVRHIP_EINVAL, "lattice index out of range: voxel too small for the cloud's extent");
         }
+        const int kb = lat_key_bits(b);
         const int64_t R = npad;
         int64_t m = R;
         g_k0.reserve(m);
         g_k1.reserve(m);
         g_v0.reserve(m);
         g_v1.reserve(m);
-        lat_point_cells_kernel<<<(unsigned)ceil_div(m, 256), 256, 0, st>>>(px.p, py.p, pz.p, pidx.p, R, b, g_k0.p,
-                                                                          g_v0.p);
+        lat_point_cells_kernel<<<(unsigned)ceil_div(m, 256), 256, 0, st>>>(px.p, py.p, pz.p, pidx.p, R, b,
+                                                                          in_keys(g_k0.p, kb), in_vals(g_v0.p, kb));
         LVRHIP_LAUNCH_CHECK();
-        lat_sort(g_k0.p, g_v0.p, m);
+        lat_sort(g_k0.p, g_v0.p, m, kb);
         g_cells.reserve(m);
         int64_t nc = lat_unique(g_k0.p, m, g_cells.p);
         if (extrude && nc > 0) {
@@ -1904,9 +1911,10 @@ struct lvrhip_surface {
             g_k1.reserve(m);
             g_v0.reserve(m);
             g_v1.reserve(m);
-            lat_extrude_kernel<<<(unsigned)ceil_div(m, 256), 256, 0, st>>>(g_cells.p, nc, b, g_k0.p, g_v0.p);
+            lat_extrude_kernel<<<(unsigned)ceil_div(m, 256), 256, 0, st>>>(g_cells.p, nc, b, in_keys(g_k0.p, kb),
+                                                                          in_vals(g_v0.p, kb));
             LVRHIP_LAUNCH_CHECK();
-            lat_sort(g_k0.p, g_v0.p, m);
+            lat_sort(g_k0.p, g_v0.p, m, kb);
             g_cells2.reserve(m);
             nc = lat_unique(g_k0.p, m, g_cells2.p);
             std::swap(g_cells.p, g_cells2.p);
@@ -1920,9 +1928,10 @@ struct lvrhip_surface {
         g_k1.reserve(m);
         g_v0.reserve(m);
         g_v1.reserve(m);
-        lat_corners_kernel<<<(unsigned)ceil_div(m, 256), 256, 0, st>>>(g_cells.p, nc, g_k0.p, g_v0.p);
+        lat_corners_kernel<<<(unsigned)ceil_div(m, 256), 256, 0, st>>>(g_cells.p, nc, b, in_keys(g_k0.p, kb),
+                                                                      in_vals(g_v0.p, kb));
         LVRHIP_LAUNCH_CHECK();
-        lat_sort(g_k0.p, g_v0.p, m);
+        lat_sort(g_k0.p, g_v0.p, m, kb);
         g_flags.reserve(m);
         lat_first_flags_kernel<<<(unsigned)ceil_div(m, 256), 256, 0, st>>>(g_k0.p, m, g_flags.p);
         LVRHIP_LAUNCH_CHECK();
@@ -1942,10 +1951,12 @@ struct lvrhip_surface {
         // vertex ids in first-use order
         g_first.reserve(nv);
         g_vidx.reserve(nv);
-        lat_first_order_kernel<<<(unsigned)ceil_div(m, 256), 256, 0, st>>>(g_flags.p, g_gid.p, g_v0.p, m, g_first.p,
-                                                                          g_vidx.p);
+        const int ob = lat_bits(m);  // first uses are orders below m
+        lat_first_order_kernel<<<(unsigned)ceil_div(m, 256), 256, 0, st>>>(g_flags.p, g_gid.p, g_v0.p, m,
+                                                                          in_keys(g_first.p, ob),
+                                                                          in_vals(g_vidx.p, ob));
         LVRHIP_LAUNCH_CHECK();
-        lat_sort(g_first.p, g_vidx.p, nv, 32);
+        lat_sort(g_first.p, g_vidx.p, nv, ob);
         g_vid.reserve(nv);
         lat_vertex_ids_kernel<<<(unsigned)ceil_div(nv, 256), 256, 0, st>>>(g_vidx.p, nv, g_vid.p);
         LVRHIP_LAUNCH_CHECK();
@@ -1953,10 +1964,10 @@ struct lvrhip_surface {
         lat_cells_kernel<<<(unsigned)ceil_div(m, 256), 256, 0, st>>>(g_gid.p, g_v0.p, g_vid.p, m, grid_cells.p);
         LVRHIP_LAUNCH_CHECK();
         grid_vtx.reserve(3 * nv);
-        lat_vertices_kernel<<<(unsigned)ceil_div(nv, 256), 256, 0, st>>>(g_first.p, g_cells.p, nv, voxel, grid_vtx.p);
+        lat_vertices_kernel<<<(unsigned)ceil_div(nv, 256), 256, 0, st>>>(g_first.p, g_cells.p, nv, b, grid_vtx.p);
         LVRHIP_LAUNCH_CHECK();
         grid_cidx.reserve(3 * nc);
-        lat_cell_index_kernel<<<(unsigned)ceil_div(nc, 256), 256, 0, st>>>(g_cells.p, nc, grid_cidx.p);
+        lat_cell_index_kernel<<<(unsigned)ceil_div(nc, 256), 256, 0, st>>>(g_cells.p, nc, b, grid_cidx.p);
         LVRHIP_LAUNCH_CHECK();
         LVRHIP_CHECK(hipStreamSynchronize(st));
         grid_nv = nv;
@@ -2012,10 +2023,11 @@ struct lvrhip_surface {
         mc_fcell.reserve(nf);
         g_k1.reserve(m);
         g_v1.reserve(m);
-        mc_emit_kernel<<<gc, 256, 0, st>>>(grid_cells.p, nc, mc_case.p, mc_keep.p, mc_off.p, mc_keys.p, mc_vals.p,
-                                           mc_fcell.p);
+        const int eb = lat_bits(3 * grid_nv);  // lattice edges
+        mc_emit_kernel<<<gc, 256, 0, st>>>(grid_cells.p, nc, mc_case.p, mc_keep.p, mc_off.p, in_keys(mc_keys.p, eb),
+                                           in_vals(mc_vals.p, eb), mc_fcell.p);
         LVRHIP_LAUNCH_CHECK();
-        lat_sort(mc_keys.p, mc_vals.p, m, 32);  // by lattice edge, stable in corner order
+        lat_sort(mc_keys.p, mc_vals.p, m, eb);  // by lattice edge, stable in corner order
         // one vertex per lattice edge: the group of its first use
         g_flags.reserve(m);
         lat_first_flags_kernel<<<(unsigned)ceil_div(m, 256), 256, 0, st>>>(mc_keys.p, m, g_flags.p);
@@ -2033,10 +2045,12 @@ struct lvrhip_surface {
         // vertex ids in first-use order
         g_first.reserve(nv);
         g_vidx.reserve(nv);
-        lat_first_order_kernel<<<(unsigned)ceil_div(m, 256), 256, 0, st>>>(g_flags.p, g_gid.p, mc_vals.p, m, g_first.p,
-                                                                          g_vidx.p);
+        const int ob = lat_bits(m);
+        lat_first_order_kernel<<<(unsigned)ceil_div(m, 256), 256, 0, st>>>(g_flags.p, g_gid.p, mc_vals.p, m,
+                                                                          in_keys(g_first.p, ob),
+                                                                          in_vals(g_vidx.p, ob));
         LVRHIP_LAUNCH_CHECK();
-        lat_sort(g_first.p, g_vidx.p, nv, 32);
+        lat_sort(g_first.p, g_vidx.p, nv, ob);
         g_vid.reserve(nv);
         lat_vertex_ids_kernel<<<(unsigned)ceil_div(nv, 256), 256, 0, st>>>(g_vidx.p, nv, g_vid.p);
         LVRHIP_LAUNCH_CHECK();
@@ -2064,9 +2078,11 @@ struct lvrhip_surface {
         mc_vals.reserve(m);
         g_k1.reserve(m);
         g_v1.reserve(m);
-        mc_face_edges_kernel<<<(unsigned)ceil_div(m, 256), 256, 0, st>>>(mesh_faces.p, nf, mc_keys.p, mc_vals.p);
+        const int vb = lat_bits(nv);
+        mc_face_edges_kernel<<<(unsigned)ceil_div(m, 256), 256, 0, st>>>(mesh_faces.p, nf, vb, in_keys(mc_keys.p, 2 * vb),
+                                                                        in_vals(mc_vals.p, 2 * vb));
         LVRHIP_LAUNCH_CHECK();
-        lat_sort(mc_keys.p, mc_vals.p, m);
+        lat_sort(mc_keys.p, mc_vals.p, m, 2 * vb);
         mc_border.reserve(m);
         mc_border_kernel<<<(unsigned)ceil_div(m, 256), 256, 0, st>>>(mc_keys.p, mc_vals.p, m, mc_border.p);
         LVRHIP_LAUNCH_CHECK();
@@ -2082,7 +2098,7 @@ struct lvrhip_surface {
             LVRHIP_CHECK(hipMemsetAsync(counter(12), 0, sizeof(uint32_t), st));
             mc_list.reserve(nv);
             mc_q.reserve(3 * nv);
-            mc_round_list_kernel<<<(unsigned)ceil_div(nv, 256), 256, 0, st>>>(mc_moves.p, nv, r, mesh_vtx.p,
+            mc_round_list_kernel<<<(unsigned)ceil_div(nv, MC_LIST_THREADS), MC_LIST_THREADS, 0, st>>>(mc_moves.p, nv, r, mesh_vtx.p,
                                                                              mc_list.p, mc_q.p, counter(12));
             LVRHIP_LAUNCH_CHECK();
             const int64_t mr = read_counter(12);

@@ -160,9 +160,9 @@ __global__ void mc_vertices_kernel(const uint64_t* __restrict__ first, int64_t n
 
 // ---- planar marching cubes: the border-edge moves (BilinearFastBox::optimizePlanarFaces) -----
 
-// the undirected edges of every face: key (low vertex id, high vertex id), value face * 3 + slot,
+// the undirected edges of every face: key (low vertex id, high vertex id) of vbits each, value face * 3 + slot,
 // slot b joining corners b and (b + 1) % 3
-__global__ void mc_face_edges_kernel(const int32_t* __restrict__ faces, int64_t nf, uint64_t* __restrict__ keys,
+__global__ void mc_face_edges_kernel(const int32_t* __restrict__ faces, int64_t nf, int vbits, uint64_t* __restrict__ keys,
                                      uint32_t* __restrict__ vals)
 {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -170,7 +170,7 @@ __global__ void mc_face_edges_kernel(const int32_t* __restrict__ faces, int64_t 
     const int64_t f = i / 3;
     const int b = (int)(i % 3);
     const uint32_t u = (uint32_t)faces[3 * f + b], v = (uint32_t)faces[3 * f + (b + 1) % 3];
-    keys[i] = u < v ? ((uint64_t)u << 32) | v : ((uint64_t)v << 32) | u;
+    keys[i] = u < v ? ((uint64_t)u << vbits) | v : ((uint64_t)v << vbits) | u;
     vals[i] = (uint32_t)i;
 }
 
@@ -187,7 +187,8 @@ __global__ void mc_border_kernel(const uint64_t* __restrict__ keys, const uint32
 }
 
 // cells whose own faces have one or two border edges: one move for each end point of each; the
-// largest count reached goes to *max_moves (one atomic per wave)
+// largest count reached goes to *max_moves (one atomic per block at most: one per wave, all on one address,
+// had taken 95 us)
 __global__ void mc_moves_kernel(const uint32_t* __restrict__ off, const uint32_t* __restrict__ ntri, int64_t nc,
                                 const uint8_t* __restrict__ border, const int32_t* __restrict__ faces,
                                 uint32_t* __restrict__ moves, uint32_t* __restrict__ max_moves)
@@ -209,20 +210,44 @@ __global__ void mc_moves_kernel(const uint32_t* __restrict__ off, const uint32_t
             }
         }
     }
+    __shared__ uint32_t top;
+    if (threadIdx.x == 0) top = 0u;
+    __syncthreads();
 #pragma unroll
     for (int m = 32; m >= 1; m >>= 1) most = max(most, (uint32_t)shfl_xor((int)most, m));
-    if (lane_id() == 0 && most > 0) atomicMax(max_moves, most);
+    if (lane_id() == 0 && most > 0) atomicMax(&top, most);
+    __syncthreads();
+    // (one address for all blocks: a block whose maximum is already there leaves it alone)
+    if (threadIdx.x == 0 && top > 0 && __hip_atomic_load(max_moves, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < top)
+        atomicMax(max_moves, top);
 }
 
 // round r: the vertices that move at least r times, with their current positions (any order:
 // every move reads its own vertex only)
-__global__ void mc_round_list_kernel(const uint32_t* __restrict__ moves, int64_t nv, uint32_t r,
-                                     const float* __restrict__ vtx, uint32_t* __restrict__ list,
-                                     float* __restrict__ q, uint32_t* __restrict__ count)
+// A block appends its vertices in one piece (one atomic per block; a wave each had taken 70 us).
+constexpr int MC_LIST_THREADS = 1024;
+__global__ __launch_bounds__(MC_LIST_THREADS) void mc_round_list_kernel(const uint32_t* __restrict__ moves, int64_t nv,
+                                                                        uint32_t r, const float* __restrict__ vtx,
+                                                                        uint32_t* __restrict__ list,
+                                                                        float* __restrict__ q,
+                                                                        uint32_t* __restrict__ count)
 {
+    __shared__ uint32_t ws[MC_LIST_THREADS / kWave], base;
     const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= nv || moves[j] < r) return;
-    const uint32_t o = atomicAdd(count, 1u);
+    const bool in = j < nv && moves[j] >= r;
+    const uint64_t m = ballot(in);
+    const int wave = threadIdx.x / kWave;
+    if (lane_id() == 0) ws[wave] = (uint32_t)__popcll(m);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        uint32_t t = 0;
+        for (int w = 0; w < MC_LIST_THREADS / kWave; w++) t += ws[w];
+        base = t ? atomicAdd(count, t) : 0u;
+    }
+    __syncthreads();
+    if (!in) return;
+    uint32_t o = base + (uint32_t)mbcnt(m);
+    for (int w = 0; w < wave; w++) o += ws[w];
     list[o] = (uint32_t)j;
     q[3 * (size_t)o] = vtx[3 * j];
     q[3 * (size_t)o + 1] = vtx[3 * j + 1];
