@@ -24,6 +24,38 @@
 
 namespace lvrhip {
 
+// dL/dp and dL/dn of each of a vertex's cnt neighbours (the same for all) from the forward's ordered sums of
+// their positions (a) and normals (b); false if there is no gradient.
+struct SdfGrad {
+    float px, py, pz, nx, ny, nz;
+};
+__device__ __forceinline__ bool sdf_grad(float ax, float ay, float az, float bx, float by, float bz, int cnt, float qx,
+                                         float qy, float qz, float wv, SdfGrad& g)
+{
+    const float c = (float)cnt;
+    ax /= c;
+    ay /= c;
+    az /= c;
+    bx /= c;
+    by /= c;
+    bz /= c;
+    const float len = sqrtf(bx * bx + by * by + bz * bz);
+    if (!(len > 0.0f)) return false;  // zero mean normal: the forward leaves it unnormalised, no gradient
+    const float mx = bx / len, my = by / len, mz = bz / len;
+    const float dx = qx - ax, dy = qy - ay, dz = qz - az;
+    const float dm = dx * mx + dy * my + dz * mz;
+    // (I - m m^T)(v - c) / (|mt| kd)
+    const float tn = wv / (len * c);
+    g.nx = (dx - dm * mx) * tn;
+    g.ny = (dy - dm * my) * tn;
+    g.nz = (dz - dm * mz) * tn;
+    const float tp = -wv / c;
+    g.px = tp * mx;
+    g.py = tp * my;
+    g.pz = tp * mz;
+    return true;
+}
+
 // SDF reverse pass: the forward's kd-NN and ordered means, then dL/dp and dL/dn of the kd
 // neighbours (atomics into sorted-position arrays).
 template <int P>
@@ -87,31 +119,17 @@ struct SinkSdfAdjoint {
             by += ny[sp];
             bz += nz[sp];
         }
-        const float c = (float)cnt;
-        ax /= c;
-        ay /= c;
-        az /= c;
-        bx /= c;
-        by /= c;
-        bz /= c;
-        const float len = sqrtf(bx * bx + by * by + bz * bz);
-        if (!(len > 0.0f)) return;  // zero mean normal: the forward leaves it unnormalised, no gradient
-        const float mx = bx / len, my = by / len, mz = bz / len;
-        const float dx = qx - ax, dy = qy - ay, dz = qz - az;
-        const float dm = dx * mx + dy * my + dz * mz;
-        // (I - m m^T)(v - c) / (|mt| kd)
-        const float tn = wv / (len * c);
-        const float hx = (dx - dm * mx) * tn, hy = (dy - dm * my) * tn, hz = (dz - dm * mz) * tn;
-        const float tp = -wv / c;
+        SdfGrad gr;
+        if (!sdf_grad(ax, ay, az, bx, by, bz, cnt, qx, qy, qz, wv, gr)) return;
         for (int j = 0; j < cnt; j++) {
             const uint32_t sp = o[j];
             if (sp >= npts) continue;
-            atomicAdd(&gpx[sp], tp * mx);
-            atomicAdd(&gpy[sp], tp * my);
-            atomicAdd(&gpz[sp], tp * mz);
-            atomicAdd(&gnx[sp], hx);
-            atomicAdd(&gny[sp], hy);
-            atomicAdd(&gnz[sp], hz);
+            atomicAdd(&gpx[sp], gr.px);
+            atomicAdd(&gpy[sp], gr.py);
+            atomicAdd(&gpz[sp], gr.pz);
+            atomicAdd(&gnx[sp], gr.nx);
+            atomicAdd(&gny[sp], gr.ny);
+            atomicAdd(&gnz[sp], gr.nz);
         }
     }
 };

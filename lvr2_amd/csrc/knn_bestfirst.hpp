@@ -28,6 +28,7 @@
 // smallest keys, identical to the tile kernel's.
 #pragma once
 
+#include "adjoint.hpp"
 #include "common.hpp"
 #include "knn_tile.hpp"
 #include "lbvh.hpp"
@@ -385,7 +386,8 @@ __device__ __forceinline__ void bf_stats(unsigned long long* stats, bool valid, 
 // (KS_CANDIDATES), nodes expanded (KS_POPS), queries left to the next pass (KS_REFINE),
 // queries resolved (KS_RESOLVED), shader-clock cycles per wave (KS_CY_TOTAL).
 //
-// One lane per query (queries in Morton order), chunks of 64 consecutive queries per wave.  With
+// One lane per query (queries in Morton order), chunks of per_wave (at most 64) consecutive queries per
+// wave: fewer for a small batch (bf_per_wave).  With
 // a work queue (QUEUE_SEGS counters QUEUE_STRIDE apart, zeroed before the launch; the grid is
 // then the waves the device holds at once) the chunks are dealt like the tile kernel's runs:
 // blocks of QUEUE_CHUNK consecutive chunks to the XCDs in turn, each XCD taking from its own
@@ -400,11 +402,12 @@ __global__ __launch_bounds__(BF_THREADS) void bf_knn_kernel(const BvhView bv, co
                                                             const float* __restrict__ qz, int qs, int64_t m,
                                                             int t, uint64_t empty, Out out,
                                                             unsigned long long* stats, uint32_t* queue, uint2* spill,
-                                                            int spill_cap)
+                                                            int spill_cap, int per_wave, uint32_t* left,
+                                                            uint32_t* left_count)
 {
     __shared__ BfPool pool;
     const int lane = threadIdx.x;
-    const int64_t nchunks = (m + BF_THREADS - 1) / BF_THREADS;
+    const int64_t nchunks = (m + per_wave - 1) / per_wave;
     const int xcd = (int)(blockIdx.x % QUEUE_SEGS);
     int seg_k = 0;
     bool once = false;
@@ -418,7 +421,7 @@ __global__ __launch_bounds__(BF_THREADS) void bf_knn_kernel(const BvhView bv, co
         }
         if (chunk < 0 || chunk >= nchunks) break;
         const unsigned long long c0 = stats ? cycles() : 0ull;
-        const int64_t i = chunk * BF_THREADS + lane;
+        const int64_t i = lane < per_wave ? chunk * per_wave + lane : m;
         int leaves = 0, nodes = 0;
         bool ok = true;
         if (i < m) {  // no barrier in the search: lanes are independent
@@ -430,14 +433,15 @@ __global__ __launch_bounds__(BF_THREADS) void bf_knn_kernel(const BvhView bv, co
             BfLane ln{0u, 0, spill + (size_t)blockIdx.x * spill_cap * BF_THREADS + lane, spill_cap};
             ok = bf_search<K>(bv, pool, ln, lane, x, y, z, L, leaves, nodes);
             L.finish(bv.rank, t);
-            out.template emit<K>(i, L, t, ok, x, y, z);
+            // the queries left go to the next pass, in any order: each result is its query's own
+            if (!out.template emit<K>(i, L, t, ok, x, y, z)) left[atomicAdd(left_count, 1u)] = (uint32_t)i;
             ok = ok && L.full();
         }
         if (stats) bf_stats<K, Out>(stats, i < m, ok, leaves, nodes, c0);
     }
 }
 
-// Wave-cooperative best-first search for the queries list[0, *count): the ones whose lane search
+// Wave-cooperative best-first search for the queries list[0, *count) (list NULL: all of them): the ones whose lane search
 // overflowed its stack (a very dense or a far-off neighbourhood, hundreds of leaves deep).  One
 // wave per query: a greedy descent to a seed leaf; then every step pops up to 64 stack entries
 // at once, the lanes expand their nodes (children within the bound pushed) or scan their leaves,
@@ -445,6 +449,15 @@ __global__ __launch_bounds__(BF_THREADS) void bf_knn_kernel(const BvhView bv, co
 // wave-wide minimum.  Lane j holds the j-th key of the list in a register.  The serial chain is
 // the tree depth plus leaves / 64 steps, not one step per node or leaf.  A query whose stack
 // outgrows BF_WAVE_STACK entries is flagged for the tile kernel.
+// Zeroes a search's work queue and the counts of the queries its passes leave.
+static __global__ void bf_reset_kernel(uint32_t* queue, int n, uint32_t* count1, uint32_t* count2)
+{
+    for (int i = threadIdx.x; i < n; i += blockDim.x) queue[i] = 0u;
+    if (threadIdx.x == 0) {
+        *count1 = 0u;
+        *count2 = 0u;
+    }
+}
 constexpr int BF_WAVE_STACK = 4096;
 constexpr int BF_WAVE_BLOCKS = 1024;  // waves striding over the list
 
@@ -463,18 +476,20 @@ __global__ __launch_bounds__(BF_THREADS) void bf_knn_wave_kernel(const BvhView b
                                                                  const float* __restrict__ qy,
                                                                  const float* __restrict__ qz, int qs,
                                                                  const uint32_t* __restrict__ list,
-                                                                 const uint32_t* __restrict__ count, int t,
-                                                                 uint64_t empty, Out out, unsigned long long* stats)
+                                                                 const uint32_t* __restrict__ count, int64_t all,
+                                                                 int t, uint64_t empty, Out out,
+                                                                 unsigned long long* stats, uint32_t* left,
+                                                                 uint32_t* left_count)
 {
     __shared__ uint2 stk[BF_WAVE_STACK];
     __shared__ uint64_t fkey[BF_KMAX];
     __shared__ uint32_t fsp[BF_KMAX];
     const int lane = threadIdx.x;
-    const int64_t n = (int64_t)*count;
+    const int64_t n = list ? (int64_t)*count : all;
     const int root = bv.nleaf > 1 ? 0 : leaf_ref(0);
     for (int64_t j = blockIdx.x; j < n; j += gridDim.x) {
         const unsigned long long c0 = stats ? cycles() : 0ull;
-        const int64_t i = list[j];
+        const int64_t i = list ? (int64_t)list[j] : j;
         const float x = qx[i * qs], y = qy[i * qs], z = qz[i * qs];
         // lane j < t holds the j-th smallest key so far (empty: none)
         uint64_t bk = empty;
@@ -631,7 +646,7 @@ __global__ __launch_bounds__(BF_THREADS) void bf_knn_wave_kernel(const BvhView b
                 L.key[q] = q < K - t ? 0ull : fkey[o];
                 L.sp[q] = q < K - t ? ~0u : fsp[o];
             }
-            out.template emit<K>(i, L, t, ok, x, y, z);
+            if (!out.template emit<K>(i, L, t, ok, x, y, z)) left[atomicAdd(left_count, 1u)] = (uint32_t)i;
         }
         if (stats) {
             const int lsum = wave_sum_int(leaves), nsum = wave_sum_int(nodes);
@@ -649,7 +664,7 @@ __global__ __launch_bounds__(BF_THREADS) void bf_knn_wave_kernel(const BvhView b
 }
 
 // Signed distance from the sorted list: positions and normals summed in ascending key order
-// (tcc:435-449).  Queries whose search overflowed are flagged in redo[i] for the tile kernel.
+// (tcc:435-449).  emit returns whether the query is resolved: false for a search that overflowed or found too few points.
 struct BfSdfOut {
     const float* px;
     const float* py;
@@ -662,16 +677,14 @@ struct BfSdfOut {
     float* out_proj;
     float* out_eucl;
     uint8_t* out_invalid;
-    uint32_t* redo;
 
     template <int K>
-    __device__ __forceinline__ void emit(int64_t i, const BfList<K>& L, int t, bool ok, float qx, float qy,
+    __device__ __forceinline__ bool emit(int64_t i, const BfList<K>& L, int t, bool ok, float qx, float qy,
                                          float qz) const
     {
         // an unfilled slot (NaN coordinates) sorts last: the tile kernel handles such queries
         ok = ok && L.full();
-        redo[i] = ok ? 0u : 1u;
-        if (!ok) return;
+        if (!ok) return false;
         float ax = 0, ay = 0, az = 0, bx = 0, by = 0, bz = 0;
         float v[K][6];
 #pragma unroll
@@ -699,6 +712,63 @@ struct BfSdfOut {
         }
         sdf_emit(ax, ay, az, bx, by, bz, t, qx, qy, qz, voxel, qorig ? qorig[i] : (uint32_t)i, out_proj, out_eucl,
                  out_invalid);
+        return true;
+    }
+};
+
+// Reverse pass of the signed distance (SinkSdfAdjoint's sums, adjoint.hpp) from the sorted list.
+struct BfSdfAdjointOut {
+    const float* px;
+    const float* py;
+    const float* pz;
+    const float* nx;
+    const float* ny;
+    const float* nz;
+    const uint32_t* qorig;  // query position -> caller's index
+    const float* w;         // dL/dproj per caller index
+    float* gpx;             // dL/dp and dL/dn, sorted positions
+    float* gpy;
+    float* gpz;
+    float* gnx;
+    float* gny;
+    float* gnz;
+
+    template <int K>
+    __device__ __forceinline__ bool emit(int64_t i, const BfList<K>& L, int t, bool ok, float qx, float qy,
+                                         float qz) const
+    {
+        ok = ok && L.full();
+        if (!ok) return false;
+        const float wv = w[qorig[i]];
+        if (wv == 0.0f) return true;
+        float ax = 0, ay = 0, az = 0, bx = 0, by = 0, bz = 0;
+#pragma unroll
+        for (int j = 0; j < K; j++) {
+            if (j >= K - t) {
+                const uint32_t s = L.sp[j];
+                ax += px[s];
+                ay += py[s];
+                az += pz[s];
+                bx += nx[s];
+                by += ny[s];
+                bz += nz[s];
+            }
+        }
+        SdfGrad g;
+        if (!sdf_grad(ax, ay, az, bx, by, bz, t, qx, qy, qz, wv, g)) return true;
+#pragma unroll
+        for (int j = 0; j < K; j++) {
+            if (j >= K - t) {
+                const uint32_t s = L.sp[j];
+                atomicAdd(&gpx[s], g.px);
+                atomicAdd(&gpy[s], g.py);
+                atomicAdd(&gpz[s], g.pz);
+                atomicAdd(&gnx[s], g.nx);
+                atomicAdd(&gny[s], g.ny);
+                atomicAdd(&gnz[s], g.nz);
+            }
+        }
+        return true;
     }
 };
 
@@ -711,13 +781,11 @@ struct BfRowsOut {
     int32_t* idx;
     float* d2;
     int32_t* count;  // optional
-    uint32_t* redo;
 
     template <int K>
-    __device__ __forceinline__ void emit(int64_t i, const BfList<K>& L, int t, bool ok, float, float, float) const
+    __device__ __forceinline__ bool emit(int64_t i, const BfList<K>& L, int t, bool ok, float, float, float) const
     {
-        redo[i] = ok ? 0u : 1u;
-        if (!ok) return;
+        if (!ok) return false;
         const size_t row = qorig[i];
         int found = 0;
 #pragma unroll
@@ -735,6 +803,7 @@ struct BfRowsOut {
             if (d2) d2[row * k + o] = INFINITY;
         }
         if (count) count[row] = found;
+        return true;
     }
 };
 
@@ -749,14 +818,12 @@ struct BfMeanNormalOut {
     const uint32_t* qorig;
     int ki;
     float* out;  // caller order, 3 floats per query
-    uint32_t* redo;
 
     template <int K>
-    __device__ __forceinline__ void emit(int64_t i, const BfList<K>& L, int t, bool ok, float, float, float) const
+    __device__ __forceinline__ bool emit(int64_t i, const BfList<K>& L, int t, bool ok, float, float, float) const
     {
         ok = ok && L.full();
-        redo[i] = ok ? 0u : 1u;
-        if (!ok) return;
+        if (!ok) return false;
         float rx = 0.0f, ry = 1.0f, rz = 0.0f;
 #pragma unroll
         for (int j = 0; j < K; j++) {
@@ -782,6 +849,7 @@ struct BfMeanNormalOut {
         out[o] = rx;
         out[o + 1] = ry;
         out[o + 2] = rz;
+        return true;
     }
 };
 
@@ -791,7 +859,6 @@ struct BfCentroidOut {
     const float4* pts;  // sorted points
     const uint32_t* qorig;
     float* out;  // caller order, 3 floats per query
-    uint32_t* redo;
     // optional: the query's vertex (caller index -> vertex id) and, per vertex, the t neighbours
     // (sorted positions) of its last search, which a later search of the vertex starts from
     // (first_bound): their keys at the new position bound the search at once.  The result is the
@@ -823,11 +890,10 @@ struct BfCentroidOut {
     }
 
     template <int K>
-    __device__ __forceinline__ void emit(int64_t i, const BfList<K>& L, int t, bool ok, float qx, float qy,
+    __device__ __forceinline__ bool emit(int64_t i, const BfList<K>& L, int t, bool ok, float qx, float qy,
                                          float qz) const
     {
-        redo[i] = ok ? 0u : 1u;
-        if (!ok) return;
+        if (!ok) return false;
         if (vid && nbr) {
             const size_t v = vid[qorig[i]];
 #pragma unroll
@@ -851,12 +917,13 @@ struct BfCentroidOut {
             out[o] = qx;
             out[o + 1] = qy;
             out[o + 2] = qz;
-            return;
+            return true;
         }
         const float c = (float)nk;
         out[o] = cx / c;
         out[o + 1] = cy / c;
         out[o + 2] = cz / c;
+        return true;
     }
 };
 

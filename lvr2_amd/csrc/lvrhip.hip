@@ -611,52 +611,60 @@ __global__ void centroid_rows_kernel(int64_t m, int k, const int32_t* __restrict
 // holds t (10: the signed distance's usual kd).
 // Query coordinates: SoA (qs = 1) or AoS (qs = 3, qy = qx + 1, qz = qx + 2).  With a queue the
 // grid is min(chunks, resident) waves; spill holds spill_cap entries per lane for each of them.
+// Queries per wave: 64 fills the lanes, but a small batch runs on more waves with fewer lanes each, which
+// wait less for each other: 500 queries (t = 10) take 100 us, by the wave search, which took them before,
+// 137 us, and at t = 32 a quarter of its time.
+inline int bf_per_wave(int64_t m, int64_t resident)
+{
+    int p = 64;
+    while (p > 1 && ceil_div(m, (int64_t)p) < resident / 4) p /= 2;
+    return p;
+}
+
 template <class Out>
 void launch_bf(const BvhView& bv, const float* qx, const float* qy, const float* qz, int qs, int64_t m, int t,
                uint64_t empty, const Out& out, hipStream_t st, unsigned long long* stats, uint32_t* queue,
-               int64_t resident, uint2* spill, int spill_cap)
+               int64_t resident, uint2* spill, int spill_cap, uint32_t* left, uint32_t* left_count)
 {
     if (m == 0) return;
-    int64_t grid = ceil_div(m, BF_THREADS);
-    if (queue) {
-        grid = std::min(grid, resident);
-        fill_u32_kernel<<<1, 256, 0, st>>>(queue, QUEUE_SEGS * QUEUE_STRIDE, 0u);
-        LVRHIP_LAUNCH_CHECK();
-    }
+    const int pw = bf_per_wave(m, resident);
+    int64_t grid = ceil_div(m, (int64_t)pw);
+    if (queue) grid = std::min(grid, resident);
     const unsigned g = (unsigned)grid;
     if (t <= 8)
         bf_knn_kernel<8, Out><<<g, BF_THREADS, 0, st>>>(bv, qx, qy, qz, qs, m, t, empty, out, stats, queue, spill,
-                                                        spill_cap);
+                                                        spill_cap, pw, left, left_count);
     else if (t <= 10)
         bf_knn_kernel<10, Out><<<g, BF_THREADS, 0, st>>>(bv, qx, qy, qz, qs, m, t, empty, out, stats, queue, spill,
-                                                         spill_cap);
+                                                         spill_cap, pw, left, left_count);
     else if (t <= 16)
         bf_knn_kernel<16, Out><<<g, BF_THREADS, 0, st>>>(bv, qx, qy, qz, qs, m, t, empty, out, stats, queue, spill,
-                                                         spill_cap);
+                                                         spill_cap, pw, left, left_count);
     else
         bf_knn_kernel<32, Out><<<g, BF_THREADS, 0, st>>>(bv, qx, qy, qz, qs, m, t, empty, out, stats, queue, spill,
-                                                         spill_cap);
+                                                         spill_cap, pw, left, left_count);
     LVRHIP_LAUNCH_CHECK();
 }
 
 // The wave-per-query pass over list[0, *count) (the queries the lane pass left).
 template <class Out>
 void launch_bf_wave(const BvhView& bv, const float* qx, const float* qy, const float* qz, int qs,
-                    const uint32_t* list, const uint32_t* count, int t, uint64_t empty, const Out& out,
-                    hipStream_t st, unsigned long long* stats)
+                    const uint32_t* list, const uint32_t* count, int64_t all, int t, uint64_t empty, const Out& out,
+                    hipStream_t st, unsigned long long* stats, uint32_t* left, uint32_t* left_count)
 {
     const unsigned grid = BF_WAVE_BLOCKS;
     if (t <= 8)
-        bf_knn_wave_kernel<8, Out><<<grid, BF_THREADS, 0, st>>>(bv, qx, qy, qz, qs, list, count, t, empty, out, stats);
+        bf_knn_wave_kernel<8, Out><<<grid, BF_THREADS, 0, st>>>(bv, qx, qy, qz, qs, list, count, all, t, empty, out,
+                                                                 stats, left, left_count);
     else if (t <= 10)
-        bf_knn_wave_kernel<10, Out><<<grid, BF_THREADS, 0, st>>>(bv, qx, qy, qz, qs, list, count, t, empty, out,
-                                                                 stats);
+        bf_knn_wave_kernel<10, Out><<<grid, BF_THREADS, 0, st>>>(bv, qx, qy, qz, qs, list, count, all, t, empty, out,
+                                                                 stats, left, left_count);
     else if (t <= 16)
-        bf_knn_wave_kernel<16, Out><<<grid, BF_THREADS, 0, st>>>(bv, qx, qy, qz, qs, list, count, t, empty, out,
-                                                                 stats);
+        bf_knn_wave_kernel<16, Out><<<grid, BF_THREADS, 0, st>>>(bv, qx, qy, qz, qs, list, count, all, t, empty, out,
+                                                                 stats, left, left_count);
     else
-        bf_knn_wave_kernel<32, Out><<<grid, BF_THREADS, 0, st>>>(bv, qx, qy, qz, qs, list, count, t, empty, out,
-                                                                 stats);
+        bf_knn_wave_kernel<32, Out><<<grid, BF_THREADS, 0, st>>>(bv, qx, qy, qz, qs, list, count, all, t, empty, out,
+                                                                 stats, left, left_count);
     LVRHIP_LAUNCH_CHECK();
 }
 
@@ -722,18 +730,18 @@ struct Profiler {
 // ---- the no-allocation signed distances (lvrhip_distances_device_noalloc) -----------------------
 // Its scratch lives in one file-scope device array, `scratch`, that every device holds from the
 // moment the library's code object is loaded until the process ends.  Layout (byte offsets):
-// redo flags and redo list (NA_MAX_QUERIES entries each), compaction block sums, two counters,
-// the work queue, and the lane search's stack spill (NA_SPILL entries per lane for NA_WAVES
+// the lists of the queries the lane search and the wave search left (NA_MAX_QUERIES entries each), two
+// counters (behind a spare area that keeps the stated size), the work queue, and the lane search's stack spill (NA_SPILL entries per lane for NA_WAVES
 // waves).  Host code never uses the array's name: it asks hipGetSymbolAddress for the address
 // on each device once (na_scratch) and passes that pointer to the kernels.
 constexpr int64_t NA_MAX_QUERIES = 1 << 20;
 constexpr int NA_SPILL = 16;
 constexpr int64_t NA_WAVES = 2048;
 constexpr size_t na_align(size_t b) { return (b + 255) / 256 * 256; }
-constexpr size_t NA_FLAGS = 0;
-constexpr size_t NA_LIST = na_align(NA_FLAGS + 4 * (size_t)NA_MAX_QUERIES);
-constexpr size_t NA_BSUM = na_align(NA_LIST + 4 * (size_t)NA_MAX_QUERIES);
-constexpr size_t NA_COUNT = na_align(NA_BSUM + 4 * (size_t)(NA_MAX_QUERIES / CF_TILE + 2));
+constexpr size_t NA_LIST1 = 0;
+constexpr size_t NA_LIST2 = na_align(NA_LIST1 + 4 * (size_t)NA_MAX_QUERIES);
+constexpr size_t NA_SPARE = na_align(NA_LIST2 + 4 * (size_t)NA_MAX_QUERIES);
+constexpr size_t NA_COUNT = na_align(NA_SPARE + 4 * (size_t)(NA_MAX_QUERIES / CF_TILE + 2));
 constexpr size_t NA_QUEUE = na_align(NA_COUNT + 4 * 4);
 constexpr size_t NA_SPILL_OFF = na_align(NA_QUEUE + 4 * (size_t)(QUEUE_SEGS * QUEUE_STRIDE));
 constexpr size_t NA_BYTES = na_align(NA_SPILL_OFF + sizeof(uint2) * (size_t)NA_SPILL * BF_THREADS * NA_WAVES);
@@ -793,7 +801,7 @@ struct lvrhip_surface {
     // normals at positions) run best-first unless the tile kernel is forced
     int search_mode = LVRHIP_SEARCH_AUTO;
     int64_t bf_resident = 4096;  // best-first waves the device holds at once
-    DBuf<uint32_t> s_redo, s_redo_list;
+    DBuf<uint32_t> s_left1, s_left2;  // the queries the lane search and the wave search left
     DBuf<uint2> s_spill;  // the lane search's stack entries beyond its LDS part
 
     DBuf<float> px, py, pz;
@@ -832,7 +840,9 @@ struct lvrhip_surface {
     // (r = 2..5), [6] temporary list lengths of the merged rounds and the adjoint, [7] the
     // lattice's, [8] queries a best-first search left to the tile kernel, [9] / [10] the mesh's
     // face and vertex counts, [11] the most moves of one mesh vertex, [12] a move round's vertices
-    static constexpr int CNT_SLOTS = 16;
+    // [13] queries a best-first search left to the wave search, [15] the kNN error code
+    static constexpr int CNT_SLOTS = 16, CNT_ERR = 15;
+    static_assert(CNT_SLOTS * sizeof(uint32_t) <= DevicePool::PINNED_BYTES, "one readback of all counters");
     DBuf<uint32_t> d_cnt;
     uint32_t* counter(int i) const
     {
@@ -841,7 +851,6 @@ struct lvrhip_surface {
     }
     int64_t nq_first = 0;  // queries of the first round of the last normals pass
     int64_t n_round[5] = {0, 0, 0, 0, 0};
-    DBuf<int> err;
     Profiler prof;
     // work counters, KS_GROUPS groups x KS_COUNT: normals rounds 1..5, merged later rounds,
     // SDF, other searches (kSearch, the ki list, the adjoint)
@@ -918,7 +927,7 @@ struct lvrhip_surface {
         prm.area_pp = area.p;
         prm.r2_margin = r2_margin;
         prm.grow_min = 1.01f;
-        prm.err = err.p;
+        prm.err = (int*)counter(CNT_ERR);
         prm.stats = nullptr;
         (void)stats_group;
         return prm;
@@ -938,19 +947,20 @@ struct lvrhip_surface {
         return (int)k;
     }
 
+    // The device counters and the error code, in one readback.
     void read_err_and_counts()
     {
-        int e = 0;
-        uint32_t c[8] = {};
-        LVRHIP_CHECK(hipMemcpyAsync(&e, err.p, sizeof(int), hipMemcpyDeviceToHost, st));
-        if (d_cnt.p) LVRHIP_CHECK(hipMemcpyAsync(c, d_cnt.p, sizeof(c), hipMemcpyDeviceToHost, st));
-        LVRHIP_CHECK(hipStreamSynchronize(st));
-        if (d_cnt.p) {
-            n_round[0] = nq_first;
-            for (int r = 2; r <= 5; r++) n_round[r - 1] = c[r];
+        if (!d_cnt.p) {
+            LVRHIP_CHECK(hipStreamSynchronize(st));
+            return;
         }
+        LVRHIP_CHECK(hipMemcpyAsync(h_pin, d_cnt.p, CNT_SLOTS * sizeof(uint32_t), hipMemcpyDeviceToHost, st));
+        LVRHIP_CHECK(hipStreamSynchronize(st));
+        n_round[0] = nq_first;
+        for (int r = 2; r <= 5; r++) n_round[r - 1] = h_pin[r];
+        const int e = (int)h_pin[CNT_ERR];
         if (e != 0) {
-            fill_u32_kernel<<<1, 64, 0, st>>>((uint32_t*)err.p, 1, 0u);
+            fill_u32_kernel<<<1, 64, 0, st>>>(counter(CNT_ERR), 1, 0u);
             LVRHIP_LAUNCH_CHECK();
             LVRHIP_CHECK(hipStreamSynchronize(st));
             throw Error(LVRHIP_ECAPACITY, e == 5 ? "kNN traversal stack overflow" : "kNN radius search did not converge");
@@ -994,9 +1004,6 @@ struct lvrhip_surface {
         n = h_off[ns];
         npad = h_pstart[ns];
         src = d_xyz;
-        err.reserve(1);
-        fill_u32_kernel<<<1, 64, 0, st>>>((uint32_t*)err.p, 1, 0u);
-        LVRHIP_LAUNCH_CHECK();
         d_cnt.reserve(CNT_SLOTS);
         fill_u32_kernel<<<1, 64, 0, st>>>(d_cnt.p, CNT_SLOTS, 0u);
         LVRHIP_LAUNCH_CHECK();
@@ -1124,7 +1131,7 @@ struct lvrhip_surface {
         LVRHIP_LAUNCH_CHECK();
         median_kernel<<<1, 1024, 0, st>>>(s_f.p, nsample, area.p);
         LVRHIP_LAUNCH_CHECK();
-        fill_u32_kernel<<<1, 64, 0, st>>>((uint32_t*)err.p, 1, 0u);
+        fill_u32_kernel<<<1, 64, 0, st>>>(counter(CNT_ERR), 1, 0u);
         LVRHIP_LAUNCH_CHECK();
         prof.stop(tok, st);
     }
@@ -1743,12 +1750,11 @@ struct lvrhip_surface {
         const uint32_t* nq_dev = nullptr;
         if (bf) {
             // best-first for every vertex; the tile kernel redoes the ones whose stacks overflowed
-            s_redo.reserve(m);
-            BfSdfOut o{px.p, py.p, pz.p, nx.p, ny.p, nz.p, s_v0.p, voxel, d_proj, d_eucl, d_inv, s_redo.p};
+            BfSdfOut o{px.p, py.p, pz.p, nx.p, ny.p, nz.p, s_v0.p, voxel, d_proj, d_eucl, d_inv};
             const int tok = prof.start(LVRHIP_T_SDF_KERNEL, st);
             enqueue_bf(m, t0, BF_EMPTY, o, 6);
             prof.stop(tok, st);
-            qsel = s_redo_list.p;
+            qsel = s_left2.p;
             nq_dev = counter(8);
         }
         TileParams prm = params(t0, 0, 2);
@@ -1804,19 +1810,17 @@ struct lvrhip_surface {
         const int t0 = clamp_k(kd);
         if (t0 > BF_KMAX)
             throw Error(LVRHIP_EINVAL, "the no-allocation distances take kd <= " + std::to_string(BF_KMAX));
-        uint32_t* flags = reinterpret_cast<uint32_t*>(scr + NA_FLAGS);
-        uint32_t* list = reinterpret_cast<uint32_t*>(scr + NA_LIST);
-        uint32_t* bsum = reinterpret_cast<uint32_t*>(scr + NA_BSUM);
+        uint32_t* list1 = reinterpret_cast<uint32_t*>(scr + NA_LIST1);
+        uint32_t* list2 = reinterpret_cast<uint32_t*>(scr + NA_LIST2);
         uint32_t* cnt = reinterpret_cast<uint32_t*>(scr + NA_COUNT);
         uint32_t* queue = reinterpret_cast<uint32_t*>(scr + NA_QUEUE);
         uint2* spill = reinterpret_cast<uint2*>(scr + NA_SPILL_OFF);
-        BfSdfOut o{px.p, py.p, pz.p, nx.p, ny.p, nz.p, nullptr, voxel, d_proj, d_eucl, d_inv, flags};
-        // every flag is written by the lane search; the queue is cleared by launch_bf
+        BfSdfOut o{px.p, py.p, pz.p, nx.p, ny.p, nz.p, nullptr, voxel, d_proj, d_eucl, d_inv};
+        bf_reset_kernel<<<1, 256, 0, st>>>(queue, QUEUE_SEGS * QUEUE_STRIDE, cnt, cnt + 1);
+        LVRHIP_LAUNCH_CHECK();
         launch_bf(view(), d_q, d_q + 1, d_q + 2, 3, m, t0, BF_EMPTY, o, st, nullptr, queue,
-                  std::min(bf_resident, NA_WAVES), spill, NA_SPILL);
-        compact_flags_with(flags, m, nullptr, nullptr, list, cnt, bsum);
-        launch_bf_wave(view(), d_q, d_q + 1, d_q + 2, 3, list, cnt, t0, BF_EMPTY, o, st, nullptr);
-        compact_flags_with(flags, m, nullptr, nullptr, list, cnt + 1, bsum);
+                  std::min(bf_resident, NA_WAVES), spill, NA_SPILL, list1, cnt);
+        launch_bf_wave(view(), d_q, d_q + 1, d_q + 2, 3, list1, cnt, m, t0, BF_EMPTY, o, st, nullptr, list2, cnt + 1);
         LVRHIP_CHECK(hipMemcpyAsync(h_pin, cnt + 1, sizeof(uint32_t), hipMemcpyDeviceToHost, st));
         LVRHIP_CHECK(hipStreamSynchronize(st));
         const uint32_t left = h_pin[0];
@@ -2139,14 +2143,26 @@ struct lvrhip_surface {
         zero_f32_kernel<<<(unsigned)ceil_div(3 * R, 256), 256, 0, st>>>(g_n.p, 3 * R);
         LVRHIP_LAUNCH_CHECK();
         sort_queries(d_q, m);
-        // 1. SDF reverse: dL/dp (through the means) and dL/dn of every vertex's kd neighbours
+        // 1. SDF reverse: dL/dp (through the means) and dL/dn of every vertex's kd neighbours, best-first like
+        // the forward (3.8 -> 1.24 ms for 500,000 vertices of the 1M-point cloud); the tile kernel does the
+        // vertices that left
+        const uint32_t* qsel = nullptr;
+        const uint32_t* nq_dev = nullptr;
+        const bool bf = best_first(t0);
+        if (bf) {
+            BfSdfAdjointOut o{px.p, py.p, pz.p, nx.p, ny.p, nz.p, s_v0.p, d_w, g_p.p, g_p.p + R, g_p.p + 2 * R,
+                              g_n.p, g_n.p + R, g_n.p + 2 * R};
+            enqueue_bf(m, t0, BF_EMPTY, o, 7);
+            qsel = s_left2.p;
+            nq_dev = counter(8);
+        }
         {
             TileParams prm = params(t0, 0, 2);
             prm.tiles_per_wave = sdf_tiles_per_wave;
             prm.r2_margin = sdf_r2_margin;
             prm.grow_min = sdf_grow_min;
             prm.stats = kstats_ptr(6);
-            QueryView qv{s_qx.p, s_qy.p, s_qz.p, nullptr, (uint32_t)m, nullptr};
+            QueryView qv{s_qx.p, s_qy.p, s_qz.p, qsel, (uint32_t)m, nq_dev};
             auto mk = [&](auto tag) {
                 constexpr int P = decltype(tag)::value;
                 SinkSdfAdjoint<P> s{};
@@ -2172,7 +2188,8 @@ struct lvrhip_surface {
                 return s;
             };
             tile<SinkSdfAdjoint>(qv, prm, lanes_per_query, mk(std::integral_constant<int, 2>()),
-                                 mk(std::integral_constant<int, 4>()), mk(std::integral_constant<int, 8>()));
+                                 mk(std::integral_constant<int, 4>()), mk(std::integral_constant<int, 8>()),
+                                 bf ? resident_waves / 16 : 0);
         }
         // 2. dL/dC per point with a normal gradient
         pca_adjoint_prep_kernel<<<(unsigned)ceil_div(R, 256), 256, 0, st>>>(
@@ -2209,43 +2226,35 @@ struct lvrhip_surface {
     bool best_first(int t) const { return search_mode != LVRHIP_SEARCH_TILE && t >= 1 && t <= BF_KMAX; }
 
     // Best-first search of the m sorted queries s_q*: one lane per query for all of them, then one
-    // wave per query for those whose lane stack overflowed; the queries both left (redo flags
-    // set by Out) end up in s_redo_list[0, *counter(8)), for the tile kernel.  Enqueue only.
+    // wave per query for those whose lane pool overflowed; the queries both left end up in
+    // s_left2[0, *counter(8)), for the tile kernel.  Enqueue only: three launches.
     template <class Out>
     void enqueue_bf(int64_t m, int t0, uint64_t empty, const Out& o, int stats_group)
     {
-        s_redo.reserve(m);
-        s_redo_list.reserve(m);
-        // A small batch goes to the wave-per-query search at once: the lane search would run it on
-        // a few waves, each as slow as its slowest lane, while every query here gets a wave.
-        if (search_mode == LVRHIP_SEARCH_WAVE || (search_mode == LVRHIP_SEARCH_AUTO && m <= BF_WAVE_BLOCKS)) {
-            fill_u32_kernel<<<(unsigned)ceil_div(m, 256), 256, 0, st>>>(s_redo.p, m, 1u);
-            LVRHIP_LAUNCH_CHECK();
-        } else {
-            uint32_t* q = nullptr;
-            if (use_queue) {
-                d_queue.reserve(QUEUE_SEGS * QUEUE_STRIDE);
-                q = d_queue.p;
-            }
+        s_left1.reserve(m);
+        s_left2.reserve(m);
+        d_queue.reserve(QUEUE_SEGS * QUEUE_STRIDE);
+        bf_reset_kernel<<<1, 256, 0, st>>>(d_queue.p, QUEUE_SEGS * QUEUE_STRIDE, counter(13), counter(8));
+        LVRHIP_LAUNCH_CHECK();
+        const bool lanes = search_mode != LVRHIP_SEARCH_WAVE;
+        if (lanes) {
+            uint32_t* q = use_queue ? d_queue.p : nullptr;
             // one spill area per wave of the grid
-            const int64_t waves = q ? std::min(ceil_div(m, BF_THREADS), bf_resident) : ceil_div(m, BF_THREADS);
+            const int64_t all = ceil_div(m, (int64_t)bf_per_wave(m, bf_resident));
+            const int64_t waves = q ? std::min(all, bf_resident) : all;
             s_spill.reserve((size_t)waves * BF_SPILL * BF_THREADS);
             launch_bf(view(), s_qx.p, s_qy.p, s_qz.p, 1, m, t0, empty, o, st, kstats_ptr(stats_group), q, bf_resident,
-                      s_spill.p, BF_SPILL);
+                      s_spill.p, BF_SPILL, s_left1.p, counter(13));
         }
-        compact_flags(s_redo.p, m, nullptr, nullptr, s_redo_list.p, counter(8));
-        launch_bf_wave(view(), s_qx.p, s_qy.p, s_qz.p, 1, s_redo_list.p, counter(8), t0, empty, o, st,
-                       kstats_ptr(stats_group == 6 ? 5 : stats_group));
-        compact_flags(s_redo.p, m, nullptr, nullptr, s_redo_list.p, counter(8));
+        launch_bf_wave(view(), s_qx.p, s_qy.p, s_qz.p, 1, lanes ? s_left1.p : nullptr, counter(13), m, t0, empty, o, st,
+                       kstats_ptr(stats_group == 6 ? 5 : stats_group), s_left2.p, counter(8));
     }
 
-    // Number of queries the last enqueue_bf left to the tile kernel (synchronises).
-    uint32_t bf_redo_count()
+    // Number of queries the last enqueue_bf left to the tile kernel (synchronises, and reports errors).
+    uint32_t bf_left()
     {
-        uint32_t c = 0;
-        LVRHIP_CHECK(hipMemcpyAsync(&c, counter(8), sizeof(c), hipMemcpyDeviceToHost, st));
-        LVRHIP_CHECK(hipStreamSynchronize(st));
-        return c;
+        check_err();
+        return h_pin[8];
     }
 
     // Sorted kSearch rows (input index, d^2; padded with -1 / +inf) for m device queries.  With
@@ -2267,14 +2276,10 @@ struct lvrhip_surface {
         }
         sort_queries(d_q, m);
         if (best_first(t0)) {
-            s_redo.reserve(m);
             const uint64_t empty = r2 >= 0.0f ? ((uint64_t)host_fbits(r2) << 32) : BF_EMPTY;
-            BfRowsOut o{s_v0.p, k, d_idx, d_d2, d_count, s_redo.p};
+            BfRowsOut o{s_v0.p, k, d_idx, d_d2, d_count};
             enqueue_bf(m, t0, empty, o, 7);
-            if (bf_redo_count() == 0) {
-                check_err();
-                return;
-            }
+            if (bf_left() == 0) return;
         }
         // the tile kernel for every query (also when a best-first stack overflowed)
         DBuf<uint64_t> keys;
@@ -2319,13 +2324,9 @@ struct lvrhip_surface {
         const int t0 = clamp_k(kc);
         if (best_first(t0)) {
             sort_queries(d_q, m);
-            s_redo.reserve(m);
-            BfCentroidOut o{pts4.p, s_v0.p, d_out, s_redo.p, vid, nbr, prefill, (uint32_t)npad};
+            BfCentroidOut o{pts4.p, s_v0.p, d_out, vid, nbr, prefill, (uint32_t)npad};
             enqueue_bf(m, t0, BF_EMPTY, o, 7);
-            if (bf_redo_count() == 0) {
-                check_err();
-                return;
-            }
+            if (bf_left() == 0) return;
         }
         DBuf<int32_t> idx;
         idx.reserve((size_t)m * t0);
@@ -2355,13 +2356,9 @@ struct lvrhip_surface {
         const int t0 = clamp_k(ki);
         if (best_first(t0)) {
             sort_queries(d_q, m);
-            s_redo.reserve(m);
-            BfMeanNormalOut o{nx.p, ny.p, nz.p, s_v0.p, ki, d_out, s_redo.p};
+            BfMeanNormalOut o{nx.p, ny.p, nz.p, s_v0.p, ki, d_out};
             enqueue_bf(m, t0, BF_EMPTY, o, 7);
-            if (bf_redo_count() == 0) {
-                check_err();
-                return;
-            }
+            if (bf_left() == 0) return;
         }
         DBuf<int32_t> idx;
         idx.reserve((size_t)m * t0);
