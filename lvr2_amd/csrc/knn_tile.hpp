@@ -109,6 +109,7 @@ struct TileParams {
     uint32_t* queue;            // optional work queue (QUEUE_SEGS counters QUEUE_STRIDE apart,
                                 // zeroed before the launch): waves take the next run of
                                 // tiles_per_wave tiles from it; else runs are strided over the grid
+    bool queue_zeroed;          // (host) the caller has zeroed it
     const float* hint_in;       // optional, per query position: the d^2 of its t-th key for an earlier
                                 // target t; a tile's first radius^2 is hint_scale times the largest
                                 // over its queries (else the radius carried from the previous tile)

@@ -21,8 +21,10 @@ void launch_tile_p(const BvhView& bv, const QueryView& qv, const TileParams& prm
     if (grid == 0) return;
     if (prm.queue) {
         grid = std::min(grid, resident);
-        fill_u32_kernel<<<1, 256, 0, st>>>(prm.queue, QUEUE_SEGS * QUEUE_STRIDE, 0u);
-        LVRHIP_LAUNCH_CHECK();
+        if (!prm.queue_zeroed) {
+            fill_u32_kernel<<<1, 256, 0, st>>>(prm.queue, QUEUE_SEGS * QUEUE_STRIDE, 0u);
+            LVRHIP_LAUNCH_CHECK();
+        }
     }
     if (prm.stats)
         knn_tile_kernel<P, SinkT<P>, true><<<(unsigned)grid, kWave, 0, st>>>(bv, qv, prm, sink);

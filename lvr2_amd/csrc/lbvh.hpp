@@ -344,11 +344,12 @@ static __global__ __launch_bounds__(256) void karras_kernel(const uint64_t* __re
 
 // Refit without atomics.  Every node of the Karras tree covers a contiguous leaf range
 // [min(i, r.w), max(i, r.w)], so its box is the union of the leaf boxes over that range: a range
-// union, answered from the doubling table T_j[i] = union of leaves [i, i + 2^j) as
-// T_j[first] U T_j[last - 2^j + 1] with j = floor(log2(length)).  Level j is built from level j - 1
-// (two buffers in turn), then the nodes whose length has that j take their box and write it into
-// their parent's child slot; leaves write theirs first.  Every slot has one writer, and min / max
-// give the same box in any order, so the result is the bottom-up refit's.
+// union, answered from blocks of 16, 256, 4,096 ... leaves (each level the unions of 16 entries of the one
+// below) by at most 15 entries of every level at either end of the range; half of the nodes cover two
+// leaves and read just those.  Every node writes its box into its parent's child slot, leaves theirs
+// before; every slot has one writer, and min / max give the same box in any order, so the result is the
+// bottom-up refit's.  (A doubling table with a launch per level for it and one for the nodes of that level took
+// 20 launches for 30,000 points and 36 for 4M, now 4 and 6.)
 
 // one child's box in its parent's a / b / c fields (left: a.xyzw b.xy, right: b.zw c.xyzw)
 __device__ __forceinline__ void put_child_box(BvhNode* nd, bool left, const float4& lo, const float4& hi)
@@ -375,36 +376,56 @@ static __global__ __launch_bounds__(256) void refit_leaf_slots_kernel(int nl, co
     put_child_box(&nodes[p], nodes[p].r.x == leaf_ref(leaf), leaf_lo[leaf], leaf_hi[leaf]);
 }
 
-// level j of the doubling table from level j - 1 (half = 2^(j-1)); entries i <= nl - 2 * half
-static __global__ __launch_bounds__(256) void range_union_level_kernel(int nl, int half, const float4* __restrict__ lo_in,
-                                                                const float4* __restrict__ hi_in,
-                                                                float4* __restrict__ lo_out, float4* __restrict__ hi_out)
+constexpr int REFIT_RADIX = 16;
+constexpr int REFIT_LEVELS = 8;  // 16^8 leaves
+struct RefitLevels {
+    const float4* lo[REFIT_LEVELS];  // [0]: the leaves
+    const float4* hi[REFIT_LEVELS];
+    int n;
+};
+
+// one level of blocks from the level below
+static __global__ __launch_bounds__(256) void refit_blocks_kernel(int n_in, const float4* __restrict__ lo_in,
+                                                                  const float4* __restrict__ hi_in,
+                                                                  float4* __restrict__ lo_out,
+                                                                  float4* __restrict__ hi_out)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i > nl - 2 * half) return;
-    const float4 a = lo_in[i], b = lo_in[i + half], c = hi_in[i], d = hi_in[i + half];
-    lo_out[i] = make_float4(fminf(a.x, b.x), fminf(a.y, b.y), fminf(a.z, b.z), 0.0f);
-    hi_out[i] = make_float4(fmaxf(c.x, d.x), fmaxf(c.y, d.y), fmaxf(c.z, d.z), 0.0f);
+    const int o = blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t first = (int64_t)o * REFIT_RADIX;
+    if (first >= n_in) return;
+    float4 lo = make_float4(INFINITY, INFINITY, INFINITY, 0.0f), hi = make_float4(-INFINITY, -INFINITY, -INFINITY, 0.0f);
+#pragma unroll
+    for (int k = 0; k < REFIT_RADIX; k++) {
+        const int64_t i = first + k < n_in ? first + k : n_in - 1;
+        const float4 a = lo_in[i], b = hi_in[i];
+        lo = make_float4(fminf(lo.x, a.x), fminf(lo.y, a.y), fminf(lo.z, a.z), 0.0f);
+        hi = make_float4(fmaxf(hi.x, b.x), fmaxf(hi.y, b.y), fmaxf(hi.z, b.z), 0.0f);
+    }
+    lo_out[o] = lo;
+    hi_out[o] = hi;
 }
 
-// the internal nodes whose leaf count has floor(log2) == j: own box, and the parent's child slot
-static __global__ __launch_bounds__(256) void refit_level_kernel(int nint, int j, const float4* __restrict__ tlo,
-                                                          const float4* __restrict__ thi, BvhNode* nodes,
-                                                          float4* __restrict__ node_lo, float4* __restrict__ node_hi)
+static __global__ __launch_bounds__(256) void refit_nodes_kernel(int nint, const RefitLevels t, BvhNode* nodes)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= nint) return;
     const int4 r = nodes[i].r;
-    const int first = min(i, r.w), last = max(i, r.w);
-    const int len = last - first + 1;
-    if (31 - __clz(len) != j) return;
-    const int second = last - (1 << j) + 1;
-    const float4 a = tlo[first], b = tlo[second], c = thi[first], d = thi[second];
-    const float4 lo = make_float4(fminf(a.x, b.x), fminf(a.y, b.y), fminf(a.z, b.z), 0.0f);
-    const float4 hi = make_float4(fmaxf(c.x, d.x), fmaxf(c.y, d.y), fmaxf(c.z, d.z), 0.0f);
-    node_lo[i] = lo;
-    node_hi[i] = hi;
-    if (r.z >= 0) put_child_box(&nodes[r.z], nodes[r.z].r.x == i, lo, hi);
+    if (r.z < 0) return;  // the root's box is in no slot
+    int a = min(i, r.w), b = max(i, r.w) + 1;
+    float4 lo = make_float4(INFINITY, INFINITY, INFINITY, 0.0f), hi = make_float4(-INFINITY, -INFINITY, -INFINITY, 0.0f);
+    for (int l = 0; l < t.n && a < b; l++) {
+        auto take = [&](int j) {
+            const float4 c = t.lo[l][j], d = t.hi[l][j];
+            lo = make_float4(fminf(lo.x, c.x), fminf(lo.y, c.y), fminf(lo.z, c.z), 0.0f);
+            hi = make_float4(fmaxf(hi.x, d.x), fmaxf(hi.y, d.y), fmaxf(hi.z, d.z), 0.0f);
+        };
+        const bool top = l == t.n - 1;
+        while (a < b && (top || a % REFIT_RADIX)) take(a++);
+        while (a < b && b % REFIT_RADIX) take(--b);
+        a /= REFIT_RADIX;
+        b /= REFIT_RADIX;
+    }
+    put_child_box(&nodes[r.z], nodes[r.z].r.x == i, lo, hi);
 }
 
 // BvhNode4 of every internal node.  One thread per node.

@@ -166,6 +166,23 @@ __device__ __forceinline__ int64_t cf_entry(int r)
     return (int64_t)blockIdx.x * CF_TILE + (int64_t)(threadIdx.x / kWave) * (CF_ITEMS * kWave) + r * kWave + lane_id();
 }
 
+// Sum of a[0, n) over the block's threads, on every thread.
+__device__ __forceinline__ uint32_t cf_block_sum(const uint32_t* __restrict__ a, int n, uint32_t* sh)
+{
+    uint32_t s = 0;
+    for (int j = threadIdx.x; j < n; j += CF_THREADS) s += a[j];
+    const uint32_t w = (uint32_t)wave_sum_int((int)s);
+    if (lane_id() == 0) sh[threadIdx.x / kWave] = w;
+    __syncthreads();
+    uint32_t t = 0;
+    for (int k = 0; k < CF_WAVES; k++) t += sh[k];
+    __syncthreads();
+    return t;
+}
+// Up to this many blocks the scatter kernels add up the counts before theirs themselves (a scan launch takes
+// about 5 us on the device, more than the sums of 1,024 counts in every block).
+constexpr int CF_SELF_BLOCKS = 1024;
+
 __global__ __launch_bounds__(CF_THREADS) void flag_block_sums_kernel(const CompactIf pred, int64_t n,
                                                                      const uint32_t* __restrict__ n_dev,
                                                                      uint32_t* __restrict__ bsum)
@@ -194,12 +211,17 @@ __global__ __launch_bounds__(CF_THREADS) void flag_block_sums_kernel(const Compa
 
 __global__ __launch_bounds__(CF_THREADS) void compact_scatter_kernel(const CompactIf pred, int64_t n,
                                                                      const uint32_t* __restrict__ n_dev,
-                                                                     const uint32_t* __restrict__ boff,
+                                                                     const uint32_t* __restrict__ boff, bool self,
+                                                                     uint32_t* __restrict__ count,
                                                                      uint32_t* __restrict__ out)
 {
+    // self: boff holds the blocks' counts (else their offsets), and the last block writes their sum
     __shared__ uint32_t ws[CF_WAVES];
     if (n_dev) n = (int64_t)*n_dev < n ? (int64_t)*n_dev : n;
+    if (self && n == 0 && blockIdx.x == 0 && threadIdx.x == 0 && count) *count = 0u;
     if ((int64_t)blockIdx.x * CF_TILE >= n) return;
+    uint32_t run = self ? cf_block_sum(boff, blockIdx.x, ws) : boff[blockIdx.x];
+    if (self && count && threadIdx.x == 0 && (int64_t)(blockIdx.x + 1) * CF_TILE >= n) *count = run + boff[blockIdx.x];
     const int wave = threadIdx.x / kWave;
     uint32_t pt[CF_ITEMS], c = 0;
     bool f[CF_ITEMS];
@@ -213,7 +235,6 @@ __global__ __launch_bounds__(CF_THREADS) void compact_scatter_kernel(const Compa
     for (int r = 0; r < CF_ITEMS; r++) c += (uint32_t)__popcll(ballot(f[r]));
     if (lane_id() == 0) ws[wave] = c;
     __syncthreads();
-    uint32_t run = boff[blockIdx.x];
     for (int w = 0; w < wave; w++) run += ws[w];
 #pragma unroll
     for (int r = 0; r < CF_ITEMS; r++) {
@@ -274,17 +295,34 @@ __global__ __launch_bounds__(CF_THREADS) void part_sums_kernel(const uint8_t* __
 __global__ __launch_bounds__(CF_THREADS) void part_scatter_kernel(const uint8_t* __restrict__ act,
                                                                   const uint32_t* __restrict__ list,
                                                                   const uint32_t* __restrict__ n_dev, uint32_t spec, int64_t nq,
-                                                                  const uint32_t* __restrict__ boff,
+                                                                  const uint32_t* __restrict__ boff, bool self,
                                                                   const uint32_t* __restrict__ total,
                                                                   uint32_t* __restrict__ out, uint32_t* __restrict__ seg)
 {
-    __shared__ uint32_t ws[CF_WAVES][ROUND_SEGS];
+    // self: boff holds the blocks' counts (else their offsets)
+    __shared__ uint32_t ws[CF_WAVES][ROUND_SEGS], start[ROUND_SEGS + 1];
     const int64_t n = (int64_t)*n_dev;
-    if (blockIdx.x == 0 && threadIdx.x <= ROUND_SEGS) {
-        seg[threadIdx.x] = threadIdx.x < ROUND_SEGS ? boff[(size_t)threadIdx.x * gridDim.x] : *total;
-        if (threadIdx.x == ROUND_SEGS) seg[ROUND_SEGS + 1] = n <= spec ? 1u : 0u;
+    if (blockIdx.x > 0 && (int64_t)blockIdx.x * CF_TILE >= n) return;
+    uint32_t run[ROUND_SEGS];
+    if (self) {
+        const int used = (int)((n + CF_TILE - 1) / CF_TILE), mine = min((int)blockIdx.x, used);  // later blocks: 0
+        uint32_t before = 0;
+        for (int k = 0; k < ROUND_SEGS; k++) {
+            const uint32_t* c = boff + (size_t)k * gridDim.x;
+            const uint32_t lo = cf_block_sum(c, mine, &ws[0][0]), hi = cf_block_sum(c + mine, used - mine, &ws[0][0]);
+            if (threadIdx.x == 0) start[k] = before;
+            run[k] = before + lo;
+            before += lo + hi;
+        }
+        if (threadIdx.x == 0) start[ROUND_SEGS] = before;
+        __syncthreads();
+        if (blockIdx.x == 0 && threadIdx.x <= ROUND_SEGS) seg[threadIdx.x] = start[threadIdx.x];
+    } else {
+        for (int k = 0; k < ROUND_SEGS; k++) run[k] = boff[(size_t)k * gridDim.x + blockIdx.x];
+        if (blockIdx.x == 0 && threadIdx.x <= ROUND_SEGS)
+            seg[threadIdx.x] = threadIdx.x < ROUND_SEGS ? boff[(size_t)threadIdx.x * gridDim.x] : *total;
     }
-    if ((int64_t)blockIdx.x * CF_TILE >= n) return;
+    if (blockIdx.x == 0 && threadIdx.x == 0) seg[ROUND_SEGS + 1] = n <= spec ? 1u : 0u;
     const int wave = threadIdx.x / kWave;
     uint32_t pt[CF_ITEMS], sg[CF_ITEMS], c[ROUND_SEGS] = {};
 #pragma unroll
@@ -301,12 +339,9 @@ __global__ __launch_bounds__(CF_THREADS) void part_scatter_kernel(const uint8_t*
 #pragma unroll
         for (int k = 0; k < ROUND_SEGS; k++) ws[wave][k] = c[k];
     __syncthreads();
-    uint32_t run[ROUND_SEGS];
 #pragma unroll
-    for (int k = 0; k < ROUND_SEGS; k++) {
-        run[k] = boff[(size_t)k * gridDim.x + blockIdx.x];
+    for (int k = 0; k < ROUND_SEGS; k++)
         for (int w = 0; w < wave; w++) run[k] += ws[w][k];
-    }
 #pragma unroll
     for (int r = 0; r < CF_ITEMS; r++)
 #pragma unroll
@@ -796,6 +831,7 @@ struct lvrhip_surface {
     // capped at what the device holds at once
     bool use_queue = true;
     int64_t resident_waves = 4096;
+    static constexpr int QUEUES = 5;  // the normals pass's launches
     DBuf<uint32_t> d_queue;
     // searches with at most BF_KMAX neighbours (distances, kSearch, radius search, interpolated
     // normals at positions) run best-first unless the tile kernel is forced
@@ -814,14 +850,14 @@ struct lvrhip_surface {
     DBuf<uint32_t> sbox;
     DBuf<MortonFrame> frames;
     DBuf<float> area;  // median leaf area per point: the first radius guess
-    DBuf<float4> leaf_lo, leaf_hi, nlo, nhi;
+    DBuf<float4> leaf_lo, leaf_hi;
     DBuf<float4> leaf_agg;  // per leaf: its point sums about the box centre (3 float4)
     DBuf<int> fr_ref;       // per scan: the FRONTIER top-level subtrees (frontier_kernel)
     DBuf<float4> fr_lo, fr_hi;
     DBuf<BvhNode> nodes;
     DBuf<BvhNode4> nodes4;
     DBuf<int> leaf_parent;
-    DBuf<float4> ru_lo[2], ru_hi[2];  // the refit's range-union levels, in turn
+    DBuf<float4> ru_lo, ru_hi;  // the refit's block unions, level after level
     int nleaf = 0;
 
     DBuf<float> nx, ny, nz, tx, ty, tz;
@@ -968,16 +1004,18 @@ struct lvrhip_surface {
     }
     void check_err() { read_err_and_counts(); }
 
+    // queue: one of the work queues that the caller has zeroed together (-1: zero the first for this launch).
     // max_waves (with the work queue): the grid's cap, below the waves the device holds for a
     // query list that is usually near empty (the launch then costs less than a full grid).
     template <template <int> class SinkT>
     void tile(const QueryView& qv, const TileParams& prm_in, int P, SinkT<2> s2, SinkT<4> s4, SinkT<8> s8,
-              int64_t max_waves = 0)
+              int64_t max_waves = 0, int queue = -1)
     {
         TileParams prm = prm_in;
         if (use_queue) {
-            d_queue.reserve(QUEUE_SEGS * QUEUE_STRIDE);
-            prm.queue = d_queue.p;
+            d_queue.reserve((size_t)QUEUES * QUEUE_SEGS * QUEUE_STRIDE);
+            prm.queue = d_queue.p + (size_t)std::max(queue, 0) * QUEUE_SEGS * QUEUE_STRIDE;
+            prm.queue_zeroed = queue >= 0;
         }
         const int64_t cap = max_waves > 0 ? std::min(max_waves, resident_waves) : resident_waves;
         switch (P) {
@@ -1044,14 +1082,11 @@ struct lvrhip_surface {
         leaf_parent.reserve(nleaf);
         nodes.reserve(nint);
         nodes4.reserve(nint);
-        nlo.reserve(nint);
-        nhi.reserve(nint);
         s_flags.reserve(std::max<int64_t>(nint, n));
         s_f.reserve(MEDIAN_MAX);
-        for (int b = 0; b < 2; b++) {
-            ru_lo[b].reserve(nleaf);
-            ru_hi[b].reserve(nleaf);
-        }
+        // a fifteenth of the leaves, and one entry more per level
+        ru_lo.reserve((size_t)nleaf / (REFIT_RADIX - 1) + REFIT_LEVELS);
+        ru_hi.reserve((size_t)nleaf / (REFIT_RADIX - 1) + REFIT_LEVELS);
     }
 
     // LBVH build from `src`, entirely on the device (no host synchronisation).
@@ -1093,23 +1128,27 @@ struct lvrhip_surface {
         if (nleaf > 1) {
             karras_kernel<<<(unsigned)ceil_div(nleaf - 1, 256), 256, 0, st>>>(s_k0.p, nleaf, nodes.p, leaf_parent.p);
             LVRHIP_LAUNCH_CHECK();
-            // the refit as range unions, level by level (lbvh.hpp)
+            // the refit as range unions (lbvh.hpp)
             refit_leaf_slots_kernel<<<(unsigned)ceil_div(nleaf, 256), 256, 0, st>>>(nleaf, leaf_parent.p, leaf_lo.p,
                                                                                    leaf_hi.p, nodes.p);
             LVRHIP_LAUNCH_CHECK();
-            const float4* tlo = leaf_lo.p;
-            const float4* thi = leaf_hi.p;
-            for (int j = 1, cur = 0; (1 << j) <= nleaf; j++, cur ^= 1) {
-                const int half = 1 << (j - 1);
-                range_union_level_kernel<<<(unsigned)ceil_div(nleaf - 2 * half + 1, 256), 256, 0, st>>>(
-                    nleaf, half, tlo, thi, ru_lo[cur].p, ru_hi[cur].p);
+            RefitLevels t{};
+            t.lo[0] = leaf_lo.p;
+            t.hi[0] = leaf_hi.p;
+            t.n = 1;
+            size_t at = 0;
+            for (int64_t in = nleaf; in > REFIT_RADIX && t.n < REFIT_LEVELS; t.n++) {
+                const int64_t on = ceil_div(in, (int64_t)REFIT_RADIX);
+                refit_blocks_kernel<<<(unsigned)ceil_div(on, 256), 256, 0, st>>>((int)in, t.lo[t.n - 1], t.hi[t.n - 1],
+                                                                                ru_lo.p + at, ru_hi.p + at);
                 LVRHIP_LAUNCH_CHECK();
-                tlo = ru_lo[cur].p;
-                thi = ru_hi[cur].p;
-                refit_level_kernel<<<(unsigned)ceil_div(nint, 256), 256, 0, st>>>(nint, j, tlo, thi, nodes.p, nlo.p,
-                                                                                 nhi.p);
-                LVRHIP_LAUNCH_CHECK();
+                t.lo[t.n] = ru_lo.p + at;
+                t.hi[t.n] = ru_hi.p + at;
+                at += (size_t)on;
+                in = on;
             }
+            refit_nodes_kernel<<<(unsigned)ceil_div(nint, 256), 256, 0, st>>>(nint, t, nodes.p);
+            LVRHIP_LAUNCH_CHECK();
         }
         if (ns > 1) {
             scan_roots_kernel<<<(unsigned)ceil_div(ns, 256), 256, 0, st>>>(d_pstart.p, ns, leaf_parent.p, nodes.p,
@@ -1163,9 +1202,12 @@ struct lvrhip_surface {
         const int64_t nb = std::max<int64_t>(ceil_div(nq, CF_TILE), 1);
         flag_block_sums_kernel<<<(unsigned)nb, CF_THREADS, 0, st>>>(pred, nq, nq_dev, bsum);
         LVRHIP_LAUNCH_CHECK();
-        scan_exclusive_kernel<<<1, 1024, 0, st>>>(bsum, nb, count_dev);
-        LVRHIP_LAUNCH_CHECK();
-        compact_scatter_kernel<<<(unsigned)nb, CF_THREADS, 0, st>>>(pred, nq, nq_dev, bsum, out);
+        const bool self = nb <= CF_SELF_BLOCKS;
+        if (!self) {
+            scan_exclusive_kernel<<<1, 1024, 0, st>>>(bsum, nb, count_dev);
+            LVRHIP_LAUNCH_CHECK();
+        }
+        compact_scatter_kernel<<<(unsigned)nb, CF_THREADS, 0, st>>>(pred, nq, nq_dev, bsum, self, count_dev, out);
         LVRHIP_LAUNCH_CHECK();
     }
 
@@ -1206,7 +1248,7 @@ struct lvrhip_surface {
 
     // A launch of the adaptive rounds: round 1 for the points of qsel (stage 1; stage 0: flags in s_flags for
     // the merged rounds), or, with seg, the next stage of every point of the partitioned list qsel.
-    void enqueue_round(int stage, const uint32_t* qsel, int64_t nq, const uint32_t* seg)
+    void enqueue_round(int stage, const uint32_t* qsel, int64_t nq, const uint32_t* seg, int queue)
     {
         const bool first = seg == nullptr;
         TileParams prm = params(clamp_k((int64_t)kn << (first ? 1 : 5)), first ? kiw : 0, 0);
@@ -1251,10 +1293,10 @@ struct lvrhip_surface {
         const int tok = prof.start(first ? LVRHIP_T_NORMALS_FIRST : LVRHIP_T_NORMALS_RETRY, st);
         if (prm.t1 > 0)
             tile<SinkNormals>(qv, prm, lanes_per_query, mk(std::integral_constant<int, 2>()),
-                              mk(std::integral_constant<int, 4>()), mk(std::integral_constant<int, 8>()));
+                              mk(std::integral_constant<int, 4>()), mk(std::integral_constant<int, 8>()), 0, queue);
         else
             tile<SinkMoments>(qv, prm, lanes_per_query, mk1(std::integral_constant<int, 2>()),
-                              mk1(std::integral_constant<int, 4>()), mk1(std::integral_constant<int, 8>()));
+                              mk1(std::integral_constant<int, 4>()), mk1(std::integral_constant<int, 8>()), 0, queue);
         prof.stop(tok, st);
     }
 
@@ -1267,19 +1309,25 @@ struct lvrhip_surface {
         nq_first = nq0;
         if (nq0 == 0) return;
         if (merge_retry) {
-            enqueue_round(0, q0, nq0, nullptr);
+            enqueue_round(0, q0, nq0, nullptr, -1);
             plane_fit(q0, nq0, nullptr, s_flags.p, clamp_k((int64_t)kn << 1), 1);
             compact_flags(s_flags.p, nq0, nullptr, q0, s_list1.p, counter(2));
             enqueue_merged_rounds(s_list1.p, counter(2), nq0);
             return;
         }
-        enqueue_round(1, q0, nq0, nullptr);
+        if (use_queue) {  // the launches' work queues at once
+            const int64_t len = (int64_t)QUEUES * QUEUE_SEGS * QUEUE_STRIDE;
+            d_queue.reserve(len);
+            fill_u32_kernel<<<(unsigned)ceil_div(len, 256), 256, 0, st>>>(d_queue.p, len, 0u);
+            LVRHIP_LAUNCH_CHECK();
+        }
+        enqueue_round(1, q0, nq0, nullptr, 0);
         uint32_t* rejected = s_list1.p;
         compact_act(-1, nq0, nullptr, q0, rejected, counter(2));
         // a point's longest way: stages 5, 3, 2, 4 or 3, 2, 15, 4
         for (int pass = 0; pass < 4; pass++) {
             partition_stages(rejected, nq0, pass == 0);
-            enqueue_round(2, s_list0.p, nq0, s_seg.p);
+            enqueue_round(2, s_list0.p, nq0, s_seg.p, 1 + pass);
             if (pass == 0) {
                 spec_resolve_kernel<<<(unsigned)ceil_div(std::max(spec_points(), 1u), 256), 256, 0, st>>>(s_seg.p, s_list0.p, spec_mom.p, spec_ok.p,
                                                                       mom.p, kround.p, act.p);
@@ -1303,10 +1351,13 @@ struct lvrhip_surface {
         const int64_t nb = std::max<int64_t>(ceil_div(nq0, CF_TILE), 1);
         part_sums_kernel<<<(unsigned)nb, CF_THREADS, 0, st>>>(act.p, list, counter(2), spec, first ? nq0 : 0, s_bsum.p);
         LVRHIP_LAUNCH_CHECK();
-        scan_exclusive_kernel<<<1, 1024, 0, st>>>(s_bsum.p, ROUND_SEGS * nb, counter(6));
-        LVRHIP_LAUNCH_CHECK();
+        const bool self = nb <= CF_SELF_BLOCKS;
+        if (!self) {
+            scan_exclusive_kernel<<<1, 1024, 0, st>>>(s_bsum.p, ROUND_SEGS * nb, counter(6));
+            LVRHIP_LAUNCH_CHECK();
+        }
         part_scatter_kernel<<<(unsigned)nb, CF_THREADS, 0, st>>>(act.p, list, counter(2), spec, first ? nq0 : 0, s_bsum.p,
-                                                                counter(6), s_list0.p, s_seg.p);
+                                                                self, counter(6), s_list0.p, s_seg.p);
         LVRHIP_LAUNCH_CHECK();
     }
 
@@ -1705,8 +1756,11 @@ struct lvrhip_surface {
         if (outM) *outM = bm;
     }
 
-    // Morton-sort m device queries; fills s_qx/s_qy/s_qz and s_v0 (sorted -> caller index).
-    void sort_queries(const float* d_q, int64_t m)
+    // Morton-sort m device queries; fills s_qx/s_qy/s_qz and s_v0 (sorted -> caller index).  lanes: for the
+    // best-first lane search, which needs neighbouring queries in a wave (and an L2) but no more: about as many
+    // cells as queries, and none when every query has a wave of its own.  The tile kernel's tiles cover
+    // several queries with one box: 32 bits.
+    void sort_queries(const float* d_q, int64_t m, bool lanes = false)
     {
         s_k0.reserve(std::max<int64_t>(m, 1));
         s_k1.reserve(std::max<int64_t>(m, 1));
@@ -1714,11 +1768,12 @@ struct lvrhip_surface {
         s_v1.reserve(std::max<int64_t>(m, 1));
         s_hist.reserve(rs_hist_size(m));
         const unsigned gb = (unsigned)ceil_div(m, 256);
-        morton_queries_kernel<<<gb, 256, 0, st>>>(d_q, m, frames.p, s_k0.p, s_v0.p);
+        // of the 63-bit code (its top 32 bits are cells of 1/1,600 of the box per axis)
+        const int bits = !lanes ? 32 : bf_per_wave(m, bf_resident) == 1 ? 0 : m <= (1 << 16) ? 16 : m <= (1 << 21) ? 24 : 32;
+        const bool odd = rs_passes(bits) & 1;  // the sort then starts from its other buffers
+        morton_queries_kernel<<<gb, 256, 0, st>>>(d_q, m, frames.p, odd ? s_k1.p : s_k0.p, odd ? s_v1.p : s_v0.p);
         LVRHIP_LAUNCH_CHECK();
-        // the top 32 bits of the 63-bit code (cells of 1/1,600 of the box per axis) order the
-        // queries well enough for the searches' locality in half the passes
-        radix_sort_pairs(s_k0.p, s_v0.p, s_k1.p, s_v1.p, m, s_hist.p, st, 64, 32);
+        if (bits) radix_sort_pairs(s_k0.p, s_v0.p, s_k1.p, s_v1.p, m, s_hist.p, st, 64, 64 - bits);
         s_qx.reserve(m);
         s_qy.reserve(m);
         s_qz.reserve(m);
@@ -1743,9 +1798,9 @@ struct lvrhip_surface {
         s_spos.reserve((size_t)m * t0);
         s_ord.reserve((size_t)m * t0);
         const int tsort = prof.start(LVRHIP_T_SDF_SORT, st);
-        sort_queries(d_q, m);
-        prof.stop(tsort, st);
         const bool bf = best_first(t0);
+        sort_queries(d_q, m, bf);
+        prof.stop(tsort, st);
         const uint32_t* qsel = nullptr;
         const uint32_t* nq_dev = nullptr;
         if (bf) {
@@ -2142,7 +2197,7 @@ struct lvrhip_surface {
         LVRHIP_LAUNCH_CHECK();
         zero_f32_kernel<<<(unsigned)ceil_div(3 * R, 256), 256, 0, st>>>(g_n.p, 3 * R);
         LVRHIP_LAUNCH_CHECK();
-        sort_queries(d_q, m);
+        sort_queries(d_q, m, best_first(t0));
         // 1. SDF reverse: dL/dp (through the means) and dL/dn of every vertex's kd neighbours, best-first like
         // the forward (3.8 -> 1.24 ms for 500,000 vertices of the 1M-point cloud); the tile kernel does the
         // vertices that left
@@ -2233,7 +2288,7 @@ struct lvrhip_surface {
     {
         s_left1.reserve(m);
         s_left2.reserve(m);
-        d_queue.reserve(QUEUE_SEGS * QUEUE_STRIDE);
+        d_queue.reserve((size_t)QUEUES * QUEUE_SEGS * QUEUE_STRIDE);
         bf_reset_kernel<<<1, 256, 0, st>>>(d_queue.p, QUEUE_SEGS * QUEUE_STRIDE, counter(13), counter(8));
         LVRHIP_LAUNCH_CHECK();
         const bool lanes = search_mode != LVRHIP_SEARCH_WAVE;
@@ -2274,14 +2329,16 @@ struct lvrhip_surface {
             LVRHIP_CHECK(hipStreamSynchronize(st));
             return;
         }
-        sort_queries(d_q, m);
-        if (best_first(t0)) {
+        const bool bf = best_first(t0);
+        sort_queries(d_q, m, bf);
+        if (bf) {
             const uint64_t empty = r2 >= 0.0f ? ((uint64_t)host_fbits(r2) << 32) : BF_EMPTY;
             BfRowsOut o{s_v0.p, k, d_idx, d_d2, d_count};
             enqueue_bf(m, t0, empty, o, 7);
             if (bf_left() == 0) return;
         }
-        // the tile kernel for every query (also when a best-first stack overflowed)
+        // the tile kernel for every query (also when a best-first search left some)
+        if (bf) sort_queries(d_q, m);
         DBuf<uint64_t> keys;
         keys.reserve((size_t)m * k);
         DBuf<float> d2tmp;
@@ -2323,7 +2380,7 @@ struct lvrhip_surface {
         if (n == 0) throw Error(LVRHIP_ESTATE, "the mesh needs a non-empty point cloud");
         const int t0 = clamp_k(kc);
         if (best_first(t0)) {
-            sort_queries(d_q, m);
+            sort_queries(d_q, m, true);
             BfCentroidOut o{pts4.p, s_v0.p, d_out, vid, nbr, prefill, (uint32_t)npad};
             enqueue_bf(m, t0, BF_EMPTY, o, 7);
             if (bf_left() == 0) return;
@@ -2355,7 +2412,7 @@ struct lvrhip_surface {
         drop_graph();
         const int t0 = clamp_k(ki);
         if (best_first(t0)) {
-            sort_queries(d_q, m);
+            sort_queries(d_q, m, true);
             BfMeanNormalOut o{nx.p, ny.p, nz.p, s_v0.p, ki, d_out};
             enqueue_bf(m, t0, BF_EMPTY, o, 7);
             if (bf_left() == 0) return;
