@@ -100,52 +100,93 @@ static __global__ void box_init_kernel(uint32_t* __restrict__ box, int ns)
     if (i < 6 * ns) box[i] = (i % 6) < 3 ? 0xFFFFFFFFu : 0u;
 }
 
-constexpr int SB_ITEMS = 16;  // points per lane
+// Points per block of scan_bbox_kernel: at least SB_MIN, and at most SB_BLOCKS blocks.
+constexpr int SB_MIN = 4096;
+constexpr int SB_BLOCKS = 1024;
+static inline int64_t sb_chunk(int64_t n)
+{
+    const int64_t c = (n + SB_BLOCKS - 1) / SB_BLOCKS;
+    return c > SB_MIN ? (c + 255) / 256 * 256 : SB_MIN;
+}
 
-// One wave per 64 * SB_ITEMS consecutive input points: reduced in registers and merged with one
-// atomic per coordinate when they belong to one scan, per point otherwise.
-static __global__ __launch_bounds__(256) void scan_bbox_kernel(const float* __restrict__ xyz, int64_t n,
+// Each wave's values to one atomic per coordinate of its scan's box.
+__device__ __forceinline__ void box_merge(uint32_t* __restrict__ b, const float mn[3], const float mx[3], int lane)
+{
+    if (lane < 3) {
+        atomicMin(&b[lane], ord_enc(lane == 0 ? mn[0] : lane == 1 ? mn[1] : mn[2]));
+        atomicMax(&b[3 + lane], ord_enc(lane == 0 ? mx[0] : lane == 1 ? mx[1] : mx[2]));
+    }
+}
+
+// One block per `chunk` consecutive input points.  Atomics on one box are served one after the
+// other, so their number is what this pass would wait for: a chunk of one scan is reduced over
+// the block (6 atomics), one that several scans meet in per row of 64 points; only a row that
+// scans meet in goes point by point.  (One merge per 1,024 points and single points in every
+// straddling 1,024 took 344 us for 12 scans and 100 us for 4M points of one scan.)
+static __global__ __launch_bounds__(256) void scan_bbox_kernel(const float* __restrict__ xyz, int64_t n, int64_t chunk,
                                                         const int64_t* __restrict__ off, int ns,
                                                         uint32_t* __restrict__ box)
 {
+    __shared__ float red[4][6];
     const int lane = lane_id();
-    const int64_t w0 = (((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / kWave) * (kWave * SB_ITEMS);
+    const int wave = (int)(threadIdx.x / kWave);
+    const int64_t w0 = (int64_t)blockIdx.x * chunk;
     if (w0 >= n) return;
-    const int64_t w1 = w0 + kWave * SB_ITEMS < n ? w0 + kWave * SB_ITEMS : n;
+    const int64_t w1 = w0 + chunk < n ? w0 + chunk : n;
     const int s0 = scan_of_pos(off, ns, w0), s1 = scan_of_pos(off, ns, w1 - 1);
     if (s0 == s1) {
         float mn[3] = {INFINITY, INFINITY, INFINITY}, mx[3] = {-INFINITY, -INFINITY, -INFINITY};
-        for (int it = 0; it < SB_ITEMS; it++) {
-            const int64_t i = w0 + (int64_t)it * kWave + lane;
-            if (i < w1) {
+#pragma unroll 4
+        for (int64_t i = w0 + threadIdx.x; i < w1; i += 256) {
 #pragma unroll
-                for (int j = 0; j < 3; j++) {
-                    const float v = xyz[3 * i + j];
-                    mn[j] = fminf(mn[j], v);
-                    mx[j] = fmaxf(mx[j], v);
-                }
+            for (int j = 0; j < 3; j++) {
+                const float v = xyz[3 * i + j];
+                mn[j] = fminf(mn[j], v);
+                mx[j] = fmaxf(mx[j], v);
             }
         }
 #pragma unroll
         for (int j = 0; j < 3; j++) {
             mn[j] = wave_min(mn[j]);
             mx[j] = wave_max(mx[j]);
+            if (lane == 0) {
+                red[wave][j] = mn[j];
+                red[wave][3 + j] = mx[j];
+            }
         }
-        if (lane < 3) {
-            atomicMin(&box[6 * s0 + lane], ord_enc(lane == 0 ? mn[0] : lane == 1 ? mn[1] : mn[2]));
-            atomicMax(&box[6 * s0 + 3 + lane], ord_enc(lane == 0 ? mx[0] : lane == 1 ? mx[1] : mx[2]));
+        __syncthreads();
+        if (wave == 0) {
+#pragma unroll
+            for (int j = 0; j < 3; j++) {
+                mn[j] = fminf(fminf(red[0][j], red[1][j]), fminf(red[2][j], red[3][j]));
+                mx[j] = fmaxf(fmaxf(red[0][3 + j], red[1][3 + j]), fmaxf(red[2][3 + j], red[3][3 + j]));
+            }
+            box_merge(box + 6 * s0, mn, mx, lane);
         }
     } else {
-        for (int it = 0; it < SB_ITEMS; it++) {
-            const int64_t i = w0 + (int64_t)it * kWave + lane;
-            if (i < w1) {
-                const int sc = scan_of_pos(off, ns, i);
+        for (int64_t r0 = w0 + wave * kWave; r0 < w1; r0 += 256) {
+            const int64_t last = (r0 + kWave < w1 ? r0 + kWave : w1) - 1;
+            const int64_t i = r0 + lane;
+            float v[3] = {__builtin_nanf(""), __builtin_nanf(""), __builtin_nanf("")};
+            if (i <= last) {
+#pragma unroll
+                for (int j = 0; j < 3; j++) v[j] = xyz[3 * i + j];
+            }
+            const int sc = scan_of_pos(off, ns, i <= last ? i : last);
+            if (uniform(sc) == __builtin_amdgcn_readlane(sc, kWave - 1)) {
+                float mn[3], mx[3];
 #pragma unroll
                 for (int j = 0; j < 3; j++) {
-                    const float v = xyz[3 * i + j];
-                    if (v == v) {
-                        atomicMin(&box[6 * sc + j], ord_enc(v));
-                        atomicMax(&box[6 * sc + 3 + j], ord_enc(v));
+                    mn[j] = wave_min(fminf(INFINITY, v[j]));
+                    mx[j] = wave_max(fmaxf(-INFINITY, v[j]));
+                }
+                box_merge(box + 6 * uniform(sc), mn, mx, lane);
+            } else {
+#pragma unroll
+                for (int j = 0; j < 3; j++) {
+                    if (v[j] == v[j]) {
+                        atomicMin(&box[6 * sc + j], ord_enc(v[j]));
+                        atomicMax(&box[6 * sc + 3 + j], ord_enc(v[j]));
                     }
                 }
             }

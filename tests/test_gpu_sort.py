@@ -50,3 +50,29 @@ def test_lattice_offsets(oracle_mod, shift, voxel):
     np.testing.assert_array_equal(ci, oci)
     np.testing.assert_array_equal(c, oc)
     np.testing.assert_array_equal(v, ov)
+
+
+@pytest.mark.parametrize("sizes", [[4_096, 65, 64, 4_095, 9_000], [64] * 70 + [5_000], [4_200_000, 70, 300_000],
+                                   [66, 4_300_000]])
+def test_scan_boxes(oracle_mod, sizes):
+    """Scan bounds inside, at the ends of and across the blocks and rows the scan boxes are reduced in."""
+    from lvr2_amd import HipSurface, scenes
+
+    p = scenes.plane_boxes_sphere(7, sum(sizes), 0.5)
+    s = HipSurface(p, scan_sizes=sizes)
+    s.setKn(2)
+    s.setKi(0)
+    s.calculateNormals()
+    k = s.adaptiveK()
+    off = np.concatenate([[0], np.cumsum(sizes)])
+    for i in {0, 1, len(sizes) - 2, len(sizes) - 1}:
+        a = p[off[i]:off[i + 1]]
+        if len(a) <= 10_000:
+            want = oracle_mod.Surface(a).normals(2, 3, (1e6, 1e6, 1e6))[2]
+        else:
+            one = HipSurface(a)
+            one.setKn(2)
+            one.setKi(0)
+            one.calculateNormals()
+            want = one.adaptiveK()
+        np.testing.assert_array_equal(k[off[i]:off[i + 1]], want)
