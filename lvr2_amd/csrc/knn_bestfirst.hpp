@@ -19,7 +19,7 @@
 // 4M-point room (t = 10) that scanned 21 leaves and expanded about 50 nodes per query; taking the nearest
 // pool entry after every leaf scans 8.6 and expands 37 (a strict best-first queue: 7.7 and 25, but it
 // holds four times the entries).  Signed distances at 700,000 vertices of that lattice, sort included:
-// 5.17 -> 1.19 ms.
+// 5.17 -> 1.19 ms (1.00 with the rest of the call's launches).
 // The few queries whose lane stack overflows (hundreds of leaves within their bound) are searched
 // again by a whole wave each (bf_knn_wave_kernel), and the tile kernel takes any that outgrow
 // that stack too.
@@ -205,6 +205,7 @@ struct BfLane {
     int nspill;
     uint2* spill;  // this lane's spilled entries (ref, d), interleaved with the wave's other lanes
     int spill_cap;
+    int lanes;  // of the wave that search, and have a spill area
 };
 
 // Puts an entry into the pool; false if neither the LDS slots nor the spill area hold it.
@@ -222,7 +223,7 @@ __device__ __forceinline__ bool bf_put(BfPool& pool, BfLane& ln, int lane, uint3
     }
     if (ln.free == 0u) {
         if (ln.nspill == ln.spill_cap) return false;
-        ln.spill[(size_t)ln.nspill * BF_THREADS] = make_uint2(ref, d16);
+        ln.spill[(size_t)ln.nspill * ln.lanes] = make_uint2(ref, d16);
         ln.nspill++;
         return true;
     }
@@ -260,7 +261,7 @@ __device__ __forceinline__ bool bf_take(BfPool& pool, BfLane& ln, int lane, floa
         ln.free = (1u << BF_POOL) - 1u;
         while (ln.nspill > 0 && ln.free != 0u) {
             ln.nspill--;
-            const uint2 e = ln.spill[(size_t)ln.nspill * BF_THREADS];
+            const uint2 e = ln.spill[(size_t)ln.nspill * ln.lanes];
             const int slot = __ffs((int)ln.free) - 1;
             ln.free &= ln.free - 1u;
             pool.ref[slot][lane] = e.x;
@@ -395,7 +396,8 @@ __device__ __forceinline__ void bf_stats(unsigned long long* stats, bool valid, 
 // of a cloud are spread over all XCDs.  Without a queue, wave b takes chunk b.
 //
 // Query i is (qx[i qs], qy[i qs], qz[i qs]): qs = 1 for SoA coordinates, 3 for an AoS buffer
-// (qy = qx + 1, qz = qx + 2).  spill: spill_cap entries per lane for each wave of the grid.
+// (qy = qx + 1, qz = qx + 2).  spill: spill_cap entries for each of the per_wave lanes of each wave of the
+// grid (all 64 lanes' would be 20 KB per wave, 64 times what a batch of one query per wave can use).
 template <int K, class Out>
 __global__ __launch_bounds__(BF_THREADS) void bf_knn_kernel(const BvhView bv, const float* __restrict__ qx,
                                                             const float* __restrict__ qy,
@@ -430,7 +432,7 @@ __global__ __launch_bounds__(BF_THREADS) void bf_knn_kernel(const BvhView bv, co
             if constexpr (bf_prefills<Out>::value) start = out.first_bound(i, t, x, y, z, empty);
             BfList<K> L;
             L.init(t, start);
-            BfLane ln{0u, 0, spill + (size_t)blockIdx.x * spill_cap * BF_THREADS + lane, spill_cap};
+            BfLane ln{0u, 0, spill + (size_t)blockIdx.x * spill_cap * per_wave + lane, spill_cap, per_wave};
             ok = bf_search<K>(bv, pool, ln, lane, x, y, z, L, leaves, nodes);
             L.finish(bv.rank, t);
             // the queries left go to the next pass, in any order: each result is its query's own

@@ -645,7 +645,7 @@ __global__ void centroid_rows_kernel(int64_t m, int k, const int32_t* __restrict
 // Best-first kNN launch for t <= BF_KMAX: the list length is the smallest of 8, 10, 16, 32 that
 // holds t (10: the signed distance's usual kd).
 // Query coordinates: SoA (qs = 1) or AoS (qs = 3, qy = qx + 1, qz = qx + 2).  With a queue the
-// grid is min(chunks, resident) waves; spill holds spill_cap entries per lane for each of them.
+// grid is min(chunks, resident) waves; spill holds spill_cap entries per searching lane of each of them.
 // Queries per wave: 64 fills the lanes, but a small batch runs on more waves with fewer lanes each, which
 // wait less for each other: 500 queries (t = 10) take 100 us, by the wave search, which took them before,
 // 137 us, and at t = 32 a quarter of its time.
@@ -2309,10 +2309,10 @@ struct lvrhip_surface {
         const bool lanes = search_mode != LVRHIP_SEARCH_WAVE;
         if (lanes) {
             uint32_t* q = use_queue ? d_queue.p : nullptr;
-            // one spill area per wave of the grid
-            const int64_t all = ceil_div(m, (int64_t)bf_per_wave(m, bf_resident));
+            // one spill area per searching lane of the grid
+            const int64_t pw = bf_per_wave(m, bf_resident), all = ceil_div(m, pw);
             const int64_t waves = q ? std::min(all, bf_resident) : all;
-            s_spill.reserve((size_t)waves * BF_SPILL * BF_THREADS);
+            s_spill.reserve((size_t)(waves * pw) * BF_SPILL);
             launch_bf(view(), s_qx.p, s_qy.p, s_qz.p, 1, m, t0, empty, o, st, kstats_ptr(stats_group), q, bf_resident,
                       s_spill.p, BF_SPILL, s_left1.p, counter(13));
         }
