@@ -69,3 +69,20 @@ def test_adaptive_k_of_scans(oracle_mod):
     s.calculateNormals()
     want = np.concatenate([oracle_mod.Surface(w.points).normals(10, 3, (1e6, 1e6, 1e6))[2] for w in (a, b)])
     np.testing.assert_array_equal(s.adaptiveK(), want)
+
+
+@pytest.mark.parametrize("lone", [1, 7, 44, 101])
+def test_lone_patches_beside_a_dense_one(oracle_mod, lone):
+    """Patches of fewer points than k, whose searches reach a dense patch just as their radius does."""
+    from lvr2_amd import HipSurface
+
+    rng = np.random.default_rng(lone)
+    flat = np.array([1.0, 1.0, 0.02])
+    dense = rng.uniform(-2, 2, (12_000, 3)) * flat
+    far = [rng.uniform(-0.1, 0.1, (lone, 3)) * flat + np.array([d, 0.3 * d, 0.0]) for d in (6.0, -33.0, 80.0)]
+    p = np.concatenate([dense] + far).astype(np.float32)
+    s = HipSurface(p)
+    s.setKn(50)
+    s.setKi(20)
+    s.calculateNormals()
+    np.testing.assert_array_equal(s.adaptiveK(), oracle_mod.Surface(p).normals(50, 3, (1e6, 1e6, 1e6))[2])
