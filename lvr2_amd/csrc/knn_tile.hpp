@@ -110,9 +110,12 @@ struct TileParams {
                                 // zeroed before the launch): waves take the next run of
                                 // tiles_per_wave tiles from it; else runs are strided over the grid
     bool queue_zeroed;          // (host) the caller has zeroed it
-    float hint_scale;           // with hints (hint1, hint3): a cluster's first radius^2 over its hints grown to t0
+    const float* hint_in;       // optional, per query position: the d^2 of its t-th key for an earlier
+                                // target t; a tile's first radius^2 is hint_scale times the largest
+                                // over its queries (else the radius carried from the previous tile)
+    float hint_scale;
     float* hint_out;            // optional, per query position: the d^2 of the t0-th key of every
-                                // query resolved
+                                // query resolved (may be hint_in: a query reads it before)
     // Several searches in one launch (one-target sinks): the query list is cut into the segments of
     // ROUND_SEGS, seg[i] .. seg[i + 1] (device), each with its own target, hints and stage;
     // seg[ROUND_SEGS + 1] != 0: every segment but the second holds all the points.
@@ -790,7 +793,7 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(tile_thre
     }
     // the search of the current tile (of its segment)
     int t0 = prm.t0;
-    const float* hint_in = nullptr;  // per query position: the d^2 of its t-th key for an earlier target t
+    const float* hint_in = prm.hint_in;
     float* hint_out = prm.hint_out;
     float hint_scale = prm.hint_scale;
 
@@ -930,7 +933,6 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(tile_thre
         int prev_lead = -1;
         int cl_att = 0;  // attempts of the current cluster
         bool in_cluster = true, in_hint = false;  // the latter: in_cluster by its hint
-        bool joined = true;                       // near the lead in the cluster's last attempt
 
         for (int attempt = 0; attempt < MAX_ATTEMPTS; attempt++) {
             const uint64_t pending = ballot(active);
@@ -968,14 +970,7 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(tile_thre
                 }
             }
             const float reach = sqrtf(r2);
-            // A query that the cluster's smaller radii left out joins only at twice its distance: a lone
-            // patch reaches a dense one just when its radius does, and queries of the dense one drawn
-            // in then would scan it, all of it within the lone patch's radius (one such tile of
-            // 483,235 points of an outdoor scan took 11 ms, all others together 0.9 ms).
-            if (cl_att == 1) joined = true;
-            const float gap = fmaxf(fmaxf(fabsf(qx - lx), fabsf(qy - ly)), fabsf(qz - lz));
-            const bool near = gap <= (joined ? reach : 0.5f * reach);
-            joined = near;
+            const bool near = fabsf(qx - lx) <= reach && fabsf(qy - ly) <= reach && fabsf(qz - lz) <= reach;
             const bool act = active && scan == cur && near && in_cluster;
             // tile box of the pending queries of that scan
             TileBox tb;
@@ -1315,12 +1310,9 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(tile_thre
                 if (cl_att > CLUSTER_GUARD) nr2 = R2 * 4.0f;  // a guard: plain doubling of R
                 if (!(nr2 > R2) || nr2 < 1e-30f) nr2 = fmaxf(R2 * 4.0f, 1e-30f);
                 if (nr2 > 1e37f) nr2 = INFINITY;
-                // Below a radius already found too wide while shrinking may go on, and to that radius,
-                // not past it, once it is over (an estimate from the few points of a lone patch goes
-                // far into the dense one that was too wide).
-                if (nr2 > r2_ceil && R2 < r2_ceil && cl_att <= CLUSTER_GUARD)
-                    nr2 = (shrinks < MAX_SHRINKS && cl_att <= CLUSTER_SHRINK) ? fmaxf(R2 + (r2_ceil - R2) * 0.5f, R2 * 1.01f)
-                                                                          : r2_ceil;
+                // below a radius already found too wide, unless shrinking is over
+                if (shrinks < MAX_SHRINKS && nr2 > r2_ceil && cl_att <= CLUSTER_SHRINK)
+                    nr2 = fmaxf(R2 + (r2_ceil - R2) * 0.5f, R2 * 1.01f);
                 r2_floor = R2;
                 r2 = nr2;
             }
