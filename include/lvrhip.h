@@ -319,8 +319,9 @@ int lvrhip_get_kernel_stats(lvrhip_t h, int64_t out[128], int reset);
 /* Launch shape of the kNN tile kernels (no lvr2 counterpart): lanes per query (2, 4 or 8;
  * queries per wavefront = 64 / lanes), consecutive tiles per wavefront in the first adaptive
  * round (default 12; the later rounds take one), and the margin of the radius^2 carried from one
- * tile to the next, as it holds for searches of 120 points (default 1.15; its excess over 1 grows up to
- * fourfold for smaller counts and falls for larger ones).  Values <= 0 keep the current setting. */
+ * tile to the next (default 1.15).  They decide the order in which a neighbourhood's moments are added
+ * up, so other settings move the last bits of the normals, and the sign of those whose plane runs
+ * through the flip point (n . (f - q) = 0 up to rounding).  Values <= 0 keep the current setting. */
 int lvrhip_set_tuning(lvrhip_t h, int lanes_per_query, int tiles_per_wave, float r2_margin);
 /* ms[i], launches[i] for i < LVRHIP_T_COUNT; either may be NULL.  reset != 0 clears them. */
 int lvrhip_get_timings(lvrhip_t h, double* ms, int64_t* launches, int reset);

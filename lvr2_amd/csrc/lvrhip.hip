@@ -953,21 +953,6 @@ struct lvrhip_surface {
         return v;
     }
 
-    // The margin of the radius^2 carried from tile to tile in a search for t points.  A tile's
-    // radius has to hold t points of each of its queries; how far their counts scatter falls with
-    // t, and so does what a radius too wide costs against one too narrow, which searches the
-    // tile a second time.  First rounds in ms at margins 1.08 / 1.15 / 1.3 / 1.5 / 1.7:
-    //   t = 20 (2M points)      3.78 / 3.56 / 3.33 / 3.19 / 3.13
-    //   t = 40 (1M, room)       2.47 / 2.42 / 2.35 / 2.30 / 2.30
-    //   t = 60 (1M, torus)      2.23 / 2.12 / 1.99 / 1.96 / 1.96
-    //   t = 100 (1M, room)      2.67 / 2.65 / 2.69 / 2.70 / 2.72
-    //   t = 200 (4M, outdoor)   9.68 / 9.97 / 10.2 / 10.5 / 10.9
-    // `m` (1.15, or as tuned) is the margin at t = 120; its excess goes with 1/t, up to fourfold.
-    static float count_margin(float m, int t)
-    {
-        return 1.0f + (m - 1.0f) * std::min(4.0f, 120.0f / (float)std::max(t, 1));
-    }
-
     TileParams params(int t0, int t1, int stats_group) const
     {
         TileParams prm{};
@@ -976,7 +961,7 @@ struct lvrhip_surface {
         prm.tiles_per_wave = tiles_per_wave;
         prm.r2_init = 0.0f;
         prm.area_pp = area.p;
-        prm.r2_margin = count_margin(r2_margin, t0);
+        prm.r2_margin = r2_margin;
         prm.grow_min = 1.01f;
         prm.err = (int*)counter(CNT_ERR);
         prm.stats = nullptr;
