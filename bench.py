@@ -426,12 +426,16 @@ def main():
     ms_step = sum(e[0].elapsed_time(e[3]) for e in evs) / args.steps
     tm = s.timings()
     kss = s.kernelStats()
-    ks = kss["sdf"]
+    ks, kw = kss["sdf"], kss["merged_rounds"]
     if ks["tiles"]:
         log(f"[bench] SDF search: {ks['resolved'] / args.steps:.0f} vertices one lane each, "
             f"{ks['refine'] / args.steps:.0f} left to the wave pass; per vertex {ks['candidates'] / max(ks['resolved'], 1):.1f} "
             f"points scanned, {ks['pops'] / max(ks['resolved'], 1):.1f} nodes expanded; slowest lane per wave "
             f"{16 * ks['attempts'] / ks['tiles']:.1f} points; {ks['cy_total'] / ks['tiles']:.0f} cycles per wave")
+    if kw["tiles"]:
+        log(f"[bench] SDF wave pass: {kw['resolved'] / args.steps:.0f} vertices, {kw['refine'] / args.steps:.0f} left "
+            f"to the tile kernel; per vertex {kw['candidates'] / kw['tiles']:.0f} points, {kw['pops'] / kw['tiles']:.0f} "
+            f"nodes, {kw['cy_total'] / kw['tiles']:.0f} cycles")
     rounds = s.normalsStats()
     mpts = n / ((t_norm + t_int) / 1e3) / 1e6
     sdf_mqps = m / (t_sdf / 1e3) / 1e6
@@ -451,11 +455,9 @@ def main():
     log(f"[bench] mesh: PMC {mesh['PMC']['ms']:.2f} ms, MC {mesh['MC']['ms']:.2f} ms, {mesh['MC']['faces']} faces")
 
     # roofline of the dominant kernel: the kNN tile kernel of the normals (fused bounding-box
-    # test + moments), over its five launches (round 1 and four that share the later rounds).
-    # Algorithmic bytes of a step: per point of each adaptive round 12 (point) + 12 k (neighbours)
-    # + 12 (normal) + 4 ki (ki list, first round only), the per-unit figure of the fused kNN + PCA
-    # step.  The rounds are the reference's; those whose rejection a larger search proves
-    # are not searched here, which the time shows and the bytes do not.
+    # test + moments), over its five adaptive-round launches.  Algorithmic bytes of a launch at
+    # k: per query point 12 (point) + 12 k (neighbours) + 12 (normal) + 4 ki (ki list, first
+    # round only), the per-unit figure of the fused kNN + PCA step.
     lanes = s.tuning()["lanes_per_query"]
     ms_first, n_first = tm["normals_first"]
     ms_retry, n_retry = tm["normals_retry"]
@@ -472,7 +474,7 @@ def main():
         "bound": "hbm",
         "limiter": "instruction issue and LDS / L2 latency (the kernel is occupancy-bound: three waves per SIMD, "
                    "set by LDS and registers); measured HBM traffic is a small fraction of the algorithmic bytes",
-        "kernel": f"knn_tile_kernel<{lanes}, SinkNormals<{lanes}> | SinkMoments<{lanes}>> (round 1 and the four launches of the later rounds)",
+        "kernel": f"knn_tile_kernel<{lanes}, SinkNormals<{lanes}> | SinkMoments<{lanes}>> (the five adaptive-round launches)",
         "achieved": round(achieved, 1),
         "peak": HBM_PEAK_GBS,
         "unit": "GB/s",

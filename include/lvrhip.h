@@ -306,10 +306,9 @@ enum {
 int lvrhip_set_profiling(lvrhip_t h, int on);
 
 /* Kernel work counters collected while profiling is on (no lvr2 counterpart):
- * out[g * 16 + c] for group g (0 the normals' first adaptive round, 5 the later rounds, which
- * share launches, and the wave-per-query pass of the signed distances, 1..3 what a merged search
- * (lvrhip_set_retry_mode) searches again for the points that stop at rounds 2..4, 6 SDF, 7 other
- * searches: kSearch, the ki list, the adjoint) and counter c (0 tiles,
+ * out[g * 16 + c] for group g (0..4 the normals' adaptive rounds 1..5, 5 the merged later
+ * rounds and the wave-per-query pass of the signed distances, 6 SDF, 7 other searches:
+ * kSearch, the ki list, the adjoint) and counter c (0 tiles,
  * 1 radius attempts, 2 LDS-resident attempts, 3 candidate points scanned in the histogram
  * pass, 4 refinement passes, 5 chunk loads, 6 queries resolved, 7 traversal node pops;
  * 8..15 shader-clock cycles summed over waves in: traversal, chunk staging, per-query leaf
@@ -342,9 +341,8 @@ int lvrhip_set_sdf_tuning(lvrhip_t h, int tiles_per_wave, float r2_margin);
  * counterpart; the results are the same either way): merged != 0 searches k = 32 kn once with
  * the four round sizes as targets, takes the first round whose neighbourhood passes
  * boundingBoxOK and searches the points that stop before round 5 again at their round's k;
- * merged == 0 (the default) searches each remaining point at the rounds still open for it, a later
- * round before an earlier one where its box proves that the earlier one fails too; the rounds share
- * launches.  lvrhip_autotune also chooses this. */
+ * merged == 0 (the default) searches round by round, each round only for the points the
+ * previous one rejected.  lvrhip_autotune also chooses this. */
 int lvrhip_set_retry_mode(lvrhip_t h, int merged);
 int lvrhip_get_retry_mode(lvrhip_t h, int* merged);
 

@@ -56,12 +56,10 @@ static_assert(CHUNK_LEAVES % (kWave / LEAF) == 0 && CHUNK_LEAVES <= kWave, "a ch
 constexpr int MAX_ATTEMPTS = 1024;    // per tile (a safety net: each cluster of queries grows x4 per
                                       // attempt after CLUSTER_GUARD of its own)
 constexpr int CLUSTER_SHRINK = 12;    // a cluster's first attempts that may shrink R or cap its growth
-constexpr int MAX_SHRINKS = 4;         // how often they may shrink it
 constexpr int CLUSTER_GUARD = 24;
 constexpr int QUEUE_SEGS = 8;     // work-queue segments: one per XCD
 constexpr int QUEUE_STRIDE = 16;  // their counters 64 bytes apart
 constexpr int QUEUE_CHUNK = 32;   // consecutive runs dealt to one segment at a time
-constexpr float HINT_LO = 0.5f;  // first histogram edge over a query's hinted radius^2
 constexpr float RUN_R2_MARGIN = 2.0f;  // radius^2 of a run's leaf list over its second tile's first
 
 struct BvhView {
@@ -116,14 +114,6 @@ struct TileParams {
     float hint_scale;
     float* hint_out;            // optional, per query position: the d^2 of the t0-th key of every
                                 // query resolved (may be hint_in: a query reads it before)
-    // Several searches in one launch (one-target sinks): the query list is cut into the segments of
-    // ROUND_SEGS, seg[i] .. seg[i + 1] (device), each with its own target, hints and stage;
-    // seg[ROUND_SEGS + 1] != 0: every segment but the second holds all the points.
-    const uint32_t* seg;
-    int kn;
-    int64_t kmax;
-    const float* hint1;  // per query position: the k-th d^2 of adaptive rounds 1 and 3
-    float* hint3;
     int leaf_hint;              // the queries are the cloud's own sorted points (query position =
                                 // sorted position): a run's first tile sizes its radius from the
                                 // boxes of its queries' leaves instead of the cloud's mean density
@@ -199,18 +189,6 @@ struct TileSmem {
     uint32_t bcnt[NT][Q];
     uint32_t scnt[NT][Q];  // per-query sink slot counters
 };
-
-// The segments of the later adaptive rounds' launches: stages (RoundState, sinks.hpp) by falling cost, so that
-// the long searches start first and the short ones fill the tail of the launch.  (A launch per stage had
-// left the device waiting for the slowest tile of each: its eight queries, scattered over a sparse list, can
-// take 0.9 ms; the five launches of 500,000 outdoor points took 5.3 ms for 4.6 ms of work.)
-constexpr int ROUND_SEGS = 5;
-__device__ __forceinline__ int seg_stage(int seg)
-{
-    return seg == 0 ? 5 : seg == 1 ? 15 : seg == 2 ? 4 : seg == 3 ? 3 : 2;
-}
-constexpr int STAGE_SPEC = 100;  // one of all rounds searched at once
-__device__ __forceinline__ int stage_round(int stage) { return stage == 15 ? 5 : stage; }
 
 // ---- work queue ---------------------------------------------------------------------------
 
@@ -463,12 +441,10 @@ __device__ __forceinline__ uint32_t slot_spos(const Sm& sm, int base, int c)
 // (replicated over the group's lanes).  rq < 0 disables the query.
 // With rin >= 0, leaves whose farthest corner is closer than sqrt(rin) are left out too:
 // every point of such a leaf has d^2 < rin (the fp32 corner distance bounds the fp32 point
-// distance from above, all roundings being monotone); *skipped is raised by their points (on the lane
-// that tested the leaf).
+// distance from above, all roundings being monotone).
 template <int P, class Sm>
 __device__ __forceinline__ int build_glist(Sm& sm, const BvhView& bv, int base, int nl, int g, int s, float qx,
-                                           float qy, float qz, float rq, float rin = -1.0f,
-                                           uint32_t* skipped = nullptr)
+                                           float qy, float qz, float rq, float rin = -1.0f)
 {
     constexpr uint64_t GM = (P == 64) ? ~0ull : ((1ull << P) - 1ull);
     int len = 0;
@@ -484,7 +460,6 @@ __device__ __forceinline__ int build_glist(Sm& sm, const BvhView& bv, int base, 
                 const float fy = fmaxf(fabsf(qy - lo.y), fabsf(qy - hi.y));
                 const float fz = fmaxf(fabsf(qz - lo.z), fabsf(qz - hi.z));
                 hit = !((fx * fx + fy * fy) + fz * fz < rin);
-                if (skipped && !hit) *skipped += __float_as_uint(lo.w);
             }
         }
         const uint32_t gm = (uint32_t)((ballot(hit) >> (g * P)) & GM);
@@ -571,9 +546,9 @@ __device__ __forceinline__ bool for_each_chunk(Sm& sm, const BvhView& bv, const 
             const int base = (cs.reverse ? nch - 1 - i : i) * CHUNK_LEAVES;
             const int nl = min(CHUNK_LEAVES, cs.ntl - base);
             if (base != cs.staged) {
-                [[maybe_unused]] const auto c0 = ws.tick();
+                [[maybe_unused]] const auto t0 = ws.tick();
                 load_chunk(sm, bv, base, nl);
-                ws.tock(KS_CY_LOAD, c0);
+                ws.tock(KS_CY_LOAD, t0);
                 ws.add(KS_CHUNKS, 1);
                 cs.staged = base;
             }
@@ -586,13 +561,13 @@ __device__ __forceinline__ bool for_each_chunk(Sm& sm, const BvhView& bv, const 
     }
     int sp = start_traversal(sm, bv, cur, tb, R2);
     for (;;) {
-        auto c0 = ws.tick();
+        auto t0 = ws.tick();
         const int nl = fill_leaves(sm, bv, tb, R2, sp, CHUNK_LEAVES, ws);
-        ws.tock(KS_CY_TRAV, c0);
+        ws.tock(KS_CY_TRAV, t0);
         if (sp < 0) return false;
-        c0 = ws.tick();
+        t0 = ws.tick();
         load_chunk(sm, bv, 0, nl);
-        ws.tock(KS_CY_LOAD, c0);
+        ws.tock(KS_CY_LOAD, t0);
         ws.add(KS_CHUNKS, 1);
         f(nl, 0);
         __syncthreads();
@@ -705,24 +680,6 @@ __device__ __forceinline__ float vbin_floor(int b, float inv_w, int nb)
     return x;
 }
 
-// The same for bins that start at an offset: bin 0 holds what lies below, the others are linear above.
-// Only monotony matters: obin_floor finds the exact edges of whatever the roundings make of it.
-__device__ __forceinline__ int obin(float d2, float inv_w, float off, int nb)
-{
-    const int b = (int)fmaxf(d2 * inv_w + off, 0.0f);
-    return b < nb - 1 ? b : nb - 1;
-}
-// Smallest non-negative float x with obin(x) >= b (b >= 1).
-__device__ __forceinline__ float obin_floor(int b, float inv_w, float off, int nb)
-{
-    float x = ((float)b - off) / inv_w;
-    if (!(x >= 0.0f) || isinf(x)) x = 0.0f;
-    for (int it = 0; it < 256 && x > 0.0f && obin(bitsf(fbits(x) - 1u), inv_w, off, nb) >= b; it++)
-        x = bitsf(fbits(x) - 1u);
-    for (int it = 0; it < 256 && obin(x, inv_w, off, nb) < b; it++) x = bitsf(fbits(x) + 1u);
-    return x;
-}
-
 // ---- the kernel -----------------------------------------------------------------------------
 
 // Per-target selection state (replicated over the P lanes of a query).
@@ -744,16 +701,6 @@ __device__ __forceinline__ auto give_lds(S& s, float4* p, int) -> decltype(s.lds
 }
 template <class S>
 __device__ __forceinline__ void give_lds(S&, float4*, long)
-{
-}
-// Sinks of segmented launches learn the stage of their tile.
-template <class S>
-__device__ __forceinline__ auto give_stage(S& s, int stage, int) -> decltype(s.rs.stage = stage, void())
-{
-    s.rs.stage = stage;
-}
-template <class S>
-__device__ __forceinline__ void give_stage(S&, int, long)
 {
 }
 
@@ -786,16 +733,7 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(tile_thre
     const uint32_t nq = qv.nq_dev ? uniform(*qv.nq_dev) : qv.nq;
     if (prm.area_pp) r2 = fmaxf(uniformf(*prm.area_pp) * (float)prm.t0 / 3.14159265f * prm.r2_margin, 1e-30f);
     const float r2_first = r2;
-    int64_t ntiles = ((int64_t)nq + Q - 1) / Q;
-    if (NT == 1 && prm.seg) {
-        ntiles = 0;
-        for (int i = 0; i < ROUND_SEGS; i++) ntiles += (int64_t)(prm.seg[i + 1] - prm.seg[i] + Q - 1) / Q;
-    }
-    // the search of the current tile (of its segment)
-    int t0 = prm.t0;
-    const float* hint_in = prm.hint_in;
-    float* hint_out = prm.hint_out;
-    float hint_scale = prm.hint_scale;
+    const int64_t ntiles = ((int64_t)nq + Q - 1) / Q;
 
     // Runs of tiles_per_wave consecutive tiles, taken from the work queue (every wave ends once
     // it is drained) or strided over the grid (a grid sized for an upper bound of the
@@ -833,43 +771,21 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(tile_thre
         TileBox rbox;
     for (int tt = 0; tt < prm.tiles_per_wave; tt++) {
         const int64_t tile = run * prm.tiles_per_wave + tt;
-        int64_t qbase = tile * Q, qend = nq;
+        const int64_t qbase = tile * Q;
         if (tile >= ntiles) break;
-        if (NT == 1 && prm.seg) {
-            int64_t at = tile;
-            int sg = 0;
-            for (; sg < ROUND_SEGS - 1; sg++) {
-                const int64_t nt = (int64_t)(prm.seg[sg + 1] - prm.seg[sg] + Q - 1) / Q;
-                if (at < nt) break;
-                at -= nt;
-            }
-            sg = uniform(sg);
-            qbase = (int64_t)prm.seg[sg] + at * Q;
-            qend = prm.seg[sg + 1];
-            const bool spec = prm.seg[ROUND_SEGS + 1] != 0u;  // all rounds at once
-            const int stage = seg_stage(sg);
-            const bool from3 = (sg == 1 || sg == 2) && !spec;
-            auto k_of = [&](int r) { return (int)min((int64_t)prm.kn << r, prm.kmax); };
-            t0 = k_of(stage_round(stage));
-            hint_in = from3 ? prm.hint3 : prm.hint1;
-            hint_scale = prm.hint_scale * (float)t0 / (float)k_of(from3 ? 3 : 1);
-            hint_out = stage == 3 && !spec ? prm.hint3 : nullptr;
-            give_stage(sink, spec ? STAGE_SPEC : stage, 0);
-        }
         const int64_t qi = qbase + g;
-        const bool valid = qi < qend;
+        const bool valid = qi < nq;
         const uint32_t qpos = valid ? (qv.qsel ? qv.qsel[qi] : (uint32_t)qi) : 0u;
         const float qx = valid ? qv.qx[qpos] : 0.0f;
         const float qy = valid ? qv.qy[qpos] : 0.0f;
         const float qz = valid ? qv.qz[qpos] : 0.0f;
         const int scan = (valid && bv.scan_of) ? (int)bv.scan_of[qpos] : 0;
-        bool active = valid && t0 > 0;
+        bool active = valid && prm.t0 > 0;
         ws.add(KS_TILES, 1);
-        // the earlier target's neighbourhood of this query, grown for this one (else 0)
-        float hq = 0.0f;
-        if (hint_in) {
-            hq = valid ? hint_in[qpos] * hint_scale : 0.0f;
-            if (!(hq > 0.0f && hq < 1e37f)) hq = 0.0f;
+        if (prm.hint_in) {
+            // the earlier target's neighbourhood of each query, grown for this one
+            const float h = uniformf(wave_max(valid ? prm.hint_in[qpos] : 0.0f));
+            if (h > 0.0f && h < 1e37f) r2 = fmaxf(h * prm.hint_scale, 1e-30f);
         } else if (prm.leaf_hint && tt == 0) {
             // a leaf's 16 points on a surface patch: its box's two largest extents a, b span
             // about (16/9) a b of surface (a 4 x 4 lattice spans 3 x 3 spacings), so t0 points
@@ -881,13 +797,13 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(tile_thre
                 const float ex = hi.x - lo.x, ey = hi.y - lo.y, ez = hi.z - lo.z;
                 const float a = fmaxf(fmaxf(ex, ey), ez), c = fminf(fminf(ex, ey), ez);
                 const float b = (ex + ey + ez) - a - c;
-                est = (float)t0 * a * b * (1.0f / (9.0f * 3.14159265f)) * prm.r2_margin;
+                est = (float)prm.t0 * a * b * (1.0f / (9.0f * 3.14159265f)) * prm.r2_margin;
             }
             const float h = uniformf(wave_max(est));
             if (h > 0.0f && h < 1e37f) r2 = h;
         }
         if (tt == 1 && prm.tiles_per_wave > 2) {
-            [[maybe_unused]] const auto c0 = ws.tick();
+            [[maybe_unused]] const auto t0 = ws.tick();
             const int64_t q0 = qbase, q1 = min((run + 1) * prm.tiles_per_wave * Q, (int64_t)nq);
             const uint32_t p0 = qv.qsel ? qv.qsel[q0] : (uint32_t)q0;
             run_scan = bv.scan_of ? uniform((int)bv.scan_of[p0]) : 0;
@@ -918,7 +834,7 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(tile_thre
                 nrun = nl;
             }
             __syncthreads();
-            ws.tock(KS_CY_TRAV, c0);
+            ws.tock(KS_CY_TRAV, t0);
         }
         sink.begin(g, s, qi, qpos, qx, qy, qz);
         if (s == 0) {
@@ -932,7 +848,6 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(tile_thre
         int shrinks = 0;
         int prev_lead = -1;
         int cl_att = 0;  // attempts of the current cluster
-        bool in_cluster = true, in_hint = false;  // the latter: in_cluster by its hint
 
         for (int attempt = 0; attempt < MAX_ATTEMPTS; attempt++) {
             const uint64_t pending = ballot(active);
@@ -952,26 +867,9 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(tile_thre
             cl_att++;
             const int cur = bv.scan_of ? __builtin_amdgcn_readlane(scan, lead) : 0;
             const float lx = readlane_f(qx, lead), ly = readlane_f(qy, lead), lz = readlane_f(qz, lead);
-            // With hints a cluster starts from those of its own queries, and takes the queries whose hint
-            // is within a factor of the lead's: one query of a sparse region would otherwise set the
-            // radius (and the reach) for queries in dense ones, whose searches then scan many times
-            // what they need.  (Round 5 searched right after round 1, k x 16, on 500,000 points of an
-            // outdoor scan: the slowest such tile alone took 16 ms.)
-            if (hint_in && cl_att == 1) {
-                const float hl = readlane_f(hq, lead);
-                in_cluster = true;
-                in_hint = hl > 0.0f;
-                if (hl > 0.0f) {
-                    const float rl = sqrtf(hl);
-                    in_cluster = lane / P == lead / P ||
-                                 (active && scan == cur && hq <= 2.0f * hl && hq >= 0.5f * hl && fabsf(qx - lx) <= rl &&
-                                  fabsf(qy - ly) <= rl && fabsf(qz - lz) <= rl);
-                    r2 = fmaxf(uniformf(wave_max(in_cluster ? hq : 0.0f)), 1e-30f);
-                }
-            }
             const float reach = sqrtf(r2);
             const bool near = fabsf(qx - lx) <= reach && fabsf(qy - ly) <= reach && fabsf(qz - lz) <= reach;
-            const bool act = active && scan == cur && near && in_cluster;
+            const bool act = active && scan == cur && near;
             // tile box of the pending queries of that scan
             TileBox tb;
             tb.lx = uniformf(wave_min(act ? qx : INFINITY));
@@ -987,7 +885,7 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(tile_thre
             Cands cs;
             float rej = INFINITY;  // nearest box the traversal left out
             {
-                [[maybe_unused]] const auto c0 = ws.tick();
+                [[maybe_unused]] const auto t0 = ws.tick();
                 int sp = 0, nl = 0;
                 if (run_ok && cur == run_scan && R2 <= run_r2 && tb.lx >= rbox.lx && tb.ly >= rbox.ly &&
                     tb.lz >= rbox.lz && tb.hx <= rbox.hx && tb.hy <= rbox.hy && tb.hz <= rbox.hz) {
@@ -1008,15 +906,12 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(tile_thre
                 // through the passes: with far more leaves in range than the tile's targets can
                 // use (the queries' t0 points each, their spread over the tile box widening the
                 // union), shrink it by the leaf count (counts grow like R^2 - r2_floor) before
-                // any point is scanned, MAX_SHRINKS times at most.  One-target searches start from a
-                // hint, so three times what they can use is an overshoot already, and their lists are
-                // long: beyond TL_CAP leaves every pass walks the tree again (with 8 as in round 1 the
-                // slowest tile of 500,000 outdoor points took the launch from 5.5 to 6.6 ms).
-                if (shrinks < MAX_SHRINKS && R2 > r2_floor && cl_att <= CLUSTER_SHRINK) {
+                // any point is scanned.  At most four times per tile.
+                if (shrinks < 4 && R2 > r2_floor && cl_att <= CLUSTER_SHRINK) {
                     const float ext = fmaxf(fmaxf(tb.hx - tb.lx, tb.hy - tb.ly), tb.hz - tb.lz);
                     const float spread = 1.0f + ext / sqrtf(R2);
-                    const float want = ((float)t0 / (float)LEAF + 1.0f) * spread * spread + (float)Q;
-                    const int big = (int)fminf((NT == 1 ? 3.0f : 8.0f) * want, 65536.0f);
+                    const float want = ((float)prm.t0 / (float)LEAF + 1.0f) * spread * spread + (float)Q;
+                    const int big = (int)fminf(8.0f * want, 65536.0f);
                     int total = nl;
                     if (overflow) total = fill_leaves(sm, bv, tb, R2, sp, 4 * big, ws, nullptr, false) + nl;
                     if (total > big) {
@@ -1024,12 +919,12 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(tile_thre
                         r2 = r2_floor + (R2 - r2_floor) * fmaxf(sqrtf(2.0f * want / (float)total), 0.125f);
                         r2_ceil = R2;
                         shrinks++;
-                        ws.tock(KS_CY_TRAV, c0);
+                        ws.tock(KS_CY_TRAV, t0);
                         __syncthreads();
                         continue;
                     }
                 }
-                ws.tock(KS_CY_TRAV, c0);
+                ws.tock(KS_CY_TRAV, t0);
                 cs.ntl = overflow ? -1 : nl;  // the passes then traverse again, chunk by chunk
                 cs.resident = false;
                 cs.staged = -1;
@@ -1044,21 +939,7 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(tile_thre
             const uint32_t hsh = narrow ? 1u : 0u;
             const int nb = HIST_WORDS << hsh;
             const int nbb = HIST_BITS + (int)hsh;
-            // A one-target search with hints (the later adaptive rounds) spends its bins where the t-th key
-            // is expected: above HINT_LO of the query's hint.  Leaves wholly below are counted whole,
-            // and the finer bins seldom hold more keys than the boundary buffer.  A hint that was too
-            // large puts the t-th key into bin 0, which the refinement passes split like any other.
-            const float lo = (NT == 1 && in_hint && cl_att == 1) ? fminf(hq * HINT_LO, R2 * 0.75f) : 0.0f;
-            const float inv_w = NT == 1 ? (float)(nb - 1) / (R2 - lo) : (float)nb / R2;
-            const float off = (NT == 1 && inv_w > 0.0f) ? 1.0f - lo * inv_w : 0.0f;  // (R2 = inf: one bin)
-            auto bin_of = [&](float d2) {
-                if constexpr (NT == 1) return obin(d2, inv_w, off, nb);
-                return vbin(d2, inv_w, nb);
-            };
-            auto bin_floor = [&](int b) {
-                if constexpr (NT == 1) return obin_floor(b, inv_w, off, nb);
-                return vbin_floor(b, inv_w, nb);
-            };
+            const float inv_w = (float)nb / R2;
             auto locate = [&](int t, int& b, int& below, int& cnt) {
                 if constexpr (NT == 1) {
                     if (narrow) return find_bin<P, Q, 2 * HIST_WORDS>(sm.hist, g, s, t, b, below, cnt);
@@ -1068,35 +949,25 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(tile_thre
             for (int b = s; b < HIST_WORDS; b += P) sm.hist[g][b] = 0u;
             __syncthreads();
             uint32_t* myhist = &sm.hist[g][0];
-            float dmin = INFINITY;  // nearest in-range candidate of this lane (0: a leaf counted whole)
-            const float lo1 = lo > 0.0f ? bin_floor(1) : -1.0f;  // below it a point is in bin 0
-            uint32_t inner = 0u;  // points of the leaves wholly below lo1 (this lane's leaves)
+            float dmin = INFINITY;  // nearest in-range candidate of this lane
             bool fine = for_each_chunk(sm, bv, tb, R2, cur, cs, ws, [&](int nl, int base) {
-                auto c0 = ws.tick();
-                const int len = NT == 1 ? build_glist<P>(sm, bv, base, nl, g, s, qx, qy, qz, act ? R2 : -1.0f, lo1, &inner)
-                                        : build_glist<P>(sm, bv, base, nl, g, s, qx, qy, qz, act ? R2 : -1.0f);
-                ws.tock(KS_CY_GLIST, c0);
-                c0 = ws.tick();
+                auto t0 = ws.tick();
+                const int len = build_glist<P>(sm, bv, base, nl, g, s, qx, qy, qz, act ? R2 : -1.0f);
+                ws.tock(KS_CY_GLIST, t0);
+                t0 = ws.tick();
                 scan_glist<P>(sm, g, s, len, [&](const float4& p, int) {
                     const float d2 = d2_contract(qx, qy, qz, p.x, p.y, p.z);
                     if (d2 <= R2) {
-                        hist_add(myhist, bin_of(d2), hsh);
+                        hist_add(myhist, vbin(d2, inv_w, nb), hsh);
                         dmin = fminf(dmin, d2);
                     }
                 });
-                ws.tock(KS_CY_HIST, c0);
+                ws.tock(KS_CY_HIST, t0);
                 if constexpr (kStats) ws.add(KS_CANDIDATES, (unsigned)(LEAF * wave_sum_int(s == 0 ? len : 0)));
             });
             if (!fine) {
                 if (lane == 0) atomicMax(prm.err, 5);
                 return;
-            }
-            if constexpr (NT == 1) {
-                if (inner) {
-                    atomicAdd(myhist, inner);
-                    dmin = 0.0f;
-                }
-                __syncthreads();
             }
             if (cs.resident) ws.add(KS_RESIDENT, 1);
 
@@ -1107,12 +978,12 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(tile_thre
             int in_range = 0;
             {
                 int b, below, cnt;
-                const int total = locate(t0, b, below, cnt);
+                const int total = locate(prm.t0, b, below, cnt);
                 in_range = total;
-                ok = act && total >= t0;
+                ok = act && total >= prm.t0;
 #pragma unroll
                 for (int tau = 0; tau < NT; tau++) {
-                    const int t = tau == 0 ? t0 : tau == 1 ? prm.t1 : tau == 2 ? prm.t2 : prm.t3;
+                    const int t = tau == 0 ? prm.t0 : tau == 1 ? prm.t1 : tau == 2 ? prm.t2 : prm.t3;
                     tg[tau].t = t;
                     tg[tau].refine = false;
                     tg[tau].below = 0;
@@ -1123,12 +994,12 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(tile_thre
                         if (t > 0) locate(t, b, below, cnt);
                     }
                     if (ok && t > 0) {
-                        const float blo = b == 0 ? 0.0f : bin_floor(b);
-                        tg[tau].klo = (uint64_t)fbits(blo) << 32;
+                        const float lo = b == 0 ? 0.0f : vbin_floor(b, inv_w, nb);
+                        tg[tau].klo = (uint64_t)fbits(lo) << 32;
                         if (b == nb - 1 || !(inv_w > 0.0f)) {
                             tg[tau].khi = ((uint64_t)fbits(R2) << 32) | 0xffffffffull;
                         } else {
-                            const float hi = bin_floor(b + 1);
+                            const float hi = vbin_floor(b + 1, inv_w, nb);
                             tg[tau].khi = ((uint64_t)fbits(hi) << 32) - 1ull;
                         }
                         tg[tau].below = below;
@@ -1205,12 +1076,12 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(tile_thre
             const bool whole = kLeaves && (NT < 2 || prm.t1 <= 0) && (NT < 3 || prm.t2 <= 0) && (NT < 4 || prm.t3 <= 0);
             const float rfull = (whole && ok) ? tg[0].dlo : -1.0f;
             auto collect = [&](int nl, int base) {
-                auto c0 = ws.tick();
+                auto t0 = ws.tick();
                 int nfull = 0;
                 const int len = whole ? build_glist_split<P>(sm, nl, g, s, qx, qy, qz, rc, rfull, nfull)
                                       : build_glist<P>(sm, bv, base, nl, g, s, qx, qy, qz, rc);
-                ws.tock(KS_CY_GLIST, c0);
-                c0 = ws.tick();
+                ws.tock(KS_CY_GLIST, t0);
+                t0 = ws.tick();
                 if constexpr (kLeaves) {
                     for (int j = s; j < nfull; j += P) {
                         const int js = sm.flist[g][j];
@@ -1240,7 +1111,7 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(tile_thre
                         }
                     }
                 });
-                ws.tock(KS_CY_COLLECT, c0);
+                ws.tock(KS_CY_COLLECT, t0);
             };
             fine = for_each_chunk(sm, bv, tb, fminf(uniformf(wave_max(rc)), R2), cur, cs, ws, collect);
             if (!fine) {
@@ -1270,7 +1141,7 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(tile_thre
                     }
                 }
             }
-            if (hint_out && kth >= 0.0f) hint_out[qpos] = kth;
+            if (prm.hint_out && kth >= 0.0f) prm.hint_out[qpos] = kth;
             __syncthreads();
             sink.finish(g, s, ok, qpos, qx, qy, qz, sm.scnt[0], sm.scnt[NT > 1 ? 1 : 0]);
             ws.tock(KS_CY_FINISH, t_fin);
@@ -1298,7 +1169,7 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(tile_thre
                 if (act && !ok) {
                     if (in_range > 0) {
                         const float disc = R2 - dm;
-                        need = dm + disc * fmaxf((float)t0 / (float)in_range * 1.25f, fmaxf(prm.grow_min, 1.5f));
+                        need = dm + disc * fmaxf((float)prm.t0 / (float)in_range * 1.25f, fmaxf(prm.grow_min, 1.5f));
                     } else if (rej < INFINITY) {
                         need = disc_hint > 0.0f ? rej + 1.5f * disc_hint : rej * 1.1f;
                     } else {
@@ -1311,7 +1182,7 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(tile_thre
                 if (!(nr2 > R2) || nr2 < 1e-30f) nr2 = fmaxf(R2 * 4.0f, 1e-30f);
                 if (nr2 > 1e37f) nr2 = INFINITY;
                 // below a radius already found too wide, unless shrinking is over
-                if (shrinks < MAX_SHRINKS && nr2 > r2_ceil && cl_att <= CLUSTER_SHRINK)
+                if (shrinks < 4 && nr2 > r2_ceil && cl_att <= CLUSTER_SHRINK)
                     nr2 = fmaxf(R2 + (r2_ceil - R2) * 0.5f, R2 * 1.01f);
                 r2_floor = R2;
                 r2 = nr2;

@@ -138,22 +138,8 @@ __global__ void gather_queries_kernel(const float* __restrict__ q, int64_t m, co
     qz[i] = q[3 * (int64_t)j + 2];
 }
 
-// Ordered compaction of the entries whose flag is set, or whose point has a given action (the adaptive
-// rounds' query lists): per-4096 block counts, one scan of the block counts, then a block-local stable
-// scatter.
-struct CompactIf {
-    const uint32_t* flags;  // per entry (NULL: by action)
-    const uint8_t* act;     // per point
-    int code;               // wanted action; < 0: any but 0
-    const uint32_t* qsel;   // entry -> point (NULL: the same)
-    __device__ __forceinline__ uint32_t point(int64_t i) const { return qsel ? qsel[i] : (uint32_t)i; }
-    __device__ __forceinline__ bool operator()(int64_t i) const
-    {
-        if (flags) return flags[i] != 0u;
-        const int a = act[point(i)];
-        return code < 0 ? a != 0 : a == code;
-    }
-};
+// Ordered compaction of the entries whose flag is set (the adaptive rounds' query lists): per-4096 block
+// counts, one scan of the block counts, then a block-local stable scatter.
 constexpr int CF_THREADS = 256;
 constexpr int CF_ITEMS = 16;
 constexpr int CF_TILE = CF_THREADS * CF_ITEMS;
@@ -183,7 +169,7 @@ __device__ __forceinline__ uint32_t cf_block_sum(const uint32_t* __restrict__ a,
 // about 5 us on the device, more than the sums of 1,024 counts in every block).
 constexpr int CF_SELF_BLOCKS = 1024;
 
-__global__ __launch_bounds__(CF_THREADS) void flag_block_sums_kernel(const CompactIf pred, int64_t n,
+__global__ __launch_bounds__(CF_THREADS) void flag_block_sums_kernel(const uint32_t* __restrict__ flags, int64_t n,
                                                                      const uint32_t* __restrict__ n_dev,
                                                                      uint32_t* __restrict__ bsum)
 {
@@ -195,7 +181,7 @@ __global__ __launch_bounds__(CF_THREADS) void flag_block_sums_kernel(const Compa
 #pragma unroll
         for (int r = 0; r < CF_ITEMS; r++) {
             const int64_t i = cf_entry(r);
-            f[r] = i < n && pred(i);
+            f[r] = i < n && flags[i] != 0u;
         }
 #pragma unroll
         for (int r = 0; r < CF_ITEMS; r++) c += (uint32_t)__popcll(ballot(f[r]));
@@ -209,10 +195,11 @@ __global__ __launch_bounds__(CF_THREADS) void flag_block_sums_kernel(const Compa
     }
 }
 
-__global__ __launch_bounds__(CF_THREADS) void compact_scatter_kernel(const CompactIf pred, int64_t n,
+__global__ __launch_bounds__(CF_THREADS) void compact_scatter_kernel(const uint32_t* __restrict__ flags, int64_t n,
                                                                      const uint32_t* __restrict__ n_dev,
                                                                      const uint32_t* __restrict__ boff, bool self,
                                                                      uint32_t* __restrict__ count,
+                                                                     const uint32_t* __restrict__ qsel,
                                                                      uint32_t* __restrict__ out)
 {
     // self: boff holds the blocks' counts (else their offsets), and the last block writes their sum
@@ -228,8 +215,8 @@ __global__ __launch_bounds__(CF_THREADS) void compact_scatter_kernel(const Compa
 #pragma unroll
     for (int r = 0; r < CF_ITEMS; r++) {
         const int64_t i = cf_entry(r);
-        f[r] = i < n && pred(i);
-        pt[r] = i < n ? pred.point(i) : 0u;
+        f[r] = i < n && flags[i] != 0u;
+        pt[r] = i < n ? (qsel ? qsel[i] : (uint32_t)i) : 0u;
     }
 #pragma unroll
     for (int r = 0; r < CF_ITEMS; r++) c += (uint32_t)__popcll(ballot(f[r]));
@@ -242,137 +229,6 @@ __global__ __launch_bounds__(CF_THREADS) void compact_scatter_kernel(const Compa
         if (f[r]) out[run + (uint32_t)mbcnt(m)] = pt[r];
         run += (uint32_t)__popcll(m);
     }
-}
-
-// Stable partition of a point list by the points' next stage (act) into the segments of ROUND_SEGS: block
-// counts per segment, one scan of the segment-major table, a stable scatter; seg[i] = where segment i starts,
-// seg[ROUND_SEGS] = the end.  Resolved points (act 0) are dropped.
-// A list of at most `spec` points goes into the segments of rounds 5, 4, 3 and 2 at once (seg[ROUND_SEGS + 1]
-// = 1): four times the searches in one launch, which a small list leaves room for, instead of up to four
-// launches one after the other, each as long as its slowest tile (spec_resolve_kernel).
-// In the first partition (nq > 0: of so many points) a point goes to round 5 at once only if at most 45 % of
-// the points were rejected.  Where more are, the cloud is sparse for its k and the k-th distance of round 1
-// says little about k x 16: 42 % of those searches needed a second radius (15 % in the room), and round 3
-// first is as good by the model and steadier.
-__device__ __forceinline__ uint32_t act_segments(int a, int64_t n, uint32_t spec, int64_t nq)
-{
-    if (n <= spec) return 0x1Du;  // stages 5, 4, 3, 2
-    if (a == 5 && 20 * n > 9 * nq && nq > 0) a = 3;
-    uint32_t m = 0u;
-    for (int i = 0; i < ROUND_SEGS; i++) m |= seg_stage(i) == a ? 1u << i : 0u;
-    return m;
-}
-__global__ __launch_bounds__(CF_THREADS) void part_sums_kernel(const uint8_t* __restrict__ act,
-                                                               const uint32_t* __restrict__ list,
-                                                               const uint32_t* __restrict__ n_dev, uint32_t spec, int64_t nq,
-                                                               uint32_t* __restrict__ bsum)
-{
-    __shared__ uint32_t ws[CF_WAVES][ROUND_SEGS];
-    const int64_t n = (int64_t)*n_dev;
-    uint32_t c[ROUND_SEGS] = {};
-    if ((int64_t)blockIdx.x * CF_TILE < n) {
-        uint32_t sg[CF_ITEMS];
-#pragma unroll
-        for (int r = 0; r < CF_ITEMS; r++) {
-            const int64_t i = cf_entry(r);
-            sg[r] = i < n ? act_segments(act[list[i]], n, spec, nq) : 0u;
-        }
-#pragma unroll
-        for (int r = 0; r < CF_ITEMS; r++)
-#pragma unroll
-            for (int k = 0; k < ROUND_SEGS; k++) c[k] += (uint32_t)__popcll(ballot((sg[r] >> k) & 1u));
-    }
-    if (lane_id() == 0)
-#pragma unroll
-        for (int k = 0; k < ROUND_SEGS; k++) ws[threadIdx.x / kWave][k] = c[k];
-    __syncthreads();
-    if (threadIdx.x < ROUND_SEGS) {
-        uint32_t t = 0;
-        for (int w = 0; w < CF_WAVES; w++) t += ws[w][threadIdx.x];
-        bsum[(size_t)threadIdx.x * gridDim.x + blockIdx.x] = t;
-    }
-}
-__global__ __launch_bounds__(CF_THREADS) void part_scatter_kernel(const uint8_t* __restrict__ act,
-                                                                  const uint32_t* __restrict__ list,
-                                                                  const uint32_t* __restrict__ n_dev, uint32_t spec, int64_t nq,
-                                                                  const uint32_t* __restrict__ boff, bool self,
-                                                                  const uint32_t* __restrict__ total,
-                                                                  uint32_t* __restrict__ out, uint32_t* __restrict__ seg)
-{
-    // self: boff holds the blocks' counts (else their offsets)
-    __shared__ uint32_t ws[CF_WAVES][ROUND_SEGS], start[ROUND_SEGS + 1];
-    const int64_t n = (int64_t)*n_dev;
-    if (blockIdx.x > 0 && (int64_t)blockIdx.x * CF_TILE >= n) return;
-    uint32_t run[ROUND_SEGS];
-    if (self) {
-        const int used = (int)((n + CF_TILE - 1) / CF_TILE), mine = min((int)blockIdx.x, used);  // later blocks: 0
-        uint32_t before = 0;
-        for (int k = 0; k < ROUND_SEGS; k++) {
-            const uint32_t* c = boff + (size_t)k * gridDim.x;
-            const uint32_t lo = cf_block_sum(c, mine, &ws[0][0]), hi = cf_block_sum(c + mine, used - mine, &ws[0][0]);
-            if (threadIdx.x == 0) start[k] = before;
-            run[k] = before + lo;
-            before += lo + hi;
-        }
-        if (threadIdx.x == 0) start[ROUND_SEGS] = before;
-        __syncthreads();
-        if (blockIdx.x == 0 && threadIdx.x <= ROUND_SEGS) seg[threadIdx.x] = start[threadIdx.x];
-    } else {
-        for (int k = 0; k < ROUND_SEGS; k++) run[k] = boff[(size_t)k * gridDim.x + blockIdx.x];
-        if (blockIdx.x == 0 && threadIdx.x <= ROUND_SEGS)
-            seg[threadIdx.x] = threadIdx.x < ROUND_SEGS ? boff[(size_t)threadIdx.x * gridDim.x] : *total;
-    }
-    if (blockIdx.x == 0 && threadIdx.x == 0) seg[ROUND_SEGS + 1] = n <= spec ? 1u : 0u;
-    const int wave = threadIdx.x / kWave;
-    uint32_t pt[CF_ITEMS], sg[CF_ITEMS], c[ROUND_SEGS] = {};
-#pragma unroll
-    for (int r = 0; r < CF_ITEMS; r++) {
-        const int64_t i = cf_entry(r);
-        pt[r] = i < n ? list[i] : 0u;
-        sg[r] = i < n ? act_segments(act[pt[r]], n, spec, nq) : 0u;
-    }
-#pragma unroll
-    for (int r = 0; r < CF_ITEMS; r++)
-#pragma unroll
-        for (int k = 0; k < ROUND_SEGS; k++) c[k] += (uint32_t)__popcll(ballot((sg[r] >> k) & 1u));
-    if (lane_id() == 0)
-#pragma unroll
-        for (int k = 0; k < ROUND_SEGS; k++) ws[wave][k] = c[k];
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < ROUND_SEGS; k++)
-        for (int w = 0; w < wave; w++) run[k] += ws[w][k];
-#pragma unroll
-    for (int r = 0; r < CF_ITEMS; r++)
-#pragma unroll
-        for (int k = 0; k < ROUND_SEGS; k++) {
-            const bool f = (sg[r] >> k) & 1u;
-            const uint64_t m = ballot(f);
-            if (f) out[run[k] + (uint32_t)mbcnt(m)] = pt[r];
-            run[k] += (uint32_t)__popcll(m);
-        }
-}
-
-// After a launch that searched rounds 2..5 of every rejected point at once: the first round whose box passes
-// (else round 5), its moments, and no stage left.  Entry i of every segment is the list's point i.
-__global__ __launch_bounds__(256) void spec_resolve_kernel(const uint32_t* __restrict__ seg,
-                                                           const uint32_t* __restrict__ list,
-                                                           const float* __restrict__ smom,
-                                                           const uint8_t* __restrict__ sok, float* __restrict__ mom,
-                                                           uint8_t* __restrict__ kround, uint8_t* __restrict__ act)
-{
-    if (seg[ROUND_SEGS + 1] == 0u) return;
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= seg[1] - seg[0]) return;
-    const uint32_t q = list[seg[0] + i];
-    // segments 4, 3, 2 are rounds 2, 3, 4; segment 0 is round 5
-    const int sg = sok[seg[4] + i] ? 4 : sok[seg[3] + i] ? 3 : sok[seg[2] + i] ? 2 : 0;
-    const float* m = smom + (size_t)(seg[sg] + i) * 9;
-    float* o = mom + (size_t)q * 9;
-#pragma unroll
-    for (int k = 0; k < 9; k++) o[k] = m[k];
-    kround[q] = (uint8_t)stage_round(seg_stage(sg));
-    act[q] = 0;
 }
 
 // interpolateSurfaceNormals (AdaptiveKSearchSurface.tcc:312-327): the point's own normal
@@ -923,10 +779,7 @@ struct lvrhip_surface {
     DBuf<uint64_t> s_k0, s_k1;
     DBuf<uint32_t> s_v0, s_v1, s_hist, s_flags, s_list0, s_list1, s_spos, s_ord, s_sample;
     DBuf<float> s_qx, s_qy, s_qz, s_f;
-    DBuf<float> s_hint, s_hint3;  // per sorted point: the k-th d^2 of adaptive rounds 1 and 3
-    DBuf<float4> pst;             // per sorted point: what its searched rounds showed (RoundState)
-    DBuf<uint32_t> s_seg;         // the segments of the later rounds' list
-    DBuf<uint8_t> act;            // per sorted point: its next stage (RoundState)
+    DBuf<float> s_hint;  // per sorted point: the k-th d^2 of its last adaptive round
     DBuf<int32_t> s_idx;
 
     BvhView view() const
@@ -1180,34 +1033,17 @@ struct lvrhip_surface {
     void compact_flags(const uint32_t* flags, int64_t nq, const uint32_t* nq_dev, const uint32_t* qsel, uint32_t* out,
                        uint32_t* count_dev)
     {
-        s_bsum.reserve(std::max<int64_t>(ceil_div(nq, CF_TILE), 1) + 1);
-        compact_flags_with(flags, nq, nq_dev, qsel, out, count_dev, s_bsum.p);
-    }
-    // the points of q[0, min(nq, *nq_dev)) with action code (< 0: any but 0), in order
-    void compact_act(int code, int64_t nq, const uint32_t* nq_dev, const uint32_t* q, uint32_t* out,
-                     uint32_t* count_dev)
-    {
-        s_bsum.reserve(std::max<int64_t>(ceil_div(nq, CF_TILE), 1) + 1);
-        compact_if(CompactIf{nullptr, act.p, code, q}, nq, nq_dev, out, count_dev, s_bsum.p);
-    }
-    // the same with the caller's block-sum buffer (ceil(nq / CF_TILE) + 1 entries)
-    void compact_flags_with(const uint32_t* flags, int64_t nq, const uint32_t* nq_dev, const uint32_t* qsel,
-                            uint32_t* out, uint32_t* count_dev, uint32_t* bsum)
-    {
-        compact_if(CompactIf{flags, nullptr, 0, qsel}, nq, nq_dev, out, count_dev, bsum);
-    }
-    void compact_if(const CompactIf& pred, int64_t nq, const uint32_t* nq_dev, uint32_t* out, uint32_t* count_dev,
-                    uint32_t* bsum)
-    {
         const int64_t nb = std::max<int64_t>(ceil_div(nq, CF_TILE), 1);
-        flag_block_sums_kernel<<<(unsigned)nb, CF_THREADS, 0, st>>>(pred, nq, nq_dev, bsum);
+        s_bsum.reserve(nb + 1);
+        flag_block_sums_kernel<<<(unsigned)nb, CF_THREADS, 0, st>>>(flags, nq, nq_dev, s_bsum.p);
         LVRHIP_LAUNCH_CHECK();
         const bool self = nb <= CF_SELF_BLOCKS;
         if (!self) {
-            scan_exclusive_kernel<<<1, 1024, 0, st>>>(bsum, nb, count_dev);
+            scan_exclusive_kernel<<<1, 1024, 0, st>>>(s_bsum.p, nb, count_dev);
             LVRHIP_LAUNCH_CHECK();
         }
-        compact_scatter_kernel<<<(unsigned)nb, CF_THREADS, 0, st>>>(pred, nq, nq_dev, bsum, self, count_dev, out);
+        compact_scatter_kernel<<<(unsigned)nb, CF_THREADS, 0, st>>>(flags, nq, nq_dev, s_bsum.p, self, count_dev, qsel,
+                                                                   out);
         LVRHIP_LAUNCH_CHECK();
     }
 
@@ -1228,55 +1064,35 @@ struct lvrhip_surface {
         a_sel.reserve(n);
         a_list.reserve(n);
         s_hint.reserve(npad);
-        s_hint3.reserve(npad);
-        pst.reserve(npad);
-        act.reserve(npad);
-        s_seg.reserve(ROUND_SEGS + 2);
-        spec_mom.reserve(4 * 9 * (size_t)spec_points());
-        spec_ok.reserve(4 * (size_t)spec_points());
-        s_bsum.reserve(ROUND_SEGS * std::max<int64_t>(ceil_div(n, CF_TILE), 1) + 1);
     }
 
-    // A rejected list up to this length is searched for rounds 2..5 at once: 4 x 16,384 searches are
-    // about three times what the device holds, as long as the launches one after the other (four of
-    // 130-290 us for the 4,000 rejected points of the 30,000-point plain scene).
-    // A quarter of the cloud at most, so that its buffers are no larger than the others.
-    static constexpr uint32_t SPEC_POINTS = 16384;
-    uint32_t spec_points() const { return (uint32_t)std::min<int64_t>(SPEC_POINTS, n / 4); }
-    DBuf<float> spec_mom;   // per entry of that launch: its moments,
-    DBuf<uint8_t> spec_ok;  // and whether its box passes
-
-    // A launch of the adaptive rounds: round 1 for the points of qsel (stage 1; stage 0: flags in s_flags for
-    // the merged rounds), or, with seg, the next stage of every point of the partitioned list qsel.
-    void enqueue_round(int stage, const uint32_t* qsel, int64_t nq, const uint32_t* seg, int queue)
+    // Adaptive round r (k = kn * 2^r) for the points of qsel: flags in s_flags the points whose box fails, unless
+    // it is the last, and in kround the others.  queue: as in tile().
+    void enqueue_round(int r, const uint32_t* qsel, int64_t nq, const uint32_t* nq_dev, int queue)
     {
-        const bool first = seg == nullptr;
-        TileParams prm = params(clamp_k((int64_t)kn << (first ? 1 : 5)), first ? kiw : 0, 0);
+        TileParams prm = params(clamp_k((int64_t)kn << r), r == 1 ? kiw : 0, 0);
         // the later rounds' query lists are sparse: a run's consecutive tiles lie far apart, so
         // its shared leaf list does not pay, and one tile per run balances their costlier tiles;
         // round 1 keeps at least two runs per resident wave (a small cloud has few tiles)
-        if (first)
+        if (r > 1)
+            prm.tiles_per_wave = 1;
+        else
             prm.tiles_per_wave = (int)std::clamp<int64_t>(
                 ceil_div(nq, kWave / lanes_per_query) / (2 * resident_waves), 1, tiles_per_wave);
-        else
-            prm.tiles_per_wave = 1;
-        // an earlier round's k-th d^2 per point sizes the first radius: on a surface the count grows
-        // like d^2 (x 1.15 of margin, for round 5 after round 1 too: 1.0 and 1.35 cost 33 % and 7 % more
-        // cycles per query there; the tuned r2_margin only sizes the radius carried from tile to tile)
-        prm.hint_scale = 1.15f;
-        prm.seg = seg;
-        prm.kn = kn;
-        prm.kmax = nscans == 1 ? n : ((int64_t)1 << 40);
-        prm.hint1 = s_hint.p;
-        prm.hint3 = s_hint3.p;
-        prm.hint_out = stage == 1 ? s_hint.p : nullptr;
+        // each round's k-th d^2 per point sizes the next round's first radius: k doubles, and
+        // on a surface the count grows like d^2 (x 1.15 of margin; the tuned r2_margin only
+        // sizes the radius carried from tile to tile)
+        prm.hint_in = r > 1 ? s_hint.p : nullptr;
+        prm.hint_scale = 2.0f * 1.15f;
+        prm.hint_out = r < 5 && !merge_retry ? s_hint.p : nullptr;
         prm.leaf_hint = 1;
-        prm.stats = kstats_ptr(first ? 0 : 5);  // the later rounds share launches
-        QueryView qv{px.p, py.p, pz.p, qsel, (uint32_t)nq, nullptr};
+        prm.stats = kstats_ptr(r - 1);
+        QueryView qv{px.p, py.p, pz.p, qsel, (uint32_t)nq, nq_dev};
         auto fill = [&](auto& s) {
             s.mom = mom.p;
-            s.retry = stage == 0 ? s_flags.p : nullptr;
-            s.rs = RoundState{pst.p, stage == 0 ? nullptr : act.p, kround.p, stage, spec_mom.p, spec_ok.p};
+            s.retry = r < 5 ? s_flags.p : nullptr;
+            s.kround = kround.p;
+            s.round = r;
             s.ki_list = ki_list.p;
             s.kiw = prm.t1;
         };
@@ -1290,7 +1106,7 @@ struct lvrhip_surface {
             fill(s);
             return s;
         };
-        const int tok = prof.start(first ? LVRHIP_T_NORMALS_FIRST : LVRHIP_T_NORMALS_RETRY, st);
+        const int tok = prof.start(r == 1 ? LVRHIP_T_NORMALS_FIRST : LVRHIP_T_NORMALS_RETRY, st);
         if (prm.t1 > 0)
             tile<SinkNormals>(qv, prm, lanes_per_query, mk(std::integral_constant<int, 2>()),
                               mk(std::integral_constant<int, 4>()), mk(std::integral_constant<int, 8>()), 0, queue);
@@ -1301,15 +1117,21 @@ struct lvrhip_surface {
     }
 
     // calculateSurfaceNormals' adaptive rounds (AdaptiveKSearchSurface.tcc:187-284) for the
-    // queries q0[0, nq0) (NULL: all points): round r's neighbourhood is k = kn * 2^r, and a point's
-    // the first whose box passes.  Rounds 2..5 are searched in the order of RoundState (sinks.hpp), or
-    // merged; the counts stay on the device, so the sequence enqueues without host synchronisation.
+    // queries q0[0, nq0) (NULL: all points): round r searches k = kn * 2^r for the queries the
+    // previous round's bounding-box test rejected; the counts stay on the device, so the
+    // sequence enqueues without host synchronisation.
+    // The radii that a tile tries decide the order in which its neighbourhoods' moments are added up, and that
+    // order decides the sign of a normal whose plane runs through the flip point: n . (f - q) is 0 up to
+    // rounding on every point of a wall seen edge-on.  Rounds out of order (a later round's box can prove that
+    // the ones between fail), radius margins by k and clusters by hint distance searched 15 to 25 % faster, and
+    // reversed normals in 2 of 28 outdoor clouds of 16M points; so the rounds run one after the other, and
+    // test_gpu_orientation.py holds the signs.
     void enqueue_normals(const uint32_t* q0, int64_t nq0)
     {
         nq_first = nq0;
         if (nq0 == 0) return;
         if (merge_retry) {
-            enqueue_round(0, q0, nq0, nullptr, -1);
+            enqueue_round(1, q0, nq0, nullptr, -1);
             plane_fit(q0, nq0, nullptr, s_flags.p, clamp_k((int64_t)kn << 1), 1);
             compact_flags(s_flags.p, nq0, nullptr, q0, s_list1.p, counter(2));
             enqueue_merged_rounds(s_list1.p, counter(2), nq0);
@@ -1321,44 +1143,15 @@ struct lvrhip_surface {
             fill_u32_kernel<<<(unsigned)ceil_div(len, 256), 256, 0, st>>>(d_queue.p, len, 0u);
             LVRHIP_LAUNCH_CHECK();
         }
-        enqueue_round(1, q0, nq0, nullptr, 0);
-        uint32_t* rejected = s_list1.p;
-        compact_act(-1, nq0, nullptr, q0, rejected, counter(2));
-        // a point's longest way: stages 5, 3, 2, 4 or 3, 2, 15, 4
-        for (int pass = 0; pass < 4; pass++) {
-            partition_stages(rejected, nq0, pass == 0);
-            enqueue_round(2, s_list0.p, nq0, s_seg.p, 1 + pass);
-            if (pass == 0) {
-                spec_resolve_kernel<<<(unsigned)ceil_div(std::max(spec_points(), 1u), 256), 256, 0, st>>>(s_seg.p, s_list0.p, spec_mom.p, spec_ok.p,
-                                                                      mom.p, kround.p, act.p);
-                LVRHIP_LAUNCH_CHECK();
-            }
+        uint32_t* lists[2] = {s_list0.p, s_list1.p};
+        for (int r = 1; r <= 5; r++) {
+            const uint32_t* qsel = r == 1 ? q0 : lists[(r - 1) & 1];
+            const uint32_t* nq_dev = r == 1 ? nullptr : counter(r);
+            enqueue_round(r, qsel, nq0, nq_dev, r - 1);
+            // rejected queries -> the next round's list and count
+            if (r < 5) compact_flags(s_flags.p, nq0, nq_dev, qsel, lists[r & 1], counter(r + 1));
         }
         plane_fit(q0, nq0, nullptr, nullptr, -1, 0);
-        // points whose neighbourhood search reaches rounds 3, 4 and 5
-        fill_u32_kernel<<<1, 64, 0, st>>>(counter(3), 3, 0u);
-        LVRHIP_LAUNCH_CHECK();
-        round_count_kernel<<<(unsigned)ceil_div(nq0, 256), 256, 0, st>>>(rejected, counter(2), nq0, kround.p,
-                                                                        counter(0));
-        LVRHIP_LAUNCH_CHECK();
-    }
-
-    // s_list0 = the points of list[0, *counter(2)) by their next stage, s_seg = the segments (the first
-    // time, a list of at most spec_points(): every round of every point)
-    void partition_stages(const uint32_t* list, int64_t nq0, bool first)
-    {
-        const uint32_t spec = first ? spec_points() : 0u;
-        const int64_t nb = std::max<int64_t>(ceil_div(nq0, CF_TILE), 1);
-        part_sums_kernel<<<(unsigned)nb, CF_THREADS, 0, st>>>(act.p, list, counter(2), spec, first ? nq0 : 0, s_bsum.p);
-        LVRHIP_LAUNCH_CHECK();
-        const bool self = nb <= CF_SELF_BLOCKS;
-        if (!self) {
-            scan_exclusive_kernel<<<1, 1024, 0, st>>>(s_bsum.p, ROUND_SEGS * nb, counter(6));
-            LVRHIP_LAUNCH_CHECK();
-        }
-        part_scatter_kernel<<<(unsigned)nb, CF_THREADS, 0, st>>>(act.p, list, counter(2), spec, first ? nq0 : 0, s_bsum.p,
-                                                                self, counter(6), s_list0.p, s_seg.p);
-        LVRHIP_LAUNCH_CHECK();
     }
 
     // Rounds 2..5 for the queries round 1 rejected, in one search with four targets
@@ -1996,7 +1789,7 @@ struct lvrhip_surface {
         LVRHIP_LAUNCH_CHECK();
         const int64_t nb = ceil_div(m, (int64_t)LAT_TILE);
         s_bsum.reserve(nb + 1);
-        flag_block_sums_kernel<<<(unsigned)nb, CF_THREADS, 0, st>>>(CompactIf{g_flags.p, nullptr, 0, nullptr}, m, nullptr, s_bsum.p);
+        flag_block_sums_kernel<<<(unsigned)nb, CF_THREADS, 0, st>>>(g_flags.p, m, nullptr, s_bsum.p);
         LVRHIP_LAUNCH_CHECK();
         scan_exclusive_kernel<<<1, 1024, 0, st>>>(s_bsum.p, nb, counter(7));
         LVRHIP_LAUNCH_CHECK();
@@ -2093,7 +1886,7 @@ struct lvrhip_surface {
         LVRHIP_LAUNCH_CHECK();
         const int64_t nb = ceil_div(m, (int64_t)LAT_TILE);
         s_bsum.reserve(nb + 1);
-        flag_block_sums_kernel<<<(unsigned)nb, CF_THREADS, 0, st>>>(CompactIf{g_flags.p, nullptr, 0, nullptr}, m, nullptr, s_bsum.p);
+        flag_block_sums_kernel<<<(unsigned)nb, CF_THREADS, 0, st>>>(g_flags.p, m, nullptr, s_bsum.p);
         LVRHIP_LAUNCH_CHECK();
         scan_exclusive_kernel<<<1, 1024, 0, st>>>(s_bsum.p, nb, counter(10));
         LVRHIP_LAUNCH_CHECK();

@@ -129,100 +129,6 @@ __device__ inline void plane_from_moments(int method, int kcount, float qx, floa
     }
 }
 
-// The adaptive rounds out of order.  A point's neighbourhood k = kn 2^r is the first of r = 1..5 whose
-// bounding box passes boundingBoxOK (AdaptiveKSearchSurface.tcc:187-216, 337-350), which fails exactly
-// when its smallest extent is below 0.05 times its largest.  The k-sets are nested, so both extents only
-// grow with r: if round b fails and its smallest extent is below 0.05 times the largest extent of an
-// earlier failed round a, every round between fails too, and need not be searched (all roundings are
-// monotone: an exact statement about the fp32 test).  After round 1 a rejected point therefore goes
-// Each launch searches every point's next stage (knn_tile.hpp, ROUND_SEGS), so four launches hold all of them.
-//   stage 5   to round 5 if its extents are far from passing (ratio < ROUND_FAR), skipping 2-4 if they
-//             are certified to fail; else, and for the other points,
-//   stage 3   to round 3, certifying round 2 or else searching it (stage 2), then
-//   stage 15  to round 5 if not searched yet, certifying round 4 or else searching it (stage 4).
-// A search's moments are kept when its box passes or in round 5, so the last kept are those of the
-// answer.  Of the room's rejected points (4M points, 25 % rejected, 91 % of them up to round 5) 61 %
-// go to round 5 at once and stop; the later rounds' launches took 14.5 ms of its normals pass, now 9.5.
-struct RoundState {
-    float4* pst;      // per point: largest extent of the last round known to fail, round 5's smallest extent
-                      // (-1: not searched, inf: it passes), round 3's largest extent
-    uint8_t* act;     // per point: the stage to search next, 0 when resolved
-    uint8_t* kround;  // per point: the round of the moments kept (0: none yet)
-    int stage;        // 1, 5, 3, 2, 15 or 4; STAGE_SPEC: one of all rounds searched at once
-    float* smom;      // then per query slot: the moments,
-    uint8_t* sok;     // and whether the box passes
-};
-constexpr float ROUND_EPS = 0.05f;
-// Which points try round 5 first: the cost of the searches (CPU model over the sampled neighbourhoods of
-// the room, the outdoor clouds and single outdoor scans) is flat within 1 % for 0.035-0.045; at 0.05 (all
-// of them) sparse scans lose 1-2 %, at 0 (none) the rooms lose 10 %.
-constexpr float ROUND_FAR = 0.04f;
-
-// Takes the extents (smallest, largest) of a searched round and whether its box passes; returns whether
-// its moments are to be kept.
-__device__ __forceinline__ bool round_decide(const RoundState& rs, uint32_t q, float mn, float mx, bool ok)
-{
-    float4* p = rs.pst + q;
-    int act = 0;
-    bool keep = ok;
-    if (rs.stage == 1) {
-        rs.kround[q] = ok ? 1 : 0;
-        if (!ok) {
-            *p = make_float4(mx, -1.0f, 0.0f, 0.0f);
-            act = mn < ROUND_FAR * mx ? 5 : 3;
-        }
-        rs.act[q] = (uint8_t)act;
-        return keep;
-    }
-    const float4 s = *p;
-    float low = s.x;
-    // round 3 known to fail with largest extent low: what follows
-    auto after3 = [&]() {
-        if (s.y < 0.0f) return 15;
-        return s.y < ROUND_EPS * low ? 0 : 4;  // (inf: round 5 passes, no certificate)
-    };
-    switch (rs.stage) {
-        case 5:
-            keep = true;
-            rs.kround[q] = 5;
-            if (ok || !(mn < ROUND_EPS * low)) {
-                p->y = ok ? INFINITY : mn;
-                act = 3;
-            }
-            break;
-        case 3:
-            if (ok) {
-                rs.kround[q] = 3;
-                act = 2;
-            } else if (mn < ROUND_EPS * low) {
-                p->x = low = mx;
-                act = after3();
-            } else {
-                p->z = mx;
-                act = 2;
-            }
-            break;
-        case 2:
-            if (ok) {
-                rs.kround[q] = 2;
-            } else if (rs.kround[q] != 3) {  // round 3 failed too
-                p->x = low = s.z;
-                act = after3();
-            }
-            break;
-        case 15:
-            keep = true;
-            rs.kround[q] = 5;
-            act = (!ok && mn < ROUND_EPS * low) ? 0 : 4;
-            break;
-        default:  // 4
-            if (ok) rs.kround[q] = 4;
-            break;
-    }
-    rs.act[q] = (uint8_t)act;
-    return keep;
-}
-
 // Fused into the kNN pass: the k-set's bounding box test (boundingBoxOK,
 // AdaptiveKSearchSurface.tcc:337-350) and its moments about the query point; the plane fit
 // itself runs in plane_fit_kernel.  Also the sorted ki-prefix for the interpolation.
@@ -231,8 +137,9 @@ struct SinkNormals {
     static constexpr int kTargets = 2;
     // parameters
     float* mom;            // [qpos * 9] moments of the k-set about q
-    uint32_t* retry;       // per query slot: 1 if the bbox test failed (merged rounds; else NULL)
-    RoundState rs;         // the rounds out of order (rs.act == NULL: merged rounds, or one given round)
+    uint32_t* retry;       // per query slot: 1 if the bbox test failed (NULL in the last round)
+    uint8_t* kround;       // per point: round if the test passed or there is no other (NULL: not kept)
+    int round;
     uint32_t* ki_list;     // out [qpos * kiw + j]: the ki nearest, unordered
     int kiw;
     // per-lane state
@@ -331,14 +238,9 @@ struct SinkNormals {
             const float e = 0.05f;
             const bool bb_ok = dx >= e * dy && dx >= e * dz && dy >= e * dx && dy >= e * dz && dz >= e * dx &&
                                dz >= e * dy;
-            float* m = mom + (size_t)qpos * 9;
-            if (rs.stage == STAGE_SPEC) {
-                rs.sok[qi_] = bb_ok ? 1 : 0;
-                m = rs.smom + (size_t)qi_ * 9;
-            } else if (rs.act &&
-                !round_decide(rs, qpos, fminf(fminf(dx, dy), dz), fmaxf(fmaxf(dx, dy), dz), bb_ok))
-                return;
             if (retry) retry[qi_] = bb_ok ? 0u : 1u;
+            if (kround && (bb_ok || !retry)) kround[qpos] = (uint8_t)round;
+            float* m = mom + (size_t)qpos * 9;
             m[0] = sx;
             m[1] = sy;
             m[2] = sz;

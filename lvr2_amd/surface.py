@@ -200,8 +200,7 @@ class HipSurface:
         return {name: (float(ms[i]), int(cnt[i])) for i, name in enumerate(TIMERS)}
 
     def kernelStats(self, reset: bool = False) -> dict:
-        """Work counters of the kNN tile kernels, per group (collected while profiling); the later rounds
-        share launches, so theirs come together under ``merged_rounds``."""
+        """Work counters of the kNN tile kernels, per group (collected while profiling)."""
         from ._lib import STAT_COUNTERS, STAT_GROUPS
 
         a = np.zeros(16 * len(STAT_GROUPS), np.int64)
@@ -215,7 +214,7 @@ class HipSurface:
         check(lib().lvrhip_set_sdf_tuning(self._h, int(tiles_per_wave), float(r2_margin)))
 
     def setRetryMode(self, merged: bool) -> None:
-        """Adaptive rounds 2..5 in one four-target search (True) or as separate searches of the rounds still open (False)."""
+        """Adaptive rounds 2..5 in one four-target search (True) or round by round (False)."""
         check(lib().lvrhip_set_retry_mode(self._h, int(bool(merged))))
 
     def autotune(self) -> dict:
