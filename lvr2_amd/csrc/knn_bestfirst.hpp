@@ -871,8 +871,9 @@ struct BfCentroidOut {
     uint32_t npts;  // sorted positions
     static constexpr bool kPrefill = true;
 
-    // the t neighbours of the vertex's last search are t points of the cloud: the t-th key is at most the
-    // largest of their keys at the new position
+    // the t neighbours of the vertex's last search are t different points of the cloud (every pass that
+    // resolves a query saves them, the tile kernel's too, or ~0 where it found fewer): the t-th key is at most
+    // the largest of their keys at the new position
     __device__ __forceinline__ uint64_t first_bound(int64_t i, int t, float qx, float qy, float qz,
                                                     uint64_t empty) const
     {

@@ -468,10 +468,11 @@ __global__ void mean_normal_rows_kernel(int64_t m, int k, int t, const int32_t* 
 }
 
 // the centroid of each row's neighbours, for the tile kernel's rows (the input position stays when
-// the row is empty)
+// the row is empty); with vid and nbr the neighbours are saved like BfCentroidOut's
 __global__ void centroid_rows_kernel(int64_t m, int k, const int32_t* __restrict__ idx,
                                      const uint32_t* __restrict__ rank, const float4* __restrict__ pts,
-                                     const float* __restrict__ q, float* __restrict__ out)
+                                     const float* __restrict__ q, const uint32_t* __restrict__ vid,
+                                     uint32_t* __restrict__ nbr, float* __restrict__ out)
 {
     const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (r >= m) return;
@@ -479,6 +480,7 @@ __global__ void centroid_rows_kernel(int64_t m, int k, const int32_t* __restrict
     int nk = 0;
     for (int j = 0; j < k; j++) {
         const int32_t id = idx[(size_t)r * k + j];
+        if (vid && nbr) nbr[(size_t)vid[r] * k + j] = id < 0 ? ~0u : rank[id];
         if (id < 0) continue;
         const float4 p = pts[rank[id]];
         cx += p.x;
@@ -2164,7 +2166,7 @@ struct lvrhip_surface {
     // The centroid of the kc cloud points nearest to each of m device positions (the vertex move
     // of BilinearFastBox::optimizePlanarFaces, BilinearFastBox.tcc:168-204); d_out in caller order.
     // vid / nbr (optional): each query's mesh vertex and, per vertex, the neighbours of its last
-    // search, saved here and, with prefill, the start of this search.
+    // search, saved here by whichever search finds them and, with prefill, the start of this search.
     void centroids_device(const float* d_q, int64_t m, int kc, float* d_out, const uint32_t* vid = nullptr,
                           uint32_t* nbr = nullptr, bool prefill = false)
     {
@@ -2189,7 +2191,8 @@ struct lvrhip_surface {
             throw;
         }
         search_mode = saved;
-        centroid_rows_kernel<<<(unsigned)ceil_div(m, 256), 256, 0, st>>>(m, t0, idx.p, rank.p, pts4.p, d_q, d_out);
+        centroid_rows_kernel<<<(unsigned)ceil_div(m, 256), 256, 0, st>>>(m, t0, idx.p, rank.p, pts4.p, d_q, vid, nbr,
+                                                                          d_out);
         LVRHIP_LAUNCH_CHECK();
         LVRHIP_CHECK(hipStreamSynchronize(st));
     }
