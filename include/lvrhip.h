@@ -100,8 +100,16 @@ int lvrhip_graph_capture(lvrhip_t h, float* d_out_normals, int rebuild);
 int lvrhip_graph_launch(lvrhip_t h);
 int lvrhip_synchronize(lvrhip_t h);
 
-/* Replaces ~CudaSurface / CudaSurface::freeGPU (CudaSurface.cu:1259-1264). */
+/* Replaces ~CudaSurface / CudaSurface::freeGPU (CudaSurface.cu:1259-1264).  Waits for the device.  The handle's
+ * device memory is kept for the next handles and calls, at most 2 GiB per device, until 64 later
+ * destructions or host-array calls have not used it, an allocation of the library fails, or
+ * lvrhip_release_memory gives it back. */
 int lvrhip_destroy(lvrhip_t h);
+
+/* Gives the device memory that the library keeps between calls back to the runtime: of one device, or of all
+ * (device -1).  For programs that are done with their surfaces, or whose other allocators need the
+ * memory; live handles keep theirs.  *bytes (may be NULL) = how much it was.  No lvr2 counterpart. */
+int lvrhip_release_memory(int device, size_t* bytes);
 
 /* Replaces CudaSurface::setKn/setKi/setKd (CudaSurface.hpp:116-142) and
  * PointsetSurface::setKn/setKi/setKd (PointsetSurface.hpp:112-126).  ki == 0 disables

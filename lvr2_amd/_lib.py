@@ -16,6 +16,7 @@ _SIGS = {
     "lvrhip_create": (C.c_int, [C.c_void_p, C.c_size_t, C.c_int, C.POINTER(C.c_void_p)]),
     "lvrhip_create_device": (C.c_int, [C.c_void_p, C.c_size_t, C.c_int, C.c_void_p, C.POINTER(C.c_void_p)]),
     "lvrhip_destroy": (C.c_int, [C.c_void_p]),
+    "lvrhip_release_memory": (C.c_int, [C.c_int, C.POINTER(C.c_size_t)]),
     "lvrhip_set_k": (C.c_int, [C.c_void_p, C.c_int, C.c_int, C.c_int]),
     "lvrhip_set_flip_point": (C.c_int, [C.c_void_p, C.c_float, C.c_float, C.c_float]),
     "lvrhip_set_method": (C.c_int, [C.c_void_p, C.c_int]),
@@ -119,3 +120,11 @@ def check(rc: int) -> None:
     if rc != 0:
         msg = lib().lvrhip_last_error().decode(errors="replace")
         raise LvrHipError(rc, msg)
+
+
+def release_memory(device: int = -1) -> int:
+    """Give the device memory that the library keeps for the next surfaces and calls (at most 2 GiB per
+    device) back to the runtime, of one device or of all (-1); returns the bytes.  Live surfaces keep theirs."""
+    n = C.c_size_t()
+    check(lib().lvrhip_release_memory(int(device), C.byref(n)))
+    return n.value

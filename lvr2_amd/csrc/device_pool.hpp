@@ -7,8 +7,11 @@
 //    device's work on it (IdleScope); freed anywhere else it goes back to the runtime.  One mutex
 //    guards the lists.
 //  - Bounded: at most CACHE_BYTES per device, no block above a quarter of that.
-//  - Given back: blocks that no allocation took over the last KEEP handle destructions are freed, and all of a
-//    device's blocks when one of its allocations fails (which is then tried again).
+//  - Given back: blocks that no allocation took over the last KEEP calls that return blocks (host-array calls and
+//    handle destructions, on any device) are freed, all of a device's blocks when one of its
+//    allocations fails (which is then tried again), and all there are by release() (lvrhip_release_memory).
+//    Not with the last handle: one surface after the other, each destroyed before the next, is what the
+//    pool is for.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -25,9 +28,10 @@ namespace lvrhip {
 class DevicePool {
 public:
     static constexpr size_t CACHE_BYTES = (size_t)2 << 30;
-    static constexpr uint64_t KEEP = 16;
+    static constexpr uint64_t KEEP = 64;
     static constexpr size_t PINNED_BYTES = 64;
     static constexpr size_t PINNED_KEPT = 64;
+    static constexpr int ALL = -1;
 
     static DevicePool& get()
     {
@@ -89,18 +93,19 @@ public:
         if (!keep) (void)hipFree(p);
     }
 
-    // a handle was destroyed on the current device: what nobody took for KEEP of these is freed
+    // a call returned its blocks: what nobody took for KEEP of these is freed
     void tick()
     {
-        int dev = 0;
-        if (hipGetDevice(&dev) != hipSuccess) return;
         uint64_t t;
         {
             std::lock_guard<std::mutex> lk(mu_);
             t = ++now_;
         }
-        if (t > KEEP) trim(dev, t - KEEP);
+        if (t > KEEP) trim(ALL, t - KEEP);
     }
+
+    // frees all that is kept for a device (ALL: for every one); returns the bytes
+    size_t release(int dev) { return trim(dev, ~0ull); }
 
     // pinned host words for readbacks
     hipError_t alloc_pinned(uint32_t** p)
@@ -146,32 +151,37 @@ private:
         return (bytes + step - 1) / step * step;
     }
 
-    // frees the device's kept blocks that were freed before `before`
-    void trim(int dev, uint64_t before)
+    // frees the kept blocks of a device (ALL: of every one) that were freed before `before`; returns the bytes
+    size_t trim(int dev, uint64_t before)
     {
         std::vector<void*> out;
+        size_t bytes = 0;
         {
             std::lock_guard<std::mutex> lk(mu_);
-            auto& c = cache_[dev];
-            for (auto& [size, v] : c.blocks) {
-                size_t w = 0;
-                for (auto& b : v) {
-                    if (b.second < before) {
-                        out.push_back(b.first);
-                        c.bytes -= size;
-                    } else {
-                        v[w++] = b;
+            for (auto& [d, c] : cache_) {
+                if (dev != ALL && d != dev) continue;
+                for (auto& [size, v] : c.blocks) {
+                    size_t w = 0;
+                    for (auto& b : v) {
+                        if (b.second < before) {
+                            out.push_back(b.first);
+                            c.bytes -= size;
+                            bytes += size;
+                        } else {
+                            v[w++] = b;
+                        }
                     }
+                    v.resize(w);
                 }
-                v.resize(w);
             }
         }
         for (void* p : out) (void)hipFree(p);
+        return bytes;
     }
 };
 
 // While one is set on a thread, the blocks that the thread frees are known to be idle: set it after waiting
-// for all work on them.
+// for all work on them.  Its end is a call's end for the pool (tick).
 struct IdleScope {
     bool on = false;
     static bool& flag()
@@ -186,7 +196,9 @@ struct IdleScope {
     }
     ~IdleScope()
     {
-        if (on) flag() = false;
+        if (!on) return;
+        flag() = false;
+        DevicePool::get().tick();
     }
 };
 

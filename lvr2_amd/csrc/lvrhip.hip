@@ -2358,7 +2358,15 @@ int lvrhip_destroy(lvrhip_t h)
         IdleScope idle;  // the handle may have worked on several streams
         if (hipDeviceSynchronize() == hipSuccess) idle.set();
         delete h;
-        DevicePool::get().tick();
+    });
+}
+
+int lvrhip_release_memory(int device, size_t* bytes)
+{
+    return guarded([&] {
+        REQUIRE(device >= -1, "device must be -1 (all) or a device's number");
+        const size_t freed = DevicePool::get().release(device);
+        if (bytes) *bytes = freed;
     });
 }
 
