@@ -51,10 +51,10 @@ public:
             auto& c = cache_[dev];
             auto it = c.blocks.find(size);
             if (it != c.blocks.end() && !it->second.empty()) {
+                live_[it->second.back().first] = {dev, size};
                 *p = it->second.back().first;
                 it->second.pop_back();
                 c.bytes -= size;
-                live_[*p] = {dev, size};
                 return hipSuccess;
             }
         }
@@ -67,16 +67,22 @@ public:
             e = hipMalloc(p, bytes);
         }
         if (e != hipSuccess) return e;
-        std::lock_guard<std::mutex> lk(mu_);
-        live_[*p] = {dev, got};
+        try {
+            std::lock_guard<std::mutex> lk(mu_);
+            live_[*p] = {dev, got};
+        } catch (...) {
+            (void)hipFree(*p);
+            throw;
+        }
         return hipSuccess;
     }
 
-    // idle: no work of any stream on the block is left
-    void free(void* p, bool idle)
+    // idle: no work of any stream on the block is left.  Runs in destructors: a block that the lists have no host
+    // memory for goes back to the runtime.
+    void free(void* p, bool idle) noexcept
     {
         bool keep = false;
-        {
+        try {
             std::lock_guard<std::mutex> lk(mu_);
             auto it = live_.find(p);
             if (it != live_.end()) {
@@ -89,12 +95,13 @@ public:
                     keep = true;
                 }
             }
+        } catch (...) {
         }
         if (!keep) (void)hipFree(p);
     }
 
     // a call returned its blocks: what nobody took for KEEP of these is freed
-    void tick()
+    void tick() noexcept
     {
         uint64_t t;
         {
@@ -105,7 +112,7 @@ public:
     }
 
     // frees all that is kept for a device (ALL: for every one); returns the bytes
-    size_t release(int dev) { return trim(dev, ~0ull); }
+    size_t release(int dev) noexcept { return trim(dev, ~0ull); }
 
     // pinned host words for readbacks
     hipError_t alloc_pinned(uint32_t** p)
@@ -120,14 +127,15 @@ public:
         }
         return hipHostMalloc(reinterpret_cast<void**>(p), PINNED_BYTES, hipHostMallocPortable);
     }
-    void free_pinned(uint32_t* p, bool idle)
+    void free_pinned(uint32_t* p, bool idle) noexcept
     {
-        if (idle) {
+        try {
             std::lock_guard<std::mutex> lk(mu_);
-            if (pinned_.size() < PINNED_KEPT) {
+            if (idle && pinned_.size() < PINNED_KEPT) {
                 pinned_.push_back(p);
                 return;
             }
+        } catch (...) {
         }
         (void)hipHostFree(p);
     }
@@ -152,31 +160,30 @@ private:
     }
 
     // frees the kept blocks of a device (ALL: of every one) that were freed before `before`; returns the bytes
-    size_t trim(int dev, uint64_t before)
+    size_t trim(int dev, uint64_t before) noexcept
     {
-        std::vector<void*> out;
         size_t bytes = 0;
-        {
-            std::lock_guard<std::mutex> lk(mu_);
-            for (auto& [d, c] : cache_) {
-                if (dev != ALL && d != dev) continue;
-                for (auto& [size, v] : c.blocks) {
-                    size_t w = 0;
-                    for (auto& b : v) {
-                        if (b.second < before) {
-                            out.push_back(b.first);
-                            c.bytes -= size;
-                            bytes += size;
-                        } else {
-                            v[w++] = b;
-                        }
-                    }
-                    v.resize(w);
+        while (void* p = take_kept(dev, before, bytes)) (void)hipFree(p);
+        return bytes;
+    }
+    void* take_kept(int dev, uint64_t before, size_t& bytes) noexcept
+    {
+        std::lock_guard<std::mutex> lk(mu_);
+        for (auto& [d, c] : cache_) {
+            if (dev != ALL && d != dev) continue;
+            for (auto& [size, v] : c.blocks) {
+                for (auto& b : v) {
+                    if (b.second >= before) continue;
+                    void* p = b.first;
+                    b = v.back();
+                    v.pop_back();
+                    c.bytes -= size;
+                    bytes += size;
+                    return p;
                 }
             }
         }
-        for (void* p : out) (void)hipFree(p);
-        return bytes;
+        return nullptr;
     }
 };
 

@@ -12,6 +12,7 @@ RUNTIME = r'''
 #include <cstddef>
 #include <cstdlib>
 #include <map>
+extern bool no_memory;
 enum hipError_t { hipSuccess = 0, hipErrorOutOfMemory = 2 };
 enum { hipHostMallocPortable = 1 };
 struct Runtime {
@@ -23,7 +24,8 @@ inline Runtime& rt() { static Runtime r; return r; }
 inline hipError_t hipGetDevice(int* d) { *d = rt().dev; return hipSuccess; }
 inline hipError_t hipMalloc(void** p, size_t n) {
     static char* next = reinterpret_cast<char*>(4096);  // addresses only
-    *p = next; next += 4096; rt().held[*p] = {rt().dev, n}; return hipSuccess; }
+    const bool m = no_memory; no_memory = false;  // the runtime's own
+    *p = next; next += 4096; rt().held[*p] = {rt().dev, n}; no_memory = m; return hipSuccess; }
 inline hipError_t hipFree(void* p) { if (!rt().held.erase(p)) std::abort(); return hipSuccess; }
 inline hipError_t hipGetLastError() { return hipSuccess; }
 inline hipError_t hipHostMalloc(void** p, size_t n, unsigned) { *p = std::malloc(n); return hipSuccess; }
@@ -33,6 +35,13 @@ inline hipError_t hipHostFree(void* p) { std::free(p); return hipSuccess; }
 PROG = r'''
 #include "device_pool.hpp"
 #include <cstdio>
+#include <new>
+bool no_memory = false;
+void* operator new(size_t n) {
+    if (no_memory) throw std::bad_alloc();
+    return std::malloc(n); }
+void operator delete(void* p) noexcept { std::free(p); }
+void operator delete(void* p, size_t) noexcept { std::free(p); }
 using lvrhip::DevicePool;
 using lvrhip::IdleScope;
 #define CHECK(c) do { if (!(c)) { std::printf("line %d: %s\n", __LINE__, #c); return 1; } } while (0)
@@ -77,6 +86,29 @@ int main(int argc, char** argv) {
             CHECK(pool().release(1) == 7 * MB && rt().held.empty());
             return 0;
         }
+        case 'h': {  // no host memory: blocks go back to the runtime, and nothing throws where nothing may
+            call(6 * MB);
+            void* p = take(2 * MB);
+            const size_t held = rt().held.size();
+            no_memory = true;
+            pool().free(p, true);
+            CHECK(rt().held.size() == held - 1);
+            pool().tick();
+            uint32_t* w = nullptr;
+            CHECK(pool().alloc_pinned(&w) == hipSuccess);
+            pool().free_pinned(w, true);
+            bool thrown = false;
+            try {
+                take(MB);
+            } catch (const std::bad_alloc&) {
+                thrown = true;
+            }
+            CHECK(thrown && rt().held.size() == held - 1);
+            CHECK(pool().release(0) == 6 * MB);
+            no_memory = false;
+            CHECK(rt().held.empty());
+            return 0;
+        }
         case 'b': {  // bounded
             for (int i = 0; i < 20; i++) {
                 IdleScope s;
@@ -107,7 +139,7 @@ def exe(tmp_path_factory):
     return str(d / "pool")
 
 
-@pytest.mark.parametrize("what", ["kept", "aged", "released", "bounded"])
+@pytest.mark.parametrize("what", ["kept", "aged", "released", "host memory", "bounded"])
 def test_pool(exe, what):
     r = subprocess.run([exe, what], capture_output=True, text=True, timeout=60,
                        env=dict(os.environ, ASAN_OPTIONS="detect_leaks=0"))
