@@ -28,6 +28,7 @@ namespace lvrhip {
 class DevicePool {
 public:
     static constexpr size_t CACHE_BYTES = (size_t)2 << 30;
+    static constexpr size_t KEPT_BLOCK = CACHE_BYTES / 4;  // the largest block kept
     static constexpr uint64_t KEEP = 64;
     static constexpr size_t PINNED_BYTES = 64;
     static constexpr size_t PINNED_KEPT = 64;
@@ -89,7 +90,7 @@ public:
                 const auto [dev, size] = it->second;
                 live_.erase(it);
                 auto& c = cache_[dev];
-                if (idle && size == size_class(size) && size <= CACHE_BYTES / 4 && c.bytes + size <= CACHE_BYTES) {
+                if (idle && size == size_class(size) && size <= KEPT_BLOCK && c.bytes + size <= CACHE_BYTES) {
                     c.blocks[size].emplace_back(p, now_);
                     c.bytes += size;
                     keep = true;
@@ -151,10 +152,12 @@ private:
     std::vector<uint32_t*> pinned_;
     uint64_t now_ = 0;
 
-    // sizes in steps of an eighth of the power of two below (at most 12.5 % more than asked for)
+    // sizes in steps of an eighth of the power of two below (at most 12.5 % more than asked for); a block too
+    // large to be kept has just the size asked for
     static size_t size_class(size_t bytes)
     {
         if (bytes <= 4096) return 4096;
+        if (bytes > KEPT_BLOCK) return bytes;
         const size_t step = ((size_t)1 << (63 - __builtin_clzll(bytes))) / 8;
         return (bytes + step - 1) / step * step;
     }

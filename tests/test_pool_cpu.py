@@ -109,6 +109,20 @@ int main(int argc, char** argv) {
             CHECK(rt().held.empty());
             return 0;
         }
+        case 'e': {  // what is too large to be kept is allocated as asked for, however large
+            const size_t sizes[] = {512 * MB + 1, 700 * MB + 5, ~(size_t)0 - 7};
+            for (size_t n : sizes) {
+                void* p = take(n);
+                CHECK(rt().held[p].second == n);
+                pool().free(p, true);
+                CHECK(rt().held.empty());
+            }
+            void* p = take(512 * MB - 1);
+            CHECK(rt().held[p].second >= 512 * MB - 1 && rt().held[p].second <= 512 * MB);
+            pool().free(p, true);
+            CHECK(rt().held.size() == 1);
+            return 0;
+        }
         case 'b': {  // bounded
             for (int i = 0; i < 20; i++) {
                 IdleScope s;
@@ -139,7 +153,7 @@ def exe(tmp_path_factory):
     return str(d / "pool")
 
 
-@pytest.mark.parametrize("what", ["kept", "aged", "released", "host memory", "bounded"])
+@pytest.mark.parametrize("what", ["kept", "aged", "released", "host memory", "exact", "bounded"])
 def test_pool(exe, what):
     r = subprocess.run([exe, what], capture_output=True, text=True, timeout=60,
                        env=dict(os.environ, ASAN_OPTIONS="detect_leaks=0"))
