@@ -100,8 +100,8 @@ int lvrhip_graph_capture(lvrhip_t h, float* d_out_normals, int rebuild);
 int lvrhip_graph_launch(lvrhip_t h);
 int lvrhip_synchronize(lvrhip_t h);
 
-/* Replaces ~CudaSurface / CudaSurface::freeGPU (CudaSurface.cu:1259-1264).  Waits for the device.  The handle's
- * device memory is kept for the next handles and calls, at most 2 GiB per device, until 64 later
+/* Replaces ~CudaSurface / CudaSurface::freeGPU (CudaSurface.cu:1259-1264).  Waits for the handle's stream.  Its
+ * device memory (unless the handle was moved between streams) is kept for the next handles and calls, at most 2 GiB per device, until 64 later
  * destructions or host-array calls have not used it, an allocation of the library fails, or
  * lvrhip_release_memory gives it back. */
 int lvrhip_destroy(lvrhip_t h);

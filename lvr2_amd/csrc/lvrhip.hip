@@ -753,6 +753,14 @@ struct lvrhip_surface {
 
     hipStream_t gst = nullptr;  // private stream for graphs when the handle's stream is the null stream
     bool own_gst = false;
+    // streams other than st and gst may have work on the handle's memory: it was moved from one to another, or a
+    // caller's capture recorded work on it (the calls that enqueue without waiting note that)
+    bool elsewhere = false;
+    void note_capture()
+    {
+        hipStreamCaptureStatus s = hipStreamCaptureStatusNone;
+        if (st && hipStreamIsCapturing(st, &s) == hipSuccess && s != hipStreamCaptureStatusNone) elsewhere = true;
+    }
     hipGraph_t graph = nullptr;
     hipGraphExec_t gexec = nullptr;
     hipStream_t graph_stream = nullptr;
@@ -2355,8 +2363,12 @@ int lvrhip_destroy(lvrhip_t h)
     return guarded([&] {
         if (!h) return;
         DeviceGuard dg(h->device);
-        IdleScope idle;  // the handle may have worked on several streams
-        if (hipDeviceSynchronize() == hipSuccess) idle.set();
+        // Not a wait for the device: that ends a capture which another stream is in, where these waits (and
+        // hipFree, in a relaxed capture) do not.
+        IdleScope idle;
+        const bool done = hipStreamSynchronize(h->st) == hipSuccess;
+        const bool graph_done = !h->gst || hipStreamSynchronize(h->gst) == hipSuccess;
+        if (done && graph_done && !h->elsewhere) idle.set();
         delete h;
     });
 }
@@ -2409,6 +2421,7 @@ int lvrhip_set_stream(lvrhip_t h, void* stream)
 {
     return guarded([&] {
         REQUIRE(h, "NULL handle");
+        if (h->st != (hipStream_t)stream) h->elsewhere = true;
         h->st = (hipStream_t)stream;
     });
 }
@@ -2427,6 +2440,7 @@ int lvrhip_interpolate_normals(lvrhip_t h)
     return guarded([&] {
         REQUIRE(h, "NULL handle");
         DeviceGuard dg(h->device);
+        h->note_capture();
         h->interpolate_normals();
     });
 }
@@ -2469,6 +2483,7 @@ int lvrhip_get_normals_device(lvrhip_t h, float* d_out)
         if (h->n == 0) return;
         REQUIRE(d_out, "output pointer is NULL");
         DeviceGuard dg(h->device);
+        h->note_capture();
         h->scatter_normals(h->nx.p, h->ny.p, h->nz.p, d_out);
     });
 }
@@ -2700,6 +2715,7 @@ int lvrhip_grid_get_device(lvrhip_t h, float* d_vertices, int32_t* d_cells, int3
     return guarded([&] {
         REQUIRE(h, "NULL handle");
         DeviceGuard dg(h->device);
+        h->note_capture();
         if (d_vertices && h->grid_nv)
             LVRHIP_CHECK(hipMemcpyAsync(d_vertices, h->grid_vtx.p, 3 * (size_t)h->grid_nv * sizeof(float),
                                         hipMemcpyDeviceToDevice, h->st));
@@ -2779,6 +2795,7 @@ int lvrhip_mesh_get_device(lvrhip_t h, float* d_vertices, int32_t* d_faces)
     return guarded([&] {
         REQUIRE(h, "NULL handle");
         DeviceGuard dg(h->device);
+        h->note_capture();
         if (d_vertices && h->mesh_nv)
             LVRHIP_CHECK(hipMemcpyAsync(d_vertices, h->mesh_vtx.p, 3 * (size_t)h->mesh_nv * sizeof(float),
                                         hipMemcpyDeviceToDevice, h->st));
@@ -2931,6 +2948,7 @@ int lvrhip_graph_launch(lvrhip_t h)
     return guarded([&] {
         REQUIRE(h, "NULL handle");
         DeviceGuard dg(h->device);
+        h->note_capture();
         h->graph_launch();
     });
 }
