@@ -101,9 +101,9 @@ int lvrhip_graph_launch(lvrhip_t h);
 int lvrhip_synchronize(lvrhip_t h);
 
 /* Replaces ~CudaSurface / CudaSurface::freeGPU (CudaSurface.cu:1259-1264).  Waits for the handle's stream.  Its
- * device memory (unless the handle was moved between streams) is kept for the next handles and calls, at most 2 GiB per device, until 64 later
- * destructions or host-array calls have not used it, an allocation of the library fails, or
- * lvrhip_release_memory gives it back. */
+ * device memory (unless the handle was moved between streams) is kept for the next handles and
+ * calls, at most 2 GiB per device, until 64 later destructions or host-array calls have not used
+ * it, an allocation of the library fails, or lvrhip_release_memory gives it back. */
 int lvrhip_destroy(lvrhip_t h);
 
 /* Gives the device memory that the library keeps between calls back to the runtime: of one device, or of all
@@ -179,8 +179,9 @@ int lvrhip_interpolated_normals(lvrhip_t h, const float* q, size_t m, float* out
 
 /* Search algorithm of the searches with at most 32 neighbours (distances, kSearch, radius
  * search, interpolated normals at positions); no lvr2 counterpart.  LVRHIP_SEARCH_AUTO (the
- * default) runs them best-first, one lane per query; the queries whose pool of subtrees overflows
- * are searched again by one wave each, and any that outgrow that by the tile kernel.
+ * default) runs them best-first, one lane per query (a batch of at most 1,024 queries one wave
+ * per query); the queries whose pool of subtrees overflows are searched again by one wave each,
+ * and any that outgrow that by the tile kernel.
  * LVRHIP_SEARCH_TILE forces the tile kernel, LVRHIP_SEARCH_WAVE the wave-per-query search for
  * every query.  All give identical results. */
 enum { LVRHIP_SEARCH_AUTO = 0, LVRHIP_SEARCH_TILE = 1, LVRHIP_SEARCH_WAVE = 2 };

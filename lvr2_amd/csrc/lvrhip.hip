@@ -505,8 +505,7 @@ __global__ void centroid_rows_kernel(int64_t m, int k, const int32_t* __restrict
 // Query coordinates: SoA (qs = 1) or AoS (qs = 3, qy = qx + 1, qz = qx + 2).  With a queue the
 // grid is min(chunks, resident) waves; spill holds spill_cap entries per searching lane of each of them.
 // Queries per wave: 64 fills the lanes, but a small batch runs on more waves with fewer lanes each, which
-// wait less for each other: 500 queries (t = 10) take 100 us, by the wave search, which took them before,
-// 137 us, and at t = 32 a quarter of its time.
+// wait less for each other.
 inline int bf_per_wave(int64_t m, int64_t resident)
 {
     int p = 64;
@@ -1572,7 +1571,7 @@ struct lvrhip_surface {
         s_hist.reserve(rs_hist_size(m));
         const unsigned gb = (unsigned)ceil_div(m, 256);
         // of the 63-bit code (its top 32 bits are cells of 1/1,600 of the box per axis)
-        const int bits = !lanes ? 32 : bf_per_wave(m, bf_resident) == 1 ? 0 : m <= (1 << 16) ? 16 : m <= (1 << 21) ? 24 : 32;
+        const int bits = !lanes ? 32 : wave_batch(m) || bf_per_wave(m, bf_resident) == 1 ? 0 : m <= (1 << 16) ? 16 : m <= (1 << 21) ? 24 : 32;
         const bool odd = rs_passes(bits) & 1;  // the sort then starts from its other buffers
         morton_queries_kernel<<<gb, 256, 0, st>>>(d_q, m, frames.p, odd ? s_k1.p : s_k0.p, odd ? s_v1.p : s_v0.p);
         LVRHIP_LAUNCH_CHECK();
@@ -2081,10 +2080,19 @@ struct lvrhip_surface {
         prof.collect();
     }
 
+    // A batch that gives every query a wave of its own is searched by waves at once.  500 queries near a surface are
+    // done sooner by lanes (t = 10: 100 us of 137), but a lane takes the leaves one after the other: where
+    // a query sees hundreds of them at almost one distance (the inside of a sphere, a curved cloud from
+    // afar) 500 took 0.5 to 1.1 ms by lanes, 0.3 ms by waves.
+    bool wave_batch(int64_t m) const
+    {
+        return search_mode == LVRHIP_SEARCH_WAVE || (search_mode == LVRHIP_SEARCH_AUTO && m <= BF_WAVE_BLOCKS);
+    }
+
     bool best_first(int t) const { return search_mode != LVRHIP_SEARCH_TILE && t >= 1 && t <= BF_KMAX; }
 
-    // Best-first search of the m sorted queries s_q*: one lane per query for all of them, then one
-    // wave per query for those whose lane pool overflowed; the queries both left end up in
+    // Best-first search of the m sorted queries s_q*: one lane per query for all of them (not in a wave_batch),
+    // then one wave per query for those whose lane pool overflowed; the queries both left end up in
     // s_left2[0, *counter(8)), for the tile kernel.  Enqueue only: three launches.
     template <class Out>
     void enqueue_bf(int64_t m, int t0, uint64_t empty, const Out& o, int stats_group)
@@ -2094,7 +2102,7 @@ struct lvrhip_surface {
         d_queue.reserve((size_t)QUEUES * QUEUE_SEGS * QUEUE_STRIDE);
         bf_reset_kernel<<<1, 256, 0, st>>>(d_queue.p, QUEUE_SEGS * QUEUE_STRIDE, counter(13), counter(8));
         LVRHIP_LAUNCH_CHECK();
-        const bool lanes = search_mode != LVRHIP_SEARCH_WAVE;
+        const bool lanes = !wave_batch(m);
         if (lanes) {
             uint32_t* q = use_queue ? d_queue.p : nullptr;
             // one spill area per searching lane of the grid
