@@ -313,8 +313,12 @@ enum {
     LVRHIP_T_COUNT = 7
 };
 int lvrhip_set_profiling(lvrhip_t h, int on);
+/* Whether profiling collects the work counters below too (the default).  The kernels that keep them use more
+ * registers and read the clock; with 0 the timers are those of the kernels that run without
+ * profiling. */
+int lvrhip_set_counters(lvrhip_t h, int on);
 
-/* Kernel work counters collected while profiling is on (no lvr2 counterpart):
+/* Kernel work counters collected while profiling is on (no lvr2 counterpart; lvrhip_set_counters):
  * out[g * 16 + c] for group g (0..4 the normals' adaptive rounds 1..5, 5 the merged later
  * rounds and the wave-per-query pass of the signed distances, 6 SDF, 7 other searches:
  * kSearch, the ki list, the adjoint) and counter c (0 tiles,

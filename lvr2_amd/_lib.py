@@ -34,6 +34,7 @@ _SIGS = {
     "lvrhip_normals_stats": (C.c_int, [C.c_void_p, C.POINTER(C.c_int64)]),
     "lvrhip_size": (C.c_int, [C.c_void_p, C.POINTER(C.c_size_t)]),
     "lvrhip_set_profiling": (C.c_int, [C.c_void_p, C.c_int]),
+    "lvrhip_set_counters": (C.c_int, [C.c_void_p, C.c_int]),
     "lvrhip_get_timings": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_int]),
     "lvrhip_get_kernel_stats": (C.c_int, [C.c_void_p, C.c_void_p, C.c_int]),
     "lvrhip_set_tuning": (C.c_int, [C.c_void_p, C.c_int, C.c_int, C.c_float]),

@@ -563,6 +563,7 @@ void launch_bf_wave(const BvhView& bv, const float* qx, const float* qy, const f
 // hipEvent pairs around kernels on the handle's stream, accumulated per timer.
 struct Profiler {
     bool on = false;
+    bool counters = true;  // while on: the kernels that keep work counters are launched
     double ms[LVRHIP_T_COUNT] = {};
     int64_t launches[LVRHIP_T_COUNT] = {};
     struct Open {
@@ -776,7 +777,7 @@ struct lvrhip_surface {
 
     unsigned long long* kstats_ptr(int group)
     {
-        if (!prof.on) return nullptr;
+        if (!prof.on || !prof.counters) return nullptr;
         if (!kstats.p) {
             kstats.reserve(KS_GROUPS * KS_COUNT);
             LVRHIP_CHECK(hipMemsetAsync(kstats.p, 0, KS_GROUPS * KS_COUNT * sizeof(unsigned long long), st));
@@ -2843,6 +2844,14 @@ int lvrhip_set_profiling(lvrhip_t h, int on)
         DeviceGuard dg(h->device);
         h->prof.collect();
         h->prof.on = on != 0;
+    });
+}
+
+int lvrhip_set_counters(lvrhip_t h, int on)
+{
+    return guarded([&] {
+        REQUIRE(h, "NULL handle");
+        h->prof.counters = on != 0;
     });
 }
 

@@ -186,7 +186,10 @@ class HipSurface:
         check(lib().lvrhip_get_normals(self._h, res.ctypes.data_as(C.c_void_p)))
         return res
 
-    def setProfiling(self, on: bool = True) -> None:
+    def setProfiling(self, on: bool = True, counters: bool = True) -> None:
+        """Timers and, with counters, the work counters of ``kernelStats`` (kept by kernels of their own,
+        which are a little slower than the ones that run without)."""
+        check(lib().lvrhip_set_counters(self._h, int(bool(counters))))
         check(lib().lvrhip_set_profiling(self._h, int(bool(on))))
 
     def timings(self, reset: bool = False) -> dict:
