@@ -212,7 +212,7 @@ int lvrhip_distances_device(lvrhip_t h, const float* d_q, size_t m, float voxel,
  * lvrhip_grid_build, run fastest).  Synchronises the handle's stream; a query whose search
  * outgrows the stacks (never seen in practice) is reported as LVRHIP_ECAPACITY. */
 #define LVRHIP_NOALLOC_MAX_QUERIES 1048576
-#define LVRHIP_NOALLOC_SCRATCH_BYTES 25167872
+#define LVRHIP_NOALLOC_SCRATCH_BYTES 25166592
 int lvrhip_distances_device_noalloc(lvrhip_t h, const float* d_q, size_t m, float voxel, float* d_proj,
                                     float* d_eucl, uint8_t* d_invalid);
 

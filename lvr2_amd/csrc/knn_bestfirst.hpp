@@ -356,7 +356,7 @@ struct bf_prefills<O, std::void_t<decltype(O::kPrefill)>> : std::integral_consta
 
 // stats (optional, KS_* counters of knn_tile.hpp): waves (KS_TILES), the largest leaf count of a
 // lane summed over waves (KS_ATTEMPTS: a wave runs as long as its slowest lane), points scanned
-// (KS_CANDIDATES), nodes expanded (KS_POPS), queries left to the tile kernel (KS_REFINE),
+// (KS_CANDIDATES), nodes expanded (KS_POPS), queries left to the next pass (KS_REFINE),
 // queries resolved (KS_RESOLVED), shader-clock cycles per wave (KS_CY_TOTAL).
 template <int K, class Out>
 __device__ __forceinline__ void bf_stats(unsigned long long* stats, bool valid, bool ok, int leaves, int nodes,
@@ -382,13 +382,8 @@ __device__ __forceinline__ void bf_stats(unsigned long long* stats, bool valid, 
     }
 }
 
-// stats (optional, KS_* counters of knn_tile.hpp): waves (KS_TILES), the largest leaf count of a
-// lane summed over waves (KS_ATTEMPTS: a wave runs as long as its slowest lane), points scanned
-// (KS_CANDIDATES), nodes expanded (KS_POPS), queries left to the next pass (KS_REFINE),
-// queries resolved (KS_RESOLVED), shader-clock cycles per wave (KS_CY_TOTAL).
-//
 // One lane per query (queries in Morton order), chunks of per_wave (at most 64) consecutive queries per
-// wave: fewer for a small batch (bf_per_wave).  With
+// wave: fewer for a smaller batch (bf_per_wave).  With
 // a work queue (QUEUE_SEGS counters QUEUE_STRIDE apart, zeroed before the launch; the grid is
 // then the waves the device holds at once) the chunks are dealt like the tile kernel's runs:
 // blocks of QUEUE_CHUNK consecutive chunks to the XCDs in turn, each XCD taking from its own
@@ -443,14 +438,6 @@ __global__ __launch_bounds__(BF_THREADS) void bf_knn_kernel(const BvhView bv, co
     }
 }
 
-// Wave-cooperative best-first search for the queries list[0, *count) (list NULL: all of them): the ones whose lane search
-// overflowed its stack (a very dense or a far-off neighbourhood, hundreds of leaves deep).  One
-// wave per query: a greedy descent to a seed leaf; then every step pops up to 64 stack entries
-// at once, the lanes expand their nodes (children within the bound pushed) or scan their leaves,
-// and the t smallest keys of the list and the scanned points are extracted by t rounds of a
-// wave-wide minimum.  Lane j holds the j-th key of the list in a register.  The serial chain is
-// the tree depth plus leaves / 64 steps, not one step per node or leaf.  A query whose stack
-// outgrows BF_WAVE_STACK entries is flagged for the tile kernel.
 // Zeroes a search's work queue and the counts of the queries its passes leave.
 static __global__ void bf_reset_kernel(uint32_t* queue, int n, uint32_t* count1, uint32_t* count2)
 {
@@ -473,6 +460,15 @@ __device__ __forceinline__ uint64_t wave_min_u64(uint64_t v)
     return v;
 }
 
+// Wave-cooperative best-first search for the queries list[0, *count) (list NULL: all of them, a
+// small batch): the ones
+// whose lane pool overflowed (a very dense or a far-off neighbourhood, hundreds of leaves deep).  One
+// wave per query: a greedy descent to a seed leaf; then every step pops up to 64 stack entries
+// at once, the lanes expand their nodes (children within the bound pushed) or scan their leaves,
+// and the t smallest keys of the list and the scanned points are extracted by t rounds of a
+// wave-wide minimum.  Lane j holds the j-th key of the list in a register.  The serial chain is
+// the tree depth plus leaves / 64 steps, not one step per node or leaf.  A query whose stack
+// outgrows BF_WAVE_STACK entries is left to the tile kernel.
 template <int K, class Out>
 __global__ __launch_bounds__(BF_THREADS) void bf_knn_wave_kernel(const BvhView bv, const float* __restrict__ qx,
                                                                  const float* __restrict__ qy,

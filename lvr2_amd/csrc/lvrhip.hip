@@ -624,7 +624,7 @@ struct Profiler {
 // Its scratch lives in one file-scope device array, `scratch`, that every device holds from the
 // moment the library's code object is loaded until the process ends.  Layout (byte offsets):
 // the lists of the queries the lane search and the wave search left (NA_MAX_QUERIES entries each), two
-// counters (behind a spare area that keeps the stated size), the work queue, and the lane search's stack spill (NA_SPILL entries per lane for NA_WAVES
+// counters, the work queue, and the lane search's stack spill (NA_SPILL entries per lane for NA_WAVES
 // waves).  Host code never uses the array's name: it asks hipGetSymbolAddress for the address
 // on each device once (na_scratch) and passes that pointer to the kernels.
 constexpr int64_t NA_MAX_QUERIES = 1 << 20;
@@ -633,8 +633,7 @@ constexpr int64_t NA_WAVES = 2048;
 constexpr size_t na_align(size_t b) { return (b + 255) / 256 * 256; }
 constexpr size_t NA_LIST1 = 0;
 constexpr size_t NA_LIST2 = na_align(NA_LIST1 + 4 * (size_t)NA_MAX_QUERIES);
-constexpr size_t NA_SPARE = na_align(NA_LIST2 + 4 * (size_t)NA_MAX_QUERIES);
-constexpr size_t NA_COUNT = na_align(NA_SPARE + 4 * (size_t)(NA_MAX_QUERIES / CF_TILE + 2));
+constexpr size_t NA_COUNT = na_align(NA_LIST2 + 4 * (size_t)NA_MAX_QUERIES);
 constexpr size_t NA_QUEUE = na_align(NA_COUNT + 4 * 4);
 constexpr size_t NA_SPILL_OFF = na_align(NA_QUEUE + 4 * (size_t)(QUEUE_SEGS * QUEUE_STRIDE));
 constexpr size_t NA_BYTES = na_align(NA_SPILL_OFF + sizeof(uint2) * (size_t)NA_SPILL * BF_THREADS * NA_WAVES);
@@ -2313,7 +2312,7 @@ int lvrhip_create_scans_device(const float* d_xyz, const int64_t* scan_offsets, 
             if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) == hipSuccess && cus > 0)
             {
                 h->resident_waves = (int64_t)cus * 16;
-                // 12 best-first waves per CU (3 per SIMD: their registers; LDS would allow 20)
+                // 12 best-first waves per CU (3 per SIMD: their registers; LDS would allow 17)
                 h->bf_resident = (int64_t)cus * 12;
             }
             h->init(d_xyz, scan_offsets, nscans);
